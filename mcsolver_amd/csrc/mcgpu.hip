@@ -120,65 +120,43 @@ struct Spins {
   PT p;
   int n;
   __device__ __forceinline__ float get(int i, int c) const { return SIO<ST>::ld(p + (size_t)c * n + i); }
-  // the spin `off` bytes away from site i's (same component)
-  __device__ __forceinline__ float get_off(int i, int c, int off) const {
-    return SIO<ST>::ld((PT)((char*)(p + (size_t)c * n + i) + off));
-  }
   __device__ __forceinline__ void set(int i, int c, float v) const { SIO<ST>::st(p + (size_t)c * n + i, v); }
 };
 template <typename ST>
 using GSpins = Spins<ST, GAS ST*>;
 
-// neighbour accessors: the global link table (site order) or a pattern row
-// (colour-permuted positions, LDS)
+// neighbour accessor of graphs without link patterns: the global link table
 struct GlobalLinks {
-  static constexpr bool BYTE_OFFSETS = false;
   const GAS uint32_t* lk;
   const GAS int32_t* lc;  // per-link coupling indices (wide graphs) or nullptr
   __device__ __forceinline__ int nbr(int l) const { return (int)(lk[l] & 0xFFFFFFu); }
   __device__ __forceinline__ uint32_t cid(int l) const { return lc ? (uint32_t)lc[l] : lk[l] >> 24; }
-  // neighbours of links l .. l+3
-  __device__ __forceinline__ void nbr4(int l, int* j) const {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) j[u] = nbr(l + u);
-  }
 };
-// LDS pattern rows are padded to a multiple of four words (16 bytes), so
-// that four links come in one 128-bit read
+// Pattern rows in LDS: zmax link words, then the site class, padded to a
+// multiple of four words so that four links come in one 128-bit read.  Graphs
+// of one coupling: each link word is the byte offset from the site's spin to
+// the neighbour's (same component).  Others: position delta << 8 | coupling.
 __host__ __device__ constexpr int pat_stride(int zmax) { return (zmax + 4) & ~3; }
-struct PatLinks {
-  static constexpr bool BYTE_OFFSETS = false;
-  const int32_t* row;  // 16-byte aligned
-  int p;
-  __device__ __forceinline__ int nbr(int l) const { return p + ((int)((uint32_t)row[l] << 8) >> 8); }
-  __device__ __forceinline__ uint32_t cid(int l) const { return (uint32_t)row[l] >> 24; }
-  // neighbours of links l .. l+3 (l a multiple of 4)
-  __device__ __forceinline__ void nbr4(int l, int* j) const {
-    const int4 w = *(const int4*)(row + l);
-    j[0] = p + ((int)((uint32_t)w.x << 8) >> 8);
-    j[1] = p + ((int)((uint32_t)w.y << 8) >> 8);
-    j[2] = p + ((int)((uint32_t)w.z << 8) >> 8);
-    j[3] = p + ((int)((uint32_t)w.w << 8) >> 8);
-  }
-};
-// pattern rows of a uniform-coupling graph in LDS: each link is the byte
-// offset from the site's spin to the neighbour's (same component), so that a
-// neighbour's address is one add
-struct PatOffLinks {
-  static constexpr bool BYTE_OFFSETS = true;
-  const int32_t* row;  // 16-byte aligned
-  int p;
-  __device__ __forceinline__ int off(int l) const { return row[l]; }
-  __device__ __forceinline__ void off4(int l, int* o) const {
-    const int4 w = *(const int4*)(row + l);
-    o[0] = w.x;
-    o[1] = w.y;
-    o[2] = w.z;
-    o[3] = w.w;
-  }
-};
+// couplings in LDS: 12 floats each, the 3x3 tensor in three 128-bit reads
+static constexpr int COUP_LDS = 12;
+template <bool UNI>
+__device__ __forceinline__ int32_t row_word(int32_t w, int ssize) {  // w: a link word of mcg_graph.pattab
+  const int32_t d = (int32_t)((uint32_t)w << 8) >> 8;
+  return UNI ? d * ssize : (int32_t)(((uint32_t)d << 8) | ((uint32_t)w >> 24));
+}
 
 static constexpr double REF_PI = 3.1415926535;  // heisenbergLib.c:6
+
+// a value that is the same in every active lane, as a scalar
+__device__ __forceinline__ int wave_uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ float wave_uniform(float x) { return __int_as_float(wave_uniform(__float_as_int(x))); }
+// a wave-uniform value kept in a vector register: FP32 adds, products and
+// FMAs whose operands are all vector registers issue at 2.8-3.2 cycles per
+// SIMD on gfx950, those with a scalar operand at 4.4 (measured, 4 waves)
+__device__ __forceinline__ float in_vgpr(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
 
 // The acceptance of a row: beta, and for exact Ising the row's threshold
 // table thr[k] = floor(2^32 exp(-beta k u)) for dE = k u (u = 1 / inv_unit, a
@@ -218,189 +196,162 @@ __device__ __forceinline__ Acc acc_of(const mcg_batch& B, float beta, int row) {
 // graph); the field is that tensor times the sum of the neighbour spins.
 // aniso = false: no site class has an on-site term (D = 0), so the D terms,
 // each an exact +0 to dE, are skipped.
+// the field: H = J . S of a uniform graph's neighbour sum, or one link's
+// J . t added to H (row-major J, the same operations in every kernel)
+template <int NC, typename CP>
+__device__ __forceinline__ void uniform_field(CP J, const float* S, float* H) {
+  H[0] = J[0] * S[0]; H[0] = fmaf(J[1], S[1], H[0]);
+  H[1] = J[3] * S[0]; H[1] = fmaf(J[4], S[1], H[1]);
+  if constexpr (NC == 3) {
+    H[0] = fmaf(J[2], S[2], H[0]);
+    H[1] = fmaf(J[5], S[2], H[1]);
+    H[2] = J[6] * S[0]; H[2] = fmaf(J[7], S[1], H[2]); H[2] = fmaf(J[8], S[2], H[2]);
+  }
+}
+template <int NC, typename CP>
+__device__ __forceinline__ void add_field(CP J, const float* t, float* H) {
+  H[0] = fmaf(J[0], t[0], H[0]); H[0] = fmaf(J[1], t[1], H[0]);
+  if constexpr (NC == 3) H[0] = fmaf(J[2], t[2], H[0]);
+  H[1] = fmaf(J[3], t[0], H[1]); H[1] = fmaf(J[4], t[1], H[1]);
+  if constexpr (NC == 3) {
+    H[1] = fmaf(J[5], t[2], H[1]);
+    H[2] = fmaf(J[6], t[0], H[2]); H[2] = fmaf(J[7], t[1], H[2]); H[2] = fmaf(J[8], t[2], H[2]);
+  }
+}
+
+// An update in its pieces, so that the sites of one draw can go through them
+// together: the field (site and neighbour spins), then the proposal and its
+// decision, then the store.
+//
+// the proposed axis of an O(n) reflection
+template <int NC>
+__device__ __forceinline__ void metro_axis(uint32_t w_a, uint32_t w_b, float* r) {
+  if constexpr (NC == 3) {
+    r[2] = fmaf((float)(w_a >> 8), 0x1p-23f, -1.0f);
+    const float rho = unit_rho(r[2]);
+    float c, sn;
+    sincos_turn(w_b, &c, &sn);
+    r[0] = rho * c;
+    r[1] = rho * sn;
+  } else {
+    sincos_turn(w_b, r, r + 1);
+    r[2] = 0.0f;
+  }
+}
+
+// the O(n) decision: s the site's spin, H its field, r the axis; n gets the
+// reflected spin (not renormalised), dE the energy change.  D: on-site terms
+// (aniso = false: none).
+template <int NC>
+__device__ __forceinline__ bool metro_decide(const float* s, const float* H, const float* r, float beta, float h,
+                                             bool aniso, const float* D, uint32_t w_c, float* n, float& dE) {
+  float p = s[0] * r[0];
+  p = fmaf(s[1], r[1], p);
+  if constexpr (NC == 3) p = fmaf(s[2], r[2], p);
+  const float a = -2.0f * p;
+  const float d0 = a * r[0], d1 = a * r[1], d2 = NC == 3 ? a * r[2] : 0.0f;
+  dE = d0 * H[0];
+  dE = fmaf(d1, H[1], dE);
+  if constexpr (NC == 3) dE = fmaf(d2, H[2], dE);
+  n[0] = s[0] + d0;
+  n[1] = s[1] + d1;
+  if constexpr (NC == 3) n[2] = s[2] + d2;
+  if (aniso) {
+    const float a0 = n[0] * n[0], b0 = s[0] * s[0], q0 = a0 - b0;
+    const float a1 = n[1] * n[1], b1 = s[1] * s[1], q1 = a1 - b1;
+    dE = fmaf(D[0], q0, dE);
+    dE = fmaf(D[1], q1, dE);
+    if constexpr (NC == 3) {
+      const float a2 = n[2] * n[2], b2 = s[2] * s[2], q2 = a2 - b2;
+      dE = fmaf(D[2], q2, dE);
+    }
+  }
+  dE = fmaf(-h, NC == 3 ? d2 : d0, dE);  // h = 0 adds an exact 0
+  const float db = dE * beta;
+  return (db <= 0.0f) | below_exp(w_c, -db);  // no branch: some lane of a wave needs the exponential
+}
+
+// the accepted spin, renormalised, as stored; its change goes to dM
+template <int NC, typename ST>
+__device__ __forceinline__ void metro_commit(const float* s, float* n, float is2, float* dMacc) {
+  float nn = n[0] * n[0];
+  nn = fmaf(n[1], n[1], nn);
+  if constexpr (NC == 3) nn = fmaf(n[2], n[2], nn);
+  const float f = renorm_factor(nn, is2);
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    n[k] *= f;
+    // FP32 storage keeps the value as computed; FP16 rounds it
+    if constexpr (std::is_same<ST, __half>::value)
+      dMacc[k] += __half2float(__float2half_rn(n[k])) - s[k];
+    else
+      dMacc[k] += n[k] - s[k];
+  }
+}
+
+// Ising: the decision for sigma = sg, spin s = sg*S and field f
+__device__ __forceinline__ bool ising_decide(float s, float f, float h, const Acc& ac, uint32_t w_c, float& dE) {
+  const float t = f - h;
+  dE = (-2.0f * s) * t;
+  if (ac.thr)
+    // exact: couplings, fields and spin lengths are multiples of powers of
+    // two small enough that every operation above is exact, dE = k u with
+    // 0 < k < nthr, and thr[k] = floor(2^32 exp(-beta k u))
+    return dE <= 0.0f || w_c < ac.thr[(int)(dE * ac.inv_unit)];
+  const float db = dE * ac.beta;
+  return (db <= 0.0f) | below_exp(w_c, -db);
+}
+
 template <int NC, typename SV, typename LK, typename CP, bool UNI = false>
-__device__ __forceinline__ void metro_core(const SV& sp, int i, const LK& lk, int zmax, CP coup, int ci, CP clsdat,
-                                           Acc ac, float h, uint32_t w_a, uint32_t w_b, uint32_t w_c,
+__device__ __forceinline__ void metro_core(const SV& sp, int i, const LK& lk, int zmax, CP coup, int cst, int ci,
+                                           CP clsdat, Acc ac, float h, uint32_t w_a, uint32_t w_b, uint32_t w_c,
                                            float& dEacc, float* dMacc, bool aniso = true) {
-  const float beta = ac.beta;
-  const float S = clsdat[ci * 8 + 0];
   if constexpr (NC == 1) {
+    const float S = clsdat[ci * 8 + 0];
     float f = 0.0f;
     if constexpr (UNI) {
-      // links four at a time: the neighbour indices are read together, then
-      // the spins, so that each site waits for two LDS round trips per four
-      // links rather than two per link (the sum keeps link order)
       float m = 0.0f;
-      int l = 0;
-      for (; l + 4 <= zmax; l += 4) {
-        int j[4];
-        float a[4];
-        if constexpr (LK::BYTE_OFFSETS) {
-          lk.off4(l, j);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) a[u] = sp.get_off(i, 0, j[u]);
-        } else {
-          lk.nbr4(l, j);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) a[u] = sp.get(j[u], 0);
-        }
-        m += a[0]; m += a[1]; m += a[2]; m += a[3];
-      }
-      for (; l < zmax; ++l) {
-        if constexpr (LK::BYTE_OFFSETS)
-          m += sp.get_off(i, 0, lk.off(l));
-        else
-          m += sp.get(lk.nbr(l), 0);
-      }
+      for (int l = 0; l < zmax; ++l) m += sp.get(lk.nbr(l), 0);
       f = coup[0] * m;
     } else {
-      for (int l = 0; l < zmax; ++l) f = fmaf(coup[lk.cid(l) * 9], sp.get(lk.nbr(l), 0), f);
+      for (int l = 0; l < zmax; ++l) f = fmaf(coup[lk.cid(l) * cst], sp.get(lk.nbr(l), 0), f);
     }
     const float sg = sp.get(i, 0);
     const float s = sg * S;
-    const float t = f - h;
-    const float dE = (-2.0f * s) * t;
-    bool acc;
-    if (ac.thr) {
-      // exact: couplings, fields and spin lengths are multiples of powers of
-      // two small enough that every operation above is exact, dE = k u with
-      // 0 < k < nthr, and thr[k] = floor(2^32 exp(-beta k u))
-      acc = dE <= 0.0f || w_c < ac.thr[(int)(dE * ac.inv_unit)];
-    } else {
-      const float db = dE * beta;
-      acc = db <= 0.0f || u24(w_c) < exp_neg(-db);
-    }
-    if (acc) {
+    float dE;
+    if (ising_decide(s, f, h, ac, w_c, dE)) {
       sp.set(i, 0, -sg);
       dEacc += dE;
       dMacc[0] += -2.0f * s;
     }
   } else {
-    const float s0 = sp.get(i, 0), s1 = sp.get(i, 1);
-    const float s2 = NC == 3 ? sp.get(i, 2) : 0.0f;
-    float H0 = 0.0f, H1 = 0.0f, H2 = 0.0f;
+    const float s[3] = {sp.get(i, 0), sp.get(i, 1), NC == 3 ? sp.get(i, 2) : 0.0f};
+    float H[3] = {0.0f, 0.0f, 0.0f};
     if constexpr (UNI) {
-      // links four at a time, as for Ising
       float S0 = 0.0f, S1 = 0.0f, S2 = 0.0f;
-      int l = 0;
-      for (; l + 4 <= zmax; l += 4) {
-        int j[4];
-        float t0[4], t1[4], t2[4];
-        if constexpr (LK::BYTE_OFFSETS) {
-          lk.off4(l, j);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            t0[u] = sp.get_off(i, 0, j[u]);
-            t1[u] = sp.get_off(i, 1, j[u]);
-            t2[u] = NC == 3 ? sp.get_off(i, 2, j[u]) : 0.0f;
-          }
-        } else {
-          lk.nbr4(l, j);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            t0[u] = sp.get(j[u], 0);
-            t1[u] = sp.get(j[u], 1);
-            t2[u] = NC == 3 ? sp.get(j[u], 2) : 0.0f;
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          S0 += t0[u];
-          S1 += t1[u];
-          if constexpr (NC == 3) S2 += t2[u];
-        }
+      for (int l = 0; l < zmax; ++l) {
+        const int j = lk.nbr(l);
+        S0 += sp.get(j, 0);
+        S1 += sp.get(j, 1);
+        if constexpr (NC == 3) S2 += sp.get(j, 2);
       }
-      for (; l < zmax; ++l) {
-        if constexpr (LK::BYTE_OFFSETS) {
-          const int o = lk.off(l);
-          S0 += sp.get_off(i, 0, o);
-          S1 += sp.get_off(i, 1, o);
-          if constexpr (NC == 3) S2 += sp.get_off(i, 2, o);
-        } else {
-          const int j = lk.nbr(l);
-          S0 += sp.get(j, 0);
-          S1 += sp.get(j, 1);
-          if constexpr (NC == 3) S2 += sp.get(j, 2);
-        }
-      }
-      H0 = coup[0] * S0; H0 = fmaf(coup[1], S1, H0);
-      H1 = coup[3] * S0; H1 = fmaf(coup[4], S1, H1);
-      if constexpr (NC == 3) {
-        H0 = fmaf(coup[2], S2, H0);
-        H1 = fmaf(coup[5], S2, H1);
-        H2 = coup[6] * S0; H2 = fmaf(coup[7], S1, H2); H2 = fmaf(coup[8], S2, H2);
-      }
+      const float S[3] = {S0, S1, S2};
+      uniform_field<NC>(coup, S, H);
     } else {
       for (int l = 0; l < zmax; ++l) {
         const int j = lk.nbr(l);
-        const CP J = coup + lk.cid(l) * 9;
-        const float t0 = sp.get(j, 0), t1 = sp.get(j, 1);
-        if constexpr (NC == 3) {
-          const float t2 = sp.get(j, 2);
-          H0 = fmaf(J[0], t0, H0); H0 = fmaf(J[1], t1, H0); H0 = fmaf(J[2], t2, H0);
-          H1 = fmaf(J[3], t0, H1); H1 = fmaf(J[4], t1, H1); H1 = fmaf(J[5], t2, H1);
-          H2 = fmaf(J[6], t0, H2); H2 = fmaf(J[7], t1, H2); H2 = fmaf(J[8], t2, H2);
-        } else {
-          H0 = fmaf(J[0], t0, H0); H0 = fmaf(J[1], t1, H0);
-          H1 = fmaf(J[3], t0, H1); H1 = fmaf(J[4], t1, H1);
-        }
+        const CP J = coup + lk.cid(l) * cst;
+        const float t[3] = {sp.get(j, 0), sp.get(j, 1), NC == 3 ? sp.get(j, 2) : 0.0f};
+        add_field<NC>(J, t, H);
       }
     }
-    float rx, ry, rz = 0.0f;
-    if constexpr (NC == 3) {
-      rz = fmaf(u24(w_a), 2.0f, -1.0f);
-      const float rho = sqrtf(fmaxf(fmaf(-rz, rz, 1.0f), 0.0f));
-      float c, sn;
-      sincos_turn(w_b, &c, &sn);
-      rx = rho * c;
-      ry = rho * sn;
-    } else {
-      sincos_turn(w_b, &rx, &ry);
-    }
-    float p = s0 * rx;
-    p = fmaf(s1, ry, p);
-    if constexpr (NC == 3) p = fmaf(s2, rz, p);
-    const float a = -2.0f * p;
-    const float d0 = a * rx, d1 = a * ry, d2 = a * rz;
-    float dE = d0 * H0;
-    dE = fmaf(d1, H1, dE);
-    if constexpr (NC == 3) dE = fmaf(d2, H2, dE);
-    float n0 = s0 + d0, n1 = s1 + d1, n2 = s2 + d2;
-    if (aniso) {
-      const float Dx = clsdat[ci * 8 + 1], Dy = clsdat[ci * 8 + 2], Dz = clsdat[ci * 8 + 3];
-      const float a0 = n0 * n0, b0 = s0 * s0, q0 = a0 - b0;
-      const float a1 = n1 * n1, b1 = s1 * s1, q1 = a1 - b1;
-      dE = fmaf(Dx, q0, dE);
-      dE = fmaf(Dy, q1, dE);
-      if constexpr (NC == 3) {
-        const float a2 = n2 * n2, b2 = s2 * s2, q2 = a2 - b2;
-        dE = fmaf(Dz, q2, dE);
-      }
-    }
-    if (h != 0.0f) dE = fmaf(-h, NC == 3 ? d2 : d0, dE);  // h = 0 would add an exact 0
-    const float db = dE * beta;
-    if (db <= 0.0f || u24(w_c) < exp_neg(-db)) {
-      float nn = n0 * n0;
-      nn = fmaf(n1, n1, nn);
-      if constexpr (NC == 3) nn = fmaf(n2, n2, nn);
-      const float f = renorm_factor(nn, clsdat[ci * 8 + 4]);
-      n0 = n0 * f;
-      n1 = n1 * f;
-      n2 = n2 * f;
-      sp.set(i, 0, n0);
-      sp.set(i, 1, n1);
-      if constexpr (NC == 3) sp.set(i, 2, n2);
+    float r[3], n[3], dE;
+    metro_axis<NC>(w_a, w_b, r);
+    const float D[3] = {clsdat[ci * 8 + 1], clsdat[ci * 8 + 2], clsdat[ci * 8 + 3]};
+    if (metro_decide<NC>(s, H, r, ac.beta, h, aniso, D, w_c, n, dE)) {
+      metro_commit<NC, typename SV::value_type>(s, n, clsdat[ci * 8 + 4], dMacc);
+      for (int k = 0; k < NC; ++k) sp.set(i, k, n[k]);
       dEacc += dE;
-      if constexpr (std::is_same<typename SV::value_type, float>::value) {
-        // FP32 storage keeps the value as computed
-        dMacc[0] += n0 - s0;
-        dMacc[1] += n1 - s1;
-        if constexpr (NC == 3) dMacc[2] += n2 - s2;
-      } else {
-        dMacc[0] += sp.get(i, 0) - s0;
-        dMacc[1] += sp.get(i, 1) - s1;
-        if constexpr (NC == 3) dMacc[2] += sp.get(i, 2) - s2;
-      }
     }
   }
 }
@@ -417,7 +368,7 @@ struct SitesPerDraw {
 template <int NC, bool UNI = false, typename SV, typename CP>
 __device__ __forceinline__ void metro_group(const SV& sp, int b, int cnt, int q, int colour,
                                             const GAS uint32_t* __restrict__ link,
-                                            const GAS int32_t* __restrict__ lcid, int zmax, CP coup,
+                                            const GAS int32_t* __restrict__ lcid, int zmax, CP coup, int cst,
                                             const GAS int32_t* __restrict__ cls, CP clsdat, Acc beta, float h,
                                             uint64_t sweep, uint32_t key0, uint32_t key1, float& dEacc,
                                             float* dMacc) {
@@ -434,68 +385,281 @@ __device__ __forceinline__ void metro_group(const SV& sp, int b, int cnt, int q,
       const uint32_t wa = NC == 3 ? w[0] : 0u;
       const uint32_t wb = NC == 3 ? w[1] : NC == 2 ? w[2 * g] : 0u;
       const uint32_t wc = NC == 3 ? w[2] : NC == 2 ? w[2 * g + 1] : w[g];
-      metro_core<NC, SV, GlobalLinks, CP, UNI>(sp, i, lk, zmax, coup, (int)cls[i], clsdat, beta, h, wa, wb, wc, dEacc,
-                                               dMacc);
+      metro_core<NC, SV, GlobalLinks, CP, UNI>(sp, i, lk, zmax, coup, cst, (int)cls[i], clsdat, beta, h, wa, wb, wc,
+                                               dEacc, dMacc);
     }
   }
 }
 
-// same, on the colour-permuted LDS replica: colour c occupies positions
-// b .. b+cnt-1, the neighbours come from the pattern row of each position
-template <int NC, typename ST, bool UNI = false>
-__device__ __forceinline__ void metro_group_pat(const Spins<ST>& sp, int b, int cnt, int q, int colour,
-                                                const uint8_t* pat, const int32_t* pattab, int zmax,
-                                                const float* coup, const float* clsdat, Acc beta, float h,
-                                                uint64_t sweep, uint32_t key0, uint32_t key1, float& dEacc,
-                                                float* dMacc, bool aniso = true) {
-  constexpr int G = SitesPerDraw<NC>::G;
-  const u32x4 x = philox4x32_10(
-      u32x4{(uint32_t)q, (uint32_t)sweep, (uint32_t)(sweep >> 32), TAG_METRO | ((uint32_t)colour << 8)}, key0, key1);
-  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+// One replica's spins, in LDS or in HBM: a site's place, and loads and stores
+// at a byte offset from it.  In LDS a place is one address per component (a
+// vector add to reach a neighbour's).  In HBM it is a 32-bit offset from
+// scalar bases, so that a neighbour's components share one add; 64-bit
+// addresses per lane took 6.5 instructions a link.
+template <int NC, typename ST>
+struct LdsView {
+  typedef ST value_type;
+  ST* p;
+  int n;
+  struct Site {
+    char* a[NC];
+  };
+  __device__ __forceinline__ Site at(int i) const {
+    Site s;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int lp = q * G + g;
-    if (lp < cnt) {
-      const int p = b + lp;
-      // 24-bit multiply: full rate, and pattern ids and strides are small
-      const int32_t* row = pattab + __umul24((uint32_t)pat[p], (uint32_t)pat_stride(zmax));
-      typedef typename std::conditional<UNI, PatOffLinks, PatLinks>::type LK;
-      const LK lk{row, p};
-      const uint32_t wa = NC == 3 ? w[0] : 0u;
-      const uint32_t wb = NC == 3 ? w[1] : NC == 2 ? w[2 * g] : 0u;
-      const uint32_t wc = NC == 3 ? w[2] : NC == 2 ? w[2 * g + 1] : w[g];
-      metro_core<NC, Spins<ST>, LK, const float*, UNI>(sp, p, lk, zmax, coup, row[zmax], clsdat, beta, h, wa, wb, wc,
-                                                       dEacc, dMacc, aniso);
+    for (int k = 0; k < NC; ++k) s.a[k] = (char*)(p + i) + k * n * (int)sizeof(ST);
+    return s;
+  }
+  static __device__ __forceinline__ float ld(const Site& s, int k, int off) { return SIO<ST>::ld((const ST*)(s.a[k] + off)); }
+  static __device__ __forceinline__ void st(const Site& s, int k, float v) { SIO<ST>::st((ST*)s.a[k], v); }
+};
+template <int NC, typename ST>
+struct HbmView {
+  typedef ST value_type;
+  GAS ST* p[NC];
+  typedef uint32_t Site;
+  __device__ __forceinline__ HbmView(GAS ST* p0, int n) {
+    // separate scalar bases: the compiler would fold the component stride
+    // into each lane's address
+    for (int c = 0; c < NC; ++c) {
+      p[c] = p0 + (size_t)c * n;
+      asm("" : "+s"(p[c]));
+    }
+  }
+  __device__ __forceinline__ Site at(int i) const { return (uint32_t)i * (uint32_t)sizeof(ST); }
+  __device__ __forceinline__ float ld(const Site& s, int k, int off) const {
+    return SIO<ST>::ld((const GAS ST*)((const GAS char*)p[k] + (s + (uint32_t)off)));
+  }
+  __device__ __forceinline__ void st(const Site& s, int k, float v) const { SIO<ST>::st((GAS ST*)((GAS char*)p[k] + s), v); }
+};
+
+// What the updates of a sweep read besides spins and draws, for graphs with
+// link patterns.  coup, clsdat: LDS (COUP_LDS floats a tensor), or HBM for
+// the classes of the streaming pass.  With one coupling or one site class
+// their values are kept in registers: read where they are used, each update
+// would wait for them.
+template <int NC, typename CP>
+struct RowTab {
+  const int32_t* rows;
+  const float* coup;
+  CP clsdat;
+  int zmax, stride;  // stride: bytes per row
+  bool aniso, one;  // any on-site term; one site class
+  float J[9];       // the coupling of a uniform graph
+  float cls0[5];    // the one class: S, D, 1/S^2
+};
+template <int NC, bool UNI, typename JP, typename CP>
+__device__ __forceinline__ void row_tab(RowTab<NC, CP>& T, const int32_t* rows, const float* coup, JP ucoup, CP clsdat,
+                                        int zmax, int ncls, bool aniso) {
+  T.rows = rows;
+  T.coup = coup;
+  T.clsdat = clsdat;
+  T.zmax = zmax;
+  T.stride = pat_stride(zmax) * 4;
+  T.aniso = aniso;
+  T.one = ncls == 1;
+  if constexpr (UNI)
+    for (int k = 0; k < 9; ++k) T.J[k] = in_vgpr(ucoup[k]);
+  for (int k = 0; k < 5; ++k) T.cls0[k] = in_vgpr(clsdat[k]);
+}
+
+// the coupling of a pattern row's link word (graphs of several couplings)
+template <int NC>
+__device__ __forceinline__ void link_coup(const float* coup, int32_t w, float* J) {
+  const float* c = coup + __umul24((uint32_t)w & 0xFFu, COUP_LDS);
+  if constexpr (NC == 1) {
+    J[0] = c[0];
+  } else {
+    const float4 a = *(const float4*)c, b = *(const float4*)(c + 4);
+    J[0] = a.x; J[1] = a.y; J[2] = a.z; J[3] = a.w; J[4] = b.x;
+    if constexpr (NC == 3) {
+      J[5] = b.y; J[6] = b.z; J[7] = b.w; J[8] = c[8];
     }
   }
 }
 
-// same, with the spins in HBM (streaming pass): pattern ids read from HBM,
-// pattern rows (raw position deltas | coupling << 24, then the class) in LDS
-template <int NC, typename ST, bool UNI>
-__device__ __forceinline__ void metro_group_gpat(const GSpins<ST>& sp, int b, int cnt, int q, int colour,
-                                                 const GAS uint8_t* __restrict__ pat, const int32_t* pattab, int zmax,
-                                                 const GAS float* coup, const GAS float* clsdat, Acc beta, float h,
-                                                 uint64_t sweep, uint32_t key0, uint32_t key1, float& dEacc,
-                                                 float* dMacc, bool aniso) {
+// four words of a pattern row
+__device__ __forceinline__ void read_row(const int32_t* row, int32_t* x) {
+  const int4 a = *(const int4*)row;
+  x[0] = a.x;
+  x[1] = a.y;
+  x[2] = a.z;
+  x[3] = a.w;
+}
+// the field of a uniform graph from the sum of the neighbour spins
+template <int NC, typename T>
+__device__ __forceinline__ void sum_field(const T& tab, const float* S, float* H) {
+  if constexpr (NC == 1)
+    H[0] = tab.J[0] * S[0];
+  else
+    uniform_field<NC>(tab.J, S, H);
+}
+
+// Field of the site at `own`, its pattern row given: every
+// neighbour is read before the first is used.  Z: the number of links, or 0
+// where it is only known at run time (then four links at a time).
+template <int NC, bool UNI, int Z, typename V, typename CP>
+__device__ __forceinline__ void row_field(const V& v, const typename V::Site& own, const int32_t* row,
+                                          const RowTab<NC, CP>& T, float* H) {
+  typedef typename V::value_type ST;
+  constexpr int B = Z == 0 ? 4 : Z == 9 ? 3 : Z;  // links per batch
+  const int zmax = Z > 0 ? Z : T.zmax;
+  float S[3] = {0.0f, 0.0f, 0.0f};
+  H[0] = H[1] = H[2] = 0.0f;
+  int32_t rw[Z > 0 ? (Z + 3) / 4 * 4 : 4];
+  if constexpr (Z > 0)
+#pragma unroll
+    for (int u = 0; u < Z; u += 4) read_row(row + u, rw + u);
+  for (int l0 = 0; l0 < zmax; l0 += B) {
+    int32_t w[B];
+    if constexpr (Z == 0) read_row(row + l0, rw);
+#pragma unroll
+    for (int u = 0; u < B; ++u) w[u] = rw[Z > 0 ? l0 + u : u];
+    float t[B][NC];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (Z == 0 && l0 + u >= zmax) w[u] = 0;  // past the last link: the site itself, not used
+      const int o = UNI ? w[u] : (w[u] >> 8) * (int)sizeof(ST);
+#pragma unroll
+      for (int k = 0; k < NC; ++k) t[u][k] = v.ld(own, k, o);
+    }
+    if constexpr (UNI) {
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        if (Z == 0 && l0 + u >= zmax) break;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) S[k] += t[u][k];
+      }
+    } else {
+      // each link's tensor is read while the one before it is used (all at
+      // once would take 9 registers a link)
+      float J[2][9];
+      link_coup<NC>(T.coup, w[0], J[0]);
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        if (u + 1 < B && (Z > 0 || l0 + u + 1 < zmax)) link_coup<NC>(T.coup, w[u + 1], J[(u + 1) & 1]);
+        if (Z == 0 && l0 + u >= zmax) break;
+        if constexpr (NC == 1)
+          H[0] = fmaf(J[u & 1][0], t[u][0], H[0]);
+        else
+          add_field<NC>(J[u & 1], t[u], H);
+        // keep the sum here: sunk to where H is used, it would hold every
+        // link's tensor and spin in registers until then
+        asm volatile("" : "+v"(H[0]), "+v"(H[1]), "+v"(H[2]));
+      }
+    }
+  }
+  if constexpr (UNI) sum_field<NC>(T, S, H);
+}
+
+// The sites of one draw (group q of a colour class of cnt positions from b
+// on), on a graph with link patterns.  They share a colour, so none is
+// another's neighbour: all fields are read, then all decisions taken, then
+// the accepted spins stored, and the sites' loads overlap instead of each
+// site waiting for its own chain.  Changes are added in site order.
+template <int NC, bool UNI, int Z, typename V, typename PP, typename CP>
+__device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, int colour, PP pat,
+                                           const RowTab<NC, CP>& T, const Acc& ac, float h, uint64_t sweep,
+                                           uint32_t key0, uint32_t key1, float& dEacc, float* dMacc) {
+  typedef typename V::value_type ST;
   constexpr int G = SitesPerDraw<NC>::G;
-  const u32x4 x = philox4x32_10(
-      u32x4{(uint32_t)q, (uint32_t)sweep, (uint32_t)(sweep >> 32), TAG_METRO | ((uint32_t)colour << 8)}, key0, key1);
-  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+  typename V::Site own[G];
+  float s[G][3], H[G][3];
+  const int32_t* row[G];
+  int cl[G];
+  bool live[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     const int lp = q * G + g;
-    if (lp < cnt) {
-      const int p = b + lp;
-      const int32_t* row = pattab + __umul24((uint32_t)pat[p], (uint32_t)pat_stride(zmax));
-      const PatLinks lk{row, p};
-      const uint32_t wa = NC == 3 ? w[0] : 0u;
-      const uint32_t wb = NC == 3 ? w[1] : NC == 2 ? w[2 * g] : 0u;
-      const uint32_t wc = NC == 3 ? w[2] : NC == 2 ? w[2 * g + 1] : w[g];
-      metro_core<NC, GSpins<ST>, PatLinks, const GAS float*, UNI>(sp, p, lk, zmax, coup, row[zmax], clsdat, beta, h,
-                                                                  wa, wb, wc, dEacc, dMacc, aniso);
+    live[g] = lp < cnt;  // the last group may be short: its missing sites read the last one
+    const int p = b + (G == 1 || live[g] ? lp : cnt - 1);
+    row[g] = (const int32_t*)((const char*)T.rows + __umul24((uint32_t)pat[p], (uint32_t)T.stride));
+    own[g] = v.at(p);
+#pragma unroll
+    for (int k = 0; k < NC; ++k) s[g][k] = v.ld(own[g], k, 0);
+  }
+  if constexpr (UNI && Z > 0) {
+    // every site's row, then every neighbour, then the sums
+    int32_t w[G][(Z + 3) / 4 * 4];
+    float t[G][Z][NC];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int u = 0; u < Z; u += 4) read_row(row[g] + u, w[g] + u);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int u = 0; u < Z; ++u)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) t[g][u][k] = v.ld(own[g], k, w[g][u]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float S[3] = {t[g][0][0], NC > 1 ? t[g][0][NC > 1 ? 1 : 0] : 0.0f, NC > 2 ? t[g][0][NC > 2 ? 2 : 0] : 0.0f};
+#pragma unroll
+      for (int u = 1; u < Z; ++u)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) S[k] += t[g][u][k];
+      sum_field<NC>(T, S, H[g]);
+    }
+  } else {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      cl[g] = Z > 0 || T.one ? 0 : row[g][T.zmax] * 8;
+      row_field<NC, UNI, Z>(v, own[g], row[g], T, H[g]);
     }
   }
+  const u32x4 x = philox4x32_10(
+      u32x4{(uint32_t)q, (uint32_t)sweep, (uint32_t)(sweep >> 32), TAG_METRO | ((uint32_t)colour << 8)}, key0, key1);
+  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+  float n[G][3], dE[G], is2[G];
+  bool acc[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float c[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) c[k] = T.cls0[k];
+    if (Z == 0 && !T.one)
+#pragma unroll
+      for (int k = 0; k < 5; ++k) c[k] = T.clsdat[cl[g] + k];
+    if constexpr (NC == 1) {
+      n[g][0] = s[g][0] * c[0];  // the spin sigma*S
+      acc[g] = ising_decide(n[g][0], H[g][0], h, ac, w[g], dE[g]) & live[g];
+    } else {
+      float r[3];
+      metro_axis<NC>(NC == 3 ? w[0] : 0u, NC == 3 ? w[1] : w[2 * g], r);
+      acc[g] = metro_decide<NC>(s[g], H[g], r, ac.beta, h, T.aniso, c + 1, NC == 3 ? w[2] : w[2 * g + 1], n[g],
+                                dE[g]) & live[g];
+      is2[g] = c[4];
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    if (acc[g]) {
+      dEacc += dE[g];
+      if constexpr (NC == 1) {
+        v.st(own[g], 0, -s[g][0]);
+        dMacc[0] += -2.0f * n[g][0];
+      } else {
+        metro_commit<NC, ST>(s[g], n[g], is2[g], dMacc);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) v.st(own[g], k, n[g][k]);
+      }
+    }
+}
+
+// f(Z) with the link count a compile-time constant for graphs of one site
+// class with a common count: square (4), triangular and cubic (6) lattices,
+// honeycomb with second neighbours (9); f(0) for any other
+template <bool UNI, typename T, typename F>
+__device__ __forceinline__ void with_links(const T& t, F&& f) {
+  if (UNI && t.one && t.zmax == 4)
+    f(std::integral_constant<int, 4>());
+  else if (t.one && t.zmax == 6)
+    f(std::integral_constant<int, 6>());
+  else if (!UNI && t.one && t.zmax == 9)
+    f(std::integral_constant<int, 9>());
+  else
+    f(std::integral_constant<int, 0>());
 }
 
 // spin vector of site i (Ising: sigma*S)
@@ -515,13 +679,13 @@ __device__ __forceinline__ void spin_vec(const SV& sp, int i, const int32_t* __r
 // per-site energy e_i (FP32): 1/2 s_i.H_i + onsite - h s_axis
 template <int NC, typename SV>
 __device__ __forceinline__ float site_energy(const SV& sp, int i, const uint32_t* __restrict__ link,
-                                             const int32_t* __restrict__ lcid, int zmax, const float* coup,
+                                             const int32_t* __restrict__ lcid, int zmax, const float* coup, int cst,
                                              const int32_t* __restrict__ cls, const float* clsdat, float h) {
   const int ci = cls[i];
   const GlobalLinks lk{gas(link) + (size_t)i * zmax, lcid ? gas(lcid) + (size_t)i * zmax : nullptr};
   if constexpr (NC == 1) {
     float f = 0.0f;
-    for (int l = 0; l < zmax; ++l) f = fmaf(coup[lk.cid(l) * 9], sp.get(lk.nbr(l), 0), f);
+    for (int l = 0; l < zmax; ++l) f = fmaf(coup[lk.cid(l) * cst], sp.get(lk.nbr(l), 0), f);
     const float s = sp.get(i, 0) * clsdat[ci * 8];
     return fmaf(0.5f * s, f, -h * s);
   } else {
@@ -529,7 +693,7 @@ __device__ __forceinline__ float site_energy(const SV& sp, int i, const uint32_t
     float H0 = 0.0f, H1 = 0.0f, H2 = 0.0f;
     for (int l = 0; l < zmax; ++l) {
       const int j = lk.nbr(l);
-      const float* J = coup + lk.cid(l) * 9;
+      const float* J = coup + lk.cid(l) * cst;
       const float t0 = sp.get(j, 0), t1 = sp.get(j, 1), t2 = NC == 3 ? sp.get(j, 2) : 0.0f;
       H0 = fmaf(J[0], t0, H0); H0 = fmaf(J[1], t1, H0); H0 = fmaf(J[2], t2, H0);
       H1 = fmaf(J[3], t0, H1); H1 = fmaf(J[4], t1, H1); H1 = fmaf(J[5], t2, H1);
@@ -644,13 +808,32 @@ __device__ __forceinline__ void group_sum8(double* v, double* s_red, int g, int 
 // measurement of one frame (all flagged observables) for one replica
 // ---------------------------------------------------------------------------
 struct FrameCtx {
-  const mcg_graph* G;
+  const mcg_graph* G;  // in device memory
   const float* coup;
+  int cst;         // floats per coupling
   const float* clsdat;
   double* s_red;   // reduction scratch (nwaves*RK)
   double* s_frm;   // per-group frame values (>= 64 doubles per group)
   int g, lt, TPR;
 };
+
+// Frames and recomputes sit inside the sweep loop.  Left to itself the
+// compiler keeps everything they read (some 60 words of the graph, an address
+// per loop and thread) in registers across the sweeps, and spills what the
+// sweeps need.  fresh reads the graph again where it is needed (scalar loads);
+// opaque hides a thread index, so that nothing computed from it is moved out
+// of the loop.
+__device__ __forceinline__ mcg_graph fresh(const mcg_graph* G) {
+  const uint64_t x = (uint64_t)G;
+  uint32_t lo = (uint32_t)wave_uniform((int)x), hi = (uint32_t)wave_uniform((int)(x >> 32));
+  asm volatile("" : "+s"(lo), "+s"(hi));
+  const uint64_t a = (uint64_t)hi << 32 | lo;
+  return *(const mcg_graph*)(const __attribute__((address_space(4))) mcg_graph*)a;
+}
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 
 // majority spin of block-spin site (heisenbergLib.c:255-267, isingLib.c:133-150)
 template <int NC, typename SV>
@@ -730,8 +913,8 @@ __device__ __forceinline__ int frame_groups(const mcg_graph& G, int flags) {
 // threads.  Fire-and-forget: nothing here waits for the atomics.
 template <int NC>
 __device__ __forceinline__ void flush_frame(const FrameCtx& C, const mcg_batch& B, int row, int flags) {
-  const mcg_graph& G = *C.G;
-  const int lt = C.lt, TPR = C.TPR;
+  const mcg_graph G = fresh(C.G);
+  const int lt = opaque(C.lt), TPR = C.TPR;
   const double* F = C.s_frm;
   const double* Cn = F + FRM_ACC;
   const int ngq = frame_groups<NC>(G, flags);
@@ -896,11 +1079,13 @@ struct PartFrame {
 // the part's copy), and block spins and groups are not measured.
 static constexpr int FSUMS = 88;     // frame sums per replica (F[0, 88))
 static constexpr int FSUMS_PQ = 9;   // of which pairs and circuits (F[0, 9))
+// Inlined wherever it is used: as a call it takes the batch, the graph and the
+// replica by address, which keeps them in scratch memory for the whole kernel.
 template <int NC, typename SV, bool FULL = true>
-__device__ void frame_sums(const SV& sp, const FrameCtx& C, const mcg_batch& B, int64_t frame, uint32_t key0,
+__device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, const mcg_batch& B, int64_t frame, uint32_t key0,
                            uint32_t key1, float h, int part, int np, const PartFrame* own = nullptr) {
-  const mcg_graph& G = *C.G;
-  const int lt = C.lt, TPR = C.TPR;
+  const mcg_graph G = fresh(C.G);
+  const int lt = opaque(C.lt), TPR = C.TPR;
   double* F = C.s_frm;  // leader-only use
   double v[RK];
   const int flags = FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS);
@@ -993,7 +1178,7 @@ __device__ void frame_sums(const SV& sp, const FrameCtx& C, const mcg_batch& B, 
         // wide graphs: the block-spin link takes the coupling of the site's
         // link l; a set high byte marks an absent link
         if (G.lcid && (wd >> 24)) continue;
-        const float* J = C.coup + (G.lcid ? G.lcid[(size_t)j * G.zmax + l] : (int)(wd >> 24)) * 9;
+        const float* J = C.coup + (G.lcid ? G.lcid[(size_t)j * G.zmax + l] : (int)(wd >> 24)) * C.cst;
         float mt[3];
         majority<NC>(sp, G, C.clsdat, t, frame, key0, key1, mt);
         if constexpr (NC == 1) {
@@ -1049,10 +1234,10 @@ __device__ void frame_sums(const SV& sp, const FrameCtx& C, const mcg_batch& B, 
 // One measured frame of the group's replica at `row`: the spin-derived sums
 // (frame_sums), then frame_apply.
 template <int NC>
-__device__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
+__device__ __forceinline__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
                             int flags, double mprev, bool have_prev, bool defer);
 template <int NC, typename SV, bool FULL = true>
-__device__ void measure_frame(const SV& sp, const FrameCtx& C, const mcg_batch& B, const double* st, int row,
+__device__ __forceinline__ void measure_frame(const SV& sp, const FrameCtx& C, const mcg_batch& B, const double* st, int row,
                               int64_t frame, uint32_t key0, uint32_t key1, float h, double mprev = 0.0,
                               bool have_prev = false, bool defer = false) {
   frame_sums<NC, SV, FULL>(sp, C, B, frame, key0, key1, h, 0, 1);
@@ -1063,9 +1248,9 @@ __device__ void measure_frame(const SV& sp, const FrameCtx& C, const mcg_batch& 
 // tracked state st and the spin-derived sums in C.s_frm (valid in the
 // group's first thread); called by every thread of the group.
 template <int NC>
-__device__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
+__device__ __forceinline__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
                             int flags, double mprev, bool have_prev, bool defer) {
-  const mcg_graph& G = *C.G;
+  const mcg_graph G = fresh(C.G);
   const int lt = C.lt;
   double* F = C.s_frm;
   // --- leader: this frame's contribution to every FP64 accumulator of the
@@ -1096,14 +1281,16 @@ __device__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double*
 // sum_i | |s_i|^2 / S_i^2 - 1 | (0 for Ising)
 static constexpr int NREC = 5;
 template <int NC, typename SV>
-__device__ void recompute(const SV& sp, const mcg_graph& G, const float* coup, const float* clsdat, float h,
+__device__ __forceinline__ void recompute(const SV& sp, const mcg_graph* Gd, const float* coup, int cst, const float* clsdat, float h,
                           double* s_red, int g, int lt, int TPR, double* out, int part = 0, int np = 1) {
+  const mcg_graph G = fresh(Gd);
+  lt = opaque(lt);
   double v[RK];
   for (int k = 0; k < RK; ++k) v[k] = 0.0;
   int lo, hi;
   slice(G.n, part, np, lo, hi);
   for (int i = lo + lt; i < hi; i += TPR) {
-    v[0] += (double)site_energy<NC>(sp, i, G.link, G.lcid, G.zmax, coup, G.cls, clsdat, h);
+    v[0] += (double)site_energy<NC>(sp, i, G.link, G.lcid, G.zmax, coup, cst, G.cls, clsdat, h);
     float s[3];
     spin_vec<NC>(sp, i, G.cls, clsdat, s);
     v[1] += s[0];
@@ -1257,7 +1444,7 @@ __device__ __forceinline__ void stage(ST* lds, ST* g, int count, int lt, int TPR
 
 __host__ __device__ inline size_t lds_fixed_bytes(int ncoup, int ncls, int ncol, int npat, int zmax, int n,
                                                   int nwaves, int R) {
-  size_t b = align16((size_t)(ncoup * 9 + ncls * 8) * 4) + align16((size_t)(ncol + 1) * 4);
+  size_t b = align16((size_t)(ncoup * COUP_LDS + ncls * 8) * 4) + align16((size_t)(ncol + 1) * 4);
   if (npat > 0) b += align16((size_t)npat * pat_stride(zmax) * 4) + align16((size_t)n);
   return b + align16((size_t)nwaves * RK * 8) + align16((size_t)R * (MCG_NSTATE + FRM) * 8) + align16((size_t)R * 16);
 }
@@ -1368,7 +1555,7 @@ struct RawBits<4> {
 // raw bit patterns of the storage type (ordinary accesses; the caller
 // orders them with fences where another workgroup reads them)
 template <typename ST, bool OUT>
-__device__ void part_copy(ST* lds_s, ST* gsp, int n, int nc, const int32_t* colptr, int ncol, int gd, int p, int np,
+__device__ __forceinline__ void part_copy(ST* lds_s, ST* gsp, int n, int nc, const int32_t* colptr, int ncol, int gd, int p, int np,
                           int lt, int TPR) {
   typedef typename RawBits<sizeof(ST)>::T U;
   U* lds = (U*)lds_s;
@@ -1395,7 +1582,7 @@ __device__ void part_copy(ST* lds_s, ST* gsp, int n, int nc, const int32_t* colp
 // (DevSpins) after the next grid barrier.  The copy is not the replica's
 // spin array: other parts still stage from that at the launch start.
 template <typename ST>
-__device__ void part_publish(const ST* lds_s, typename RawBits<sizeof(ST)>::T* dst, int n, int dn, int nc,
+__device__ __forceinline__ void part_publish(const ST* lds_s, typename RawBits<sizeof(ST)>::T* dst, int n, int dn, int nc,
                              const int32_t* colptr, int ncol, int gd, int p, int np, int lt, int TPR) {
   typedef typename RawBits<sizeof(ST)>::T U;
   const U* lds = (const U*)lds_s;
@@ -1470,7 +1657,7 @@ __device__ __forceinline__ void tail_rest(const SV& sv, const mcg_graph& G, cons
                                           double mprev = 0.0, bool have_prev = false, bool defer = false) {
   if (rec) {
     double r4[NREC];
-    recompute<NC>(sv, G, s_coup, s_cls, h, s_red, g, lt, TPR, r4);
+    recompute<NC>(sv, C.G, s_coup, C.cst, s_cls, h, s_red, g, lt, TPR, r4);
     if (lt == 0) {
       const double d = fabs(st[MCG_S_E] - r4[0]);
       if (d > st[MCG_S_DRIFT]) st[MCG_S_DRIFT] = d;
@@ -1587,12 +1774,12 @@ __device__ __forceinline__ double frame_mprev3(const SweepArgs& a, int64_t f, in
   return dev_load(a.mprev3 + (size_t)((f + 2) % 3) * nrow + row);
 }
 template <int NC>
-__device__ __forceinline__ void take_frame(const mcg_graph& G, const mcg_batch& B, const SweepArgs& a, double* s_st,
+__device__ __forceinline__ void take_frame(const mcg_graph* Gd, const mcg_batch& B, const SweepArgs& a, double* s_st,
                                            double* s_frm, int lane, int64_t f, int row, int nrow, double mp,
                                            int flags) {
   double* F = s_frm + lane * FRM;
   double* Cn = F + FRM_ACC;
-  frame_terms<NC>(G, B, s_st + lane * MCG_NSTATE, F, flags, f, Cn);
+  frame_terms<NC>(fresh(Gd), B, s_st + lane * MCG_NSTATE, F, flags, f, Cn);
   const double Mf = Cn[MCG_A_MM];
   Cn[MCG_A_MM] = mp * Mf;
   dev_store(a.mprev3 + (size_t)(f % 3) * nrow + row, Mf);
@@ -1607,7 +1794,7 @@ __device__ __forceinline__ void take_frame(const mcg_graph& G, const mcg_batch& 
 // the part's workgroup; false: time-out (the caller leaves the kernel).
 // A part overwrites its slot only after the next grid barrier, which part 0
 // passes after reading it.
-__device__ bool gather_frame_sums(const SweepArgs& a, const mcg_batch& B, double* F, int slot, int part, int np,
+__device__ __forceinline__ bool gather_frame_sums(const SweepArgs& a, const mcg_batch& B, double* F, int slot, int part, int np,
                                   int64_t frame, int* s_flag) {
   double* fp = a.fpart + (size_t)slot * MAX_PARTS * FSUMS;
   uint32_t* cnt = a.sync + (size_t)slot * SYNC_STRIDE;
@@ -1772,6 +1959,11 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
   constexpr int GD = SitesPerDraw<NC>::G;
   const int zmax = G.zmax;
   const bool split = pi.np > 1;
+  RowTab<NC, const float*> T;
+  beta.beta = in_vgpr(beta.beta);
+  h = in_vgpr(h);
+  if constexpr (MODE == 0 || MODE == 3)
+    row_tab<NC, MODE == 3>(T, s_pat, coup, coup + (MODE == 3 ? G.ucid : 0) * COUP_LDS, clsdat, zmax, G.ncls, aniso);
   // A colour's groups are dealt out in rounds of TPR; the last, partial
   // round falls to the first lanes of the deal.  The deal starts at wave r
   // of the group, chosen so that the groups' partial rounds land on
@@ -1798,47 +1990,47 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
     float xE = 0.0f, xM[3] = {0.0f, 0.0f, 0.0f};
     if constexpr (MODE == 0 || MODE == 3) {
       constexpr bool UNI = MODE == 3;
-      const float* cp = UNI ? coup + G.ucid * 9 : coup;
       const int qm = q1 - pl.rem;  // the pool takes the last rem groups (unsplit replicas only)
-      int q = q0 + lt;
-      for (; q < qm; q += TPR)
-        metro_group_pat<NC, ST, UNI>(sp, b, cnt, q, c, s_pid, s_pat, zmax, cp, clsdat, beta, h, kk, key0, key1, fE,
-                                     fM, aniso);
-      if (pl.pr >= 0) {
-        const float4 pv = pl.par[pl.pr];
-        float pe = 0.0f, pm[3] = {0.0f, 0.0f, 0.0f};
-        const Spins<ST> psp{pl.spin0 + (size_t)pl.sstride * pl.pr, G.n};
-        metro_group_pat<NC, ST, UNI>(psp, b, cnt, qm + pl.pq, c, s_pid, s_pat, zmax, cp, clsdat,
-                                     beta.at(pv.x, __float_as_int(pv.w)), pv.y, kk, key0,
-                                     __float_as_uint(pv.z), pe, pm, aniso);
-        // the first pool group after a tail stores, later ones add
-        double* pp = pl.pp + threadIdx.x;
-        const bool first = pfresh && c == 0;
-        pp[0] = first ? (double)pe : pp[0] + (double)pe;
+      const LdsView<NC, ST> v{sp.p, sp.n};
+      with_links<UNI>(T, [&](auto zc) {
+        constexpr int Z = decltype(zc)::value;
+        int q = q0 + lt;
+        for (; q < qm; q += TPR)
+          metro_rows<NC, UNI, Z>(v, b, cnt, q, c, s_pid, T, beta, h, kk, key0, key1, fE, fM);
+        if (pl.pr >= 0) {
+          const float4 pv = pl.par[pl.pr];
+          float pe = 0.0f, pm[3] = {0.0f, 0.0f, 0.0f};
+          const LdsView<NC, ST> pv_s{pl.spin0 + pl.sstride * pl.pr, G.n};
+          metro_rows<NC, UNI, Z>(pv_s, b, cnt, qm + pl.pq, c, s_pid, T, beta.at(pv.x, __float_as_int(pv.w)), pv.y, kk,
+                                 key0, __float_as_uint(pv.z), pe, pm);
+          // the first pool group after a tail stores, later ones add
+          double* pp = pl.pp + threadIdx.x;
+          const bool first = pfresh && c == 0;
+          pp[0] = first ? (double)pe : pp[0] + (double)pe;
 #pragma unroll
-        for (int k = 1; k <= NC; ++k) pp[k * pl.nr] = first ? (double)pm[k - 1] : pp[k * pl.nr] + (double)pm[k - 1];
-      }
-      for (int j = q - qm; j < nx; j += TPR)
-        metro_group_pat<NC, ST, UNI>(sp, b, cnt, xl[j], c, s_pid, s_pat, zmax, cp, clsdat, beta, h, kk, key0, key1,
-                                     xE, xM, aniso);
+          for (int k = 1; k <= NC; ++k) pp[k * pl.nr] = first ? (double)pm[k - 1] : pp[k * pl.nr] + (double)pm[k - 1];
+        }
+        for (int j = q - qm; j < nx; j += TPR)
+          metro_rows<NC, UNI, Z>(v, b, cnt, xl[j], c, s_pid, T, beta, h, kk, key0, key1, xE, xM);
+      });
     } else if constexpr (MODE == 1) {
       const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
       if (G.ucid >= 0) {
-        const float* cp = coup + G.ucid * 9;
+        const float* cp = coup + G.ucid * COUP_LDS;
         int q = q0 + lt;
         for (; q < q1; q += TPR)
-          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, gas(G.cls), clsdat, beta, h, kk, key0,
+          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0,
                                 key1, fE, fM);
         for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, gas(G.cls), clsdat, beta, h, kk,
+          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, COUP_LDS, gas(G.cls), clsdat, beta, h, kk,
                                 key0, key1, xE, xM);
       } else {
         int q = q0 + lt;
         for (; q < q1; q += TPR)
-          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, coup, gas(G.cls), clsdat, beta, h, kk, key0, key1,
+          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, coup, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0, key1,
                           fE, fM);
         for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, coup, gas(G.cls), clsdat, beta, h, kk, key0,
+          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, coup, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0,
                           key1, xE, xM);
       }
     } else {
@@ -1848,18 +2040,18 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
       if (uni) {
         int q = q0 + lt;
         for (; q < q1; q += TPR)
-          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, gas(G.cls), gas(clsdat), beta, h, kk,
+          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk,
                                 key0, key1, fE, fM);
         for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, gas(G.cls), gas(clsdat), beta, h,
+          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h,
                                 kk, key0, key1, xE, xM);
       } else {
         int q = q0 + lt;
         for (; q < q1; q += TPR)
-          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, gas(G.cls), gas(clsdat), beta, h, kk, key0,
+          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk, key0,
                           key1, fE, fM);
         for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, gas(G.cls), gas(clsdat), beta, h, kk,
+          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk,
                           key0, key1, xE, xM);
       }
     }
@@ -1922,7 +2114,9 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   const mcg_graph G = B.graphs[w.graph];
   const int R = w.nrep;
   const int TPR = blockDim.x / R;
-  const int g = threadIdx.x / TPR;
+  // a group is whole waves, so its index, and with it the replica's record,
+  // row, keys, couplings and LDS base, are scalars
+  const int g = wave_uniform((int)threadIdx.x / TPR);
   const int lt = threadIdx.x - g * TPR;
   const ItemRep ir = recs[w.off + g];
   const int rep = ir.rep;
@@ -1938,8 +2132,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   extern __shared__ __align__(16) unsigned char smem[];
   size_t off = 0;
   float* s_coup = (float*)smem;
-  float* s_clsl = s_coup + ncl * 9;
-  off += align16((size_t)(ncl * 9 + ncs * 8) * 4);
+  float* s_clsl = s_coup + ncl * COUP_LDS;
+  off += align16((size_t)(ncl * COUP_LDS + ncs * 8) * 4);
   int32_t* s_colptr = (int32_t*)(smem + off);
   off += align16((size_t)(G.ncol + 1) * 4);
   int32_t* s_pat = (int32_t*)(smem + off);
@@ -1957,7 +2151,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   if (PERSIST) off += persist_lds_bytes(B.nrow, B.nrep);
   ST* s_spin = (ST*)(smem + off);
 
-  for (int t = threadIdx.x; t < ncl * 9; t += blockDim.x) s_coup[t] = G.coup[t];
+  for (int t = threadIdx.x; t < ncl * 9; t += blockDim.x) s_coup[t / 9 * COUP_LDS + t % 9] = G.coup[t];
   for (int t = threadIdx.x; t < ncs * 8; t += blockDim.x) s_clsl[t] = G.clsdat[t];
   // does any site class carry an on-site term? (metro_core skips them if not)
   int anz = 0;
@@ -1968,10 +2162,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   if (perm) {
     for (int t = threadIdx.x; t < G.npat * (zmax + 1); t += blockDim.x) {
       const int l = t % (zmax + 1);
-      int32_t v = G.pattab[t];
-      // uniform graphs: links as byte offsets between spins (PatOffLinks)
-      if (MODE == 3 && l < zmax) v = ((int32_t)((uint32_t)v << 8) >> 8) * (int32_t)sizeof(ST);
-      s_pat[(t / (zmax + 1)) * pat_stride(zmax) + l] = v;
+      const int32_t v = G.pattab[t];
+      s_pat[(t / (zmax + 1)) * pat_stride(zmax) + l] = l < zmax ? row_word<MODE == 3>(v, sizeof(ST)) : v;
     }
     for (int t = threadIdx.x; t < n; t += blockDim.x) s_pid[t] = G.pat[t];
   }
@@ -2015,7 +2207,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
     pi.hx = a.halo + w.hoff;
     pi.halo = a.halo;
   }
-  FrameCtx C{&G, wide ? G.coup : s_coup, wide ? G.clsdat : s_clsl, s_red, s_frm + g * FRM, g, lt, TPR};
+  FrameCtx C{B.graphs + w.graph, wide ? G.coup : s_coup, wide ? 9 : COUP_LDS, wide ? G.clsdat : s_clsl, s_red, s_frm + g * FRM, g, lt, TPR};
   if constexpr (PERSIST) {
     // Persistent launch: many sweeps with the replicas in LDS.  After each
     // sweep every replica's energy is published at the device coherence
@@ -2103,8 +2295,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       const int64_t k = a.k_begin + s;
       const uint64_t kk = (uint64_t)(a.philox_base + k);
       const int par = (int)(k & 1);
-      const int rowg = ir.row0 + s_rung[rep];
-      const float bg = s_beta[rowg], hg = s_h[rowg];
+      const int rowg = wave_uniform(ir.row0 + s_rung[rep]);
+      const float bg = wave_uniform(s_beta[rowg]), hg = wave_uniform(s_h[rowg]);
       const bool meas = k >= a.nthermal && ((k - a.nthermal + 1) % a.spf) == 0;
       const bool therm_end = (k + 1 == a.nthermal);
       const bool rec = !a.rec_host && recompute_due(B, a.philox_base + k);
@@ -2129,7 +2321,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
                        rec ? nullptr : a.eslot + (size_t)par * nrepb * MAX_PARTS, s_frm, pl.rem);
         if (rec) {
           double r4[NREC];
-          recompute<NC>(sp, G, C.coup, C.clsdat, hg, s_red, g, lt, TPR, r4);
+          recompute<NC>(sp, C.G, C.coup, C.cst, C.clsdat, hg, s_red, g, lt, TPR, r4);
           if (lt == 0) {
             const double d = fabs(st[MCG_S_E] - r4[0]);
             if (d > st[MCG_S_DRIFT]) st[MCG_S_DRIFT] = d;
@@ -2175,7 +2367,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
         }
       }
       if (meas && l_grp && !frames_after) {
-        take_frame<NC>(G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, frame_mprev3<NC>(a, fcur, rowg_l, nrow),
+        take_frame<NC>(C.G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, frame_mprev3<NC>(a, fcur, rowg_l, nrow),
                        fflags);
         last_row = rowg_l;
       }
@@ -2284,7 +2476,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       // the frame of every replica (first wave, lane g), while the other
       // waves run the tempering pass
       if (meas && l_grp && frames_after) {
-        take_frame<NC>(G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, mp, fflags);
+        take_frame<NC>(C.G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, mp, fflags);
         last_row = rowg_l;
       }
       if (pt_now) {
@@ -2455,7 +2647,16 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
 #define MCG_PASS_UNROLL 1
 #endif
 static constexpr int PASS_GPT = MCG_PASS_GPT;
-static constexpr int PASS_PAT_INTS = 4096;  // LDS for pattern rows (16 KB)
+static constexpr int PASS_PAT_INTS = 4096;  // most LDS for pattern rows (16 KB)
+// the pass uses link patterns, and its LDS for them: rows, and the couplings
+// of graphs that have several
+__host__ __device__ inline bool pass_patterns(const mcg_graph& G) {
+  return G.npat > 0 && G.lcid == nullptr && G.npat * pat_stride(G.zmax) <= PASS_PAT_INTS;
+}
+__host__ __device__ inline size_t pass_lds_bytes(const mcg_graph& G) {
+  return pass_patterns(G) ? (size_t)G.npat * pat_stride(G.zmax) * 4 + (G.ucid >= 0 ? 0 : (size_t)G.ncoup * COUP_LDS * 4)
+                          : 0;
+}
 // Workgroups are dealt to the 8 XCDs in turn (workgroup b to XCD b % 8),
 // and each XCD has its own L2.  xcd_item maps workgroup b to a work item so
 // that every XCD takes one contiguous run of the `total` items: the items of
@@ -2479,7 +2680,7 @@ __host__ __device__ inline int xcd_grid(int total) { return (total + NXCD - 1) /
 template <int NC, typename ST>
 __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, const int32_t* __restrict__ rep_list, int colour,
                                               int64_t sweep, int nchunk, int nitems) {
-  __shared__ int32_t s_pat[PASS_PAT_INTS];
+  extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double s_red[4 * 4];
   const int item = xcd_item(blockIdx.x, nitems);
   if (item < 0) return;  // the whole workgroup
@@ -2488,12 +2689,20 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
   const mcg_replica rp = B.reps[rep];
   const mcg_graph G = B.graphs[rp.graph];
   const int zmax = G.zmax;
-  const bool pats = G.npat > 0 && G.lcid == nullptr && G.npat * pat_stride(zmax) <= PASS_PAT_INTS;
+  const bool pats = pass_patterns(G), uni = G.ucid >= 0;
+  int32_t* s_pat = (int32_t*)smem;
+  float* s_coup = (float*)(s_pat + G.npat * pat_stride(zmax));
   int anz = 0;
   if (pats) {
-    for (int t = threadIdx.x; t < G.npat * (zmax + 1); t += blockDim.x)
-      s_pat[(t / (zmax + 1)) * pat_stride(zmax) + t % (zmax + 1)] = G.pattab[t];
-    // does any site class carry an on-site term? (metro_core skips them if not)
+    for (int t = threadIdx.x; t < G.npat * (zmax + 1); t += blockDim.x) {
+      const int l = t % (zmax + 1);
+      const int32_t w = G.pattab[t];
+      s_pat[t / (zmax + 1) * pat_stride(zmax) + l] =
+          l == zmax ? w : uni ? row_word<true>(w, sizeof(ST)) : row_word<false>(w, sizeof(ST));
+    }
+    if (!uni)
+      for (int t = threadIdx.x; t < G.ncoup * 9; t += blockDim.x) s_coup[t / 9 * COUP_LDS + t % 9] = G.coup[t];
+    // does any site class carry an on-site term? (the D terms are skipped if not)
     for (int t = threadIdx.x; t < G.ncls; t += blockDim.x)
       anz |= (G.clsdat[t * 8 + 1] != 0.0f) | (G.clsdat[t * 8 + 2] != 0.0f) | (G.clsdat[t * 8 + 3] != 0.0f);
   }
@@ -2503,29 +2712,50 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
     const int b = G.col_ptr[colour], cnt = G.col_ptr[colour + 1] - b;
     const int ngrp = (cnt + SitesPerDraw<NC>::G - 1) / SitesPerDraw<NC>::G;
     const int row = rp.row0 + B.rung[rep];
-    const float h = B.row_h[row];
-    const Acc beta = acc_of(B, B.row_beta[row], row);
+    const float h = in_vgpr(B.row_h[row]);
+    const Acc beta = acc_of(B, in_vgpr(B.row_beta[row]), row);
     const uint32_t key1 = B.seed_hi ^ rp.serial;
-    const GSpins<ST> sp{gas((ST*)B.spins + rp.spin_off), G.n};
-    const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
+    GAS ST* spins = gas((ST*)B.spins + rp.spin_off);
+    const int q0 = chunk * PASS_GPT * (int)blockDim.x + (int)threadIdx.x;
+    auto groups = [&](auto&& update) {
 #pragma unroll MCG_PASS_UNROLL
-    for (int u = 0; u < PASS_GPT; ++u) {
-      const int q = (chunk * PASS_GPT + u) * (int)blockDim.x + (int)threadIdx.x;
-      if (q >= ngrp) break;
-      if (pats) {
-        if (G.ucid >= 0)
-          metro_group_gpat<NC, ST, true>(sp, b, cnt, q, colour, gas(G.pat), s_pat, zmax, gas(G.coup) + G.ucid * 9,
-                                         gas(G.clsdat), beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM, aniso);
-        else
-          metro_group_gpat<NC, ST, false>(sp, b, cnt, q, colour, gas(G.pat), s_pat, zmax, gas(G.coup),
-                                          gas(G.clsdat), beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM, aniso);
-      } else if (G.ucid >= 0) {
-        metro_group<NC, true>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup) + G.ucid * 9, gas(G.cls),
-                              gas(G.clsdat), beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
-      } else {
-        metro_group<NC>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup), gas(G.cls), gas(G.clsdat),
-                        beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
+      for (int u = 0; u < PASS_GPT; ++u) {
+        const int q = q0 + u * (int)blockDim.x;
+        if (q >= ngrp) break;
+        update(q);
       }
+    };
+    if (pats) {
+      const HbmView<NC, ST> v(spins, G.n);
+      const GAS uint8_t* pat = gas(G.pat);
+      auto rows = [&](auto uc) {
+        constexpr bool UNI = decltype(uc)::value;
+        RowTab<NC, const GAS float*> T;
+        row_tab<NC, UNI>(T, s_pat, s_coup, gas(G.coup) + (UNI ? G.ucid * 9 : 0), gas(G.clsdat), zmax, G.ncls, aniso);
+        with_links<UNI>(T, [&](auto zc) {
+          groups([&](int q) {
+            metro_rows<NC, UNI, decltype(zc)::value>(v, b, cnt, q, colour, pat, T, beta, h, (uint64_t)sweep, B.seed_lo,
+                                                     key1, dE, dM);
+          });
+        });
+      };
+      if (uni)
+        rows(std::true_type());
+      else
+        rows(std::false_type());
+    } else {
+      const GSpins<ST> sp{spins, G.n};
+      const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
+      if (uni)
+        groups([&](int q) {
+          metro_group<NC, true>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup) + G.ucid * 9, 9, gas(G.cls),
+                                gas(G.clsdat), beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
+        });
+      else
+        groups([&](int q) {
+          metro_group<NC>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup), 9, gas(G.cls), gas(G.clsdat),
+                          beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
+        });
     }
   }
   // every lane reaches here: DPP sums per wave, the waves' totals through LDS
@@ -2564,7 +2794,7 @@ __global__ __launch_bounds__(1024) void k_measure(mcg_batch B, const int32_t* __
   __syncthreads();
   if (mode & 1) {
     double r4[NREC];
-    recompute<NC>(sp, G, G.coup, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r4);
+    recompute<NC>(sp, B.graphs + rp.graph, G.coup, 9, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r4);
     if (threadIdx.x == 0) {
       double d = 0.0;
       if (!(mode & 8)) {
@@ -2581,7 +2811,7 @@ __global__ __launch_bounds__(1024) void k_measure(mcg_batch B, const int32_t* __
   if ((mode & 2) && threadIdx.x == 0) st[MCG_S_EREF] = st[MCG_S_E];
   __syncthreads();
   if (mode & 4) {
-    FrameCtx C{&G, G.coup, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
+    FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
     measure_frame<NC>(sp, C, B, st, row, frame, B.seed_lo, B.seed_hi ^ rp.serial, h);
   }
   __syncthreads();
@@ -2614,7 +2844,7 @@ __global__ __launch_bounds__(256) void k_frame_part(mcg_batch B, const int32_t* 
   double* out = fsum + (size_t)rep * FSLOTS;
   if (mode & 1) {
     double r[NREC];
-    recompute<NC>(sp, G, G.coup, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r, part, np);
+    recompute<NC>(sp, B.graphs + rp.graph, G.coup, 9, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r, part, np);
     if (threadIdx.x == 0)
       for (int k = 0; k < NREC; ++k)
         if (r[k] != 0.0) atomicAdd(out + FSUMS + k, r[k]);
@@ -2622,7 +2852,7 @@ __global__ __launch_bounds__(256) void k_frame_part(mcg_batch B, const int32_t* 
   if (mode & 4) {
     for (int t = threadIdx.x; t < FSUMS; t += blockDim.x) s_frm[t] = 0.0;
     __syncthreads();
-    FrameCtx C{&G, G.coup, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
+    FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
     frame_sums<NC>(sp, C, B, frame, B.seed_lo, B.seed_hi ^ rp.serial, h, part, np);
     if (threadIdx.x == 0)
       for (int k = 0; k < FSUMS; ++k)
@@ -2659,7 +2889,7 @@ __global__ __launch_bounds__(64) void k_frame_end(mcg_batch B, const int32_t* __
   if ((mode & 2) && lt == 0) st[MCG_S_EREF] = st[MCG_S_E];
   __syncthreads();
   if (mode & 4) {
-    FrameCtx C{&G, G.coup, G.clsdat, s_red, s_frm, 0, lt, (int)blockDim.x};
+    FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, lt, (int)blockDim.x};
     frame_apply<NC>(C, B, st, row, frame, B.meas, 0.0, false, false);
   }
   __syncthreads();
@@ -3021,6 +3251,7 @@ struct RunCtx {
   double lds_updates_per_sweep = 0;
   int device = 0;
   int stream_ncol = 0, stream_maxcnt = 0;  // colours and largest colour class of the streamed graphs
+  uint32_t stream_lds = 0;                 // LDS of the streaming pass (pattern rows, couplings)
   int frame_np_stream = 1, frame_np_all = 1;  // workgroups per replica of the split measurement
   bool frame_spins = true;  // a measured frame reads spins (launch_frame)
   // what the plan was made for: a run whose plan or batch differs in any of
@@ -3525,14 +3756,14 @@ int check_persist(const mcg_batch* B, const mcg_plan* P, RunCtx& X, bool* ok) {
 
 
 template <int NC, typename ST>
-int launch_pass(const mcg_batch* B, const int32_t* dreps, int nreps, int maxcnt, int colour, int64_t sweep,
+int launch_pass(const mcg_batch* B, const int32_t* dreps, int nreps, int maxcnt, uint32_t lds, int colour, int64_t sweep,
                 hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   if (nreps == 0) return 0;
   const int ngrp = (maxcnt + SitesPerDraw<NC>::G - 1) / SitesPerDraw<NC>::G;
   const int chunks = std::max(1, (ngrp + 256 * PASS_GPT - 1) / (256 * PASS_GPT));
   const int64_t items = (int64_t)chunks * nreps;
   if (items > (1 << 30)) return fail("streaming pass: %lld work items", (long long)items);
-  hipExtLaunchKernelGGL((k_pass<NC, ST>), dim3((unsigned)xcd_grid((int)items)), dim3(256), 0, s, e0, e1, 0, *B, dreps,
+  hipExtLaunchKernelGGL((k_pass<NC, ST>), dim3((unsigned)xcd_grid((int)items)), dim3(256), lds, s, e0, e1, 0, *B, dreps,
                         colour, sweep, chunks, (int)items);
   HIPCHK(hipGetLastError());
   return 0;
@@ -3606,12 +3837,12 @@ int stream_sweeps(const mcg_batch* B, const mcg_plan* P, RunCtx& X, int64_t k0, 
       if (plain) {
         for (int i = 0; i < nrs; ++i) {
           hipEvent_t e0, e1;
-          if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps + i, 1, maxn, c, kk, s, e0, e1)) return -1;
+          if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps + i, 1, maxn, X.stream_lds, c, kk, s, e0, e1)) return -1;
           T.launches += 1;
         }
       } else {
         hipEvent_t e0, e1;
-        if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps, nrs, maxn, c, kk, s, e0, e1)) return -1;
+        if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps, nrs, maxn, X.stream_lds, c, kk, s, e0, e1)) return -1;
         T.launches += 1;
       }
     }
@@ -3674,6 +3905,7 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   }
   // colour classes of the streamed graphs (the streaming grid covers the largest)
   X.stream_ncol = X.stream_maxcnt = 0;
+  X.stream_lds = 0;
   {
     std::vector<char> seen(B->ngraph, 0);
     for (int r : X.hstream) {
@@ -3684,6 +3916,7 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
       std::vector<int32_t> cp(G.ncol + 1);
       HIPCHK(hipMemcpy(cp.data(), G.col_ptr, cp.size() * 4, hipMemcpyDeviceToHost));
       X.stream_ncol = std::max(X.stream_ncol, G.ncol);
+      X.stream_lds = std::max(X.stream_lds, (uint32_t)pass_lds_bytes(G));
       for (int c = 0; c < G.ncol; ++c) X.stream_maxcnt = std::max(X.stream_maxcnt, cp[c + 1] - cp[c]);
     }
   }
