@@ -302,60 +302,6 @@ __device__ __forceinline__ bool ising_decide(float s, float f, float h, const Ac
   return (db <= 0.0f) | below_exp(w_c, -db);
 }
 
-template <int NC, typename SV, typename LK, typename CP, bool UNI = false>
-__device__ __forceinline__ void metro_core(const SV& sp, int i, const LK& lk, int zmax, CP coup, int cst, int ci,
-                                           CP clsdat, Acc ac, float h, uint32_t w_a, uint32_t w_b, uint32_t w_c,
-                                           float& dEacc, float* dMacc, bool aniso = true) {
-  if constexpr (NC == 1) {
-    const float S = clsdat[ci * 8 + 0];
-    float f = 0.0f;
-    if constexpr (UNI) {
-      float m = 0.0f;
-      for (int l = 0; l < zmax; ++l) m += sp.get(lk.nbr(l), 0);
-      f = coup[0] * m;
-    } else {
-      for (int l = 0; l < zmax; ++l) f = fmaf(coup[lk.cid(l) * cst], sp.get(lk.nbr(l), 0), f);
-    }
-    const float sg = sp.get(i, 0);
-    const float s = sg * S;
-    float dE;
-    if (ising_decide(s, f, h, ac, w_c, dE)) {
-      sp.set(i, 0, -sg);
-      dEacc += dE;
-      dMacc[0] += -2.0f * s;
-    }
-  } else {
-    const float s[3] = {sp.get(i, 0), sp.get(i, 1), NC == 3 ? sp.get(i, 2) : 0.0f};
-    float H[3] = {0.0f, 0.0f, 0.0f};
-    if constexpr (UNI) {
-      float S0 = 0.0f, S1 = 0.0f, S2 = 0.0f;
-      for (int l = 0; l < zmax; ++l) {
-        const int j = lk.nbr(l);
-        S0 += sp.get(j, 0);
-        S1 += sp.get(j, 1);
-        if constexpr (NC == 3) S2 += sp.get(j, 2);
-      }
-      const float S[3] = {S0, S1, S2};
-      uniform_field<NC>(coup, S, H);
-    } else {
-      for (int l = 0; l < zmax; ++l) {
-        const int j = lk.nbr(l);
-        const CP J = coup + lk.cid(l) * cst;
-        const float t[3] = {sp.get(j, 0), sp.get(j, 1), NC == 3 ? sp.get(j, 2) : 0.0f};
-        add_field<NC>(J, t, H);
-      }
-    }
-    float r[3], n[3], dE;
-    metro_axis<NC>(w_a, w_b, r);
-    const float D[3] = {clsdat[ci * 8 + 1], clsdat[ci * 8 + 2], clsdat[ci * 8 + 3]};
-    if (metro_decide<NC>(s, H, r, ac.beta, h, aniso, D, w_c, n, dE)) {
-      metro_commit<NC, typename SV::value_type>(s, n, clsdat[ci * 8 + 4], dMacc);
-      for (int k = 0; k < NC; ++k) sp.set(i, k, n[k]);
-      dEacc += dE;
-    }
-  }
-}
-
 // One Philox draw (128 bits) serves G sites of a colour class: 4 Ising
 // updates (one acceptance word each), 2 XY updates (angle + acceptance), or
 // 1 Heisenberg update (r_z, angle, acceptance).  Group q of colour c covers
@@ -364,32 +310,6 @@ template <int NC>
 struct SitesPerDraw {
   static constexpr int G = NC == 1 ? 4 : NC == 2 ? 2 : 1;
 };
-
-template <int NC, bool UNI = false, typename SV, typename CP>
-__device__ __forceinline__ void metro_group(const SV& sp, int b, int cnt, int q, int colour,
-                                            const GAS uint32_t* __restrict__ link,
-                                            const GAS int32_t* __restrict__ lcid, int zmax, CP coup, int cst,
-                                            const GAS int32_t* __restrict__ cls, CP clsdat, Acc beta, float h,
-                                            uint64_t sweep, uint32_t key0, uint32_t key1, float& dEacc,
-                                            float* dMacc) {
-  constexpr int G = SitesPerDraw<NC>::G;
-  const u32x4 x = philox4x32_10(
-      u32x4{(uint32_t)q, (uint32_t)sweep, (uint32_t)(sweep >> 32), TAG_METRO | ((uint32_t)colour << 8)}, key0, key1);
-  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int p = q * G + g;
-    if (p < cnt) {
-      const int i = b + p;
-      const GlobalLinks lk{link + (size_t)i * zmax, lcid ? lcid + (size_t)i * zmax : nullptr};
-      const uint32_t wa = NC == 3 ? w[0] : 0u;
-      const uint32_t wb = NC == 3 ? w[1] : NC == 2 ? w[2 * g] : 0u;
-      const uint32_t wc = NC == 3 ? w[2] : NC == 2 ? w[2 * g + 1] : w[g];
-      metro_core<NC, SV, GlobalLinks, CP, UNI>(sp, i, lk, zmax, coup, cst, (int)cls[i], clsdat, beta, h, wa, wb, wc,
-                                               dEacc, dMacc);
-    }
-  }
-}
 
 // One replica's spins, in LDS or in HBM: a site's place, and loads and stores
 // at a byte offset from it.  In LDS a place is one address per component (a
@@ -410,6 +330,7 @@ struct LdsView {
     for (int k = 0; k < NC; ++k) s.a[k] = (char*)(p + i) + k * n * (int)sizeof(ST);
     return s;
   }
+  __device__ __forceinline__ Site base() const { return at(0); }
   static __device__ __forceinline__ float ld(const Site& s, int k, int off) { return SIO<ST>::ld((const ST*)(s.a[k] + off)); }
   static __device__ __forceinline__ void st(const Site& s, int k, float v) { SIO<ST>::st((ST*)s.a[k], v); }
 };
@@ -427,55 +348,53 @@ struct HbmView {
     }
   }
   __device__ __forceinline__ Site at(int i) const { return (uint32_t)i * (uint32_t)sizeof(ST); }
+  __device__ __forceinline__ Site base() const { return 0; }
   __device__ __forceinline__ float ld(const Site& s, int k, int off) const {
     return SIO<ST>::ld((const GAS ST*)((const GAS char*)p[k] + (s + (uint32_t)off)));
   }
   __device__ __forceinline__ void st(const Site& s, int k, float v) const { SIO<ST>::st((GAS ST*)((GAS char*)p[k] + s), v); }
 };
 
-// What the updates of a sweep read besides spins and draws, for graphs with
-// link patterns.  coup, clsdat: LDS (COUP_LDS floats a tensor), or HBM for
-// the classes of the streaming pass.  With one coupling or one site class
-// their values are kept in registers: read where they are used, each update
-// would wait for them.
-template <int NC, typename CP>
-struct RowTab {
+// What the updates of a sweep read besides spins and draws.  Neighbours come
+// from link patterns (rows in LDS, pat: the row of each position) or from the
+// global link table (link, lcid).  coup (cst floats a tensor), clsdat: LDS or
+// HBM.  With one coupling or one site class their values are kept in
+// registers: read where they are used, each update would wait for them.
+template <int NC, typename PP, typename KP, typename CP>
+struct SweepTab {
   const int32_t* rows;
-  const float* coup;
+  int stride;  // bytes per row
+  PP pat;
+  const GAS uint32_t* link;
+  const GAS int32_t *lcid, *cls;
+  KP coup;
+  int cst;
   CP clsdat;
-  int zmax, stride;  // stride: bytes per row
+  int zmax;
   bool aniso, one;  // any on-site term; one site class
   float J[9];       // the coupling of a uniform graph
   float cls0[5];    // the one class: S, D, 1/S^2
 };
-template <int NC, bool UNI, typename JP, typename CP>
-__device__ __forceinline__ void row_tab(RowTab<NC, CP>& T, const int32_t* rows, const float* coup, JP ucoup, CP clsdat,
-                                        int zmax, int ncls, bool aniso) {
+template <int NC, bool UNI, typename PP, typename KP, typename CP, typename JP>
+__device__ __forceinline__ SweepTab<NC, PP, KP, CP> sweep_tab(const mcg_graph& G, const int32_t* rows, PP pat, KP coup,
+                                                              int cst, JP ucoup, CP clsdat, bool aniso) {
+  SweepTab<NC, PP, KP, CP> T;
   T.rows = rows;
+  T.stride = pat_stride(G.zmax) * 4;
+  T.pat = pat;
+  T.link = gas(G.link);
+  T.lcid = G.lcid ? gas(G.lcid) : nullptr;
+  T.cls = gas(G.cls);
   T.coup = coup;
+  T.cst = cst;
   T.clsdat = clsdat;
-  T.zmax = zmax;
-  T.stride = pat_stride(zmax) * 4;
+  T.zmax = G.zmax;
   T.aniso = aniso;
-  T.one = ncls == 1;
+  T.one = G.ncls == 1;
   if constexpr (UNI)
     for (int k = 0; k < 9; ++k) T.J[k] = in_vgpr(ucoup[k]);
   for (int k = 0; k < 5; ++k) T.cls0[k] = in_vgpr(clsdat[k]);
-}
-
-// the coupling of a pattern row's link word (graphs of several couplings)
-template <int NC>
-__device__ __forceinline__ void link_coup(const float* coup, int32_t w, float* J) {
-  const float* c = coup + __umul24((uint32_t)w & 0xFFu, COUP_LDS);
-  if constexpr (NC == 1) {
-    J[0] = c[0];
-  } else {
-    const float4 a = *(const float4*)c, b = *(const float4*)(c + 4);
-    J[0] = a.x; J[1] = a.y; J[2] = a.z; J[3] = a.w; J[4] = b.x;
-    if constexpr (NC == 3) {
-      J[5] = b.y; J[6] = b.z; J[7] = b.w; J[8] = c[8];
-    }
-  }
+  return T;
 }
 
 // four words of a pattern row
@@ -495,34 +414,78 @@ __device__ __forceinline__ void sum_field(const T& tab, const float* S, float* H
     uniform_field<NC>(tab.J, S, H);
 }
 
-// Field of the site at `own`, its pattern row given: every
-// neighbour is read before the first is used.  Z: the number of links, or 0
-// where it is only known at run time (then four links at a time).
-template <int NC, bool UNI, int Z, typename V, typename CP>
-__device__ __forceinline__ void row_field(const V& v, const typename V::Site& own, const int32_t* row,
-                                          const RowTab<NC, CP>& T, float* H) {
+// one coupling of a graph of several: 128-bit reads from LDS
+template <int NC>
+__device__ __forceinline__ void read_coup(const float* c, float* J) {
+  if constexpr (NC == 1) {
+    J[0] = c[0];
+  } else {
+    const float4 a = *(const float4*)c, b = *(const float4*)(c + 4);
+    J[0] = a.x; J[1] = a.y; J[2] = a.z; J[3] = a.w; J[4] = b.x;
+    if constexpr (NC == 3) {
+      J[5] = b.y; J[6] = b.z; J[7] = b.w; J[8] = c[8];
+    }
+  }
+}
+template <int NC>
+__device__ __forceinline__ void read_coup(const GAS float* c, float* J) {
+#pragma unroll
+  for (int k = 0; k < (NC == 1 ? 1 : NC == 2 ? 5 : 9); ++k) J[k] = c[k];
+}
+
+// the next B link words of a site from link l on: pattern row words, or the
+// link table's (neighbour | coupling << 24)
+template <bool PAT, int B, typename T>
+__device__ __forceinline__ void link_words(const T& tab, const int32_t* row, const GAS uint32_t* lk, int l, int zmax,
+                                           int32_t* w) {
+  if constexpr (PAT) {
+#pragma unroll
+    for (int u = 0; u < B; u += 4) read_row(row + l + u, w + u);
+  } else {
+#pragma unroll
+    for (int u = 0; u < B; ++u) w[u] = (int32_t)lk[l + u < zmax ? l + u : zmax - 1];
+  }
+}
+// the neighbour of a link word
+template <bool PAT, bool UNI, typename V>
+__device__ __forceinline__ float link_spin(const V& v, const typename V::Site& own, int32_t w, int k) {
   typedef typename V::value_type ST;
+  if constexpr (PAT)
+    return v.ld(own, k, UNI ? w : (w >> 8) * (int)sizeof(ST));
+  else
+    return v.ld(v.base(), k, (int)(((uint32_t)w & 0xFFFFFFu) * (uint32_t)sizeof(ST)));
+}
+
+// Field of the site at `own` (its pattern row, or its link table row lk and
+// coupling row lc): every neighbour is read before the first is used.  Z: the
+// number of links, or 0 where it is only known at run time (then four links
+// at a time).
+template <int NC, bool PAT, bool UNI, int Z, typename V, typename T>
+__device__ __forceinline__ void site_field(const V& v, const typename V::Site& own, const int32_t* row,
+                                           const GAS uint32_t* lk, const GAS int32_t* lc, const T& tab, float* H) {
   constexpr int B = Z == 0 ? 4 : Z == 9 ? 3 : Z;  // links per batch
-  const int zmax = Z > 0 ? Z : T.zmax;
+  const int zmax = Z > 0 ? Z : tab.zmax;
   float S[3] = {0.0f, 0.0f, 0.0f};
   H[0] = H[1] = H[2] = 0.0f;
   int32_t rw[Z > 0 ? (Z + 3) / 4 * 4 : 4];
-  if constexpr (Z > 0)
-#pragma unroll
-    for (int u = 0; u < Z; u += 4) read_row(row + u, rw + u);
+  if constexpr (Z > 0) link_words<PAT, Z>(tab, row, lk, 0, Z, rw);
   for (int l0 = 0; l0 < zmax; l0 += B) {
     int32_t w[B];
-    if constexpr (Z == 0) read_row(row + l0, rw);
-#pragma unroll
-    for (int u = 0; u < B; ++u) w[u] = rw[Z > 0 ? l0 + u : u];
-    float t[B][NC];
+    if constexpr (Z == 0) link_words<PAT, 4>(tab, row, lk, l0, zmax, rw);
+    uint32_t c[B];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-      if (Z == 0 && l0 + u >= zmax) w[u] = 0;  // past the last link: the site itself, not used
-      const int o = UNI ? w[u] : (w[u] >> 8) * (int)sizeof(ST);
-#pragma unroll
-      for (int k = 0; k < NC; ++k) t[u][k] = v.ld(own, k, o);
+      w[u] = rw[Z > 0 ? l0 + u : u];
+      if (PAT && Z == 0 && l0 + u >= zmax) w[u] = 0;  // past the last link: the site itself, not used
+      if constexpr (!UNI)
+        c[u] = PAT ? (uint32_t)w[u] & 0xFFu
+                   : lc ? (uint32_t)lc[l0 + u < zmax ? l0 + u : zmax - 1] : (uint32_t)w[u] >> 24;
     }
+    float t[B][NC];
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+#pragma unroll
+      for (int k = 0; k < NC; ++k) t[u][k] = link_spin<PAT, UNI>(v, own, w[u], k);
     if constexpr (UNI) {
 #pragma unroll
       for (int u = 0; u < B; ++u) {
@@ -534,10 +497,10 @@ __device__ __forceinline__ void row_field(const V& v, const typename V::Site& ow
       // each link's tensor is read while the one before it is used (all at
       // once would take 9 registers a link)
       float J[2][9];
-      link_coup<NC>(T.coup, w[0], J[0]);
+      read_coup<NC>(tab.coup + c[0] * tab.cst, J[0]);
 #pragma unroll
       for (int u = 0; u < B; ++u) {
-        if (u + 1 < B && (Z > 0 || l0 + u + 1 < zmax)) link_coup<NC>(T.coup, w[u + 1], J[(u + 1) & 1]);
+        if (u + 1 < B && (Z > 0 || l0 + u + 1 < zmax)) read_coup<NC>(tab.coup + c[u + 1] * tab.cst, J[(u + 1) & 1]);
         if (Z == 0 && l0 + u >= zmax) break;
         if constexpr (NC == 1)
           H[0] = fmaf(J[u & 1][0], t[u][0], H[0]);
@@ -549,23 +512,26 @@ __device__ __forceinline__ void row_field(const V& v, const typename V::Site& ow
       }
     }
   }
-  if constexpr (UNI) sum_field<NC>(T, S, H);
+  if constexpr (UNI) sum_field<NC>(tab, S, H);
 }
 
-// The sites of one draw (group q of a colour class of cnt positions from b
-// on), on a graph with link patterns.  They share a colour, so none is
-// another's neighbour: all fields are read, then all decisions taken, then
-// the accepted spins stored, and the sites' loads overlap instead of each
-// site waiting for its own chain.  Changes are added in site order.
-template <int NC, bool UNI, int Z, typename V, typename PP, typename CP>
-__device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, int colour, PP pat,
-                                           const RowTab<NC, CP>& T, const Acc& ac, float h, uint64_t sweep,
-                                           uint32_t key0, uint32_t key1, float& dEacc, float* dMacc) {
+// The sites of one draw: group q of a colour class of cnt positions from b
+// on.  They share a colour, so none is another's neighbour: all fields are
+// read, then all decisions taken, then the accepted spins stored, and the
+// sites' loads overlap instead of each site waiting for its own chain.
+// Changes are added in site order.  PAT: neighbours from link patterns,
+// otherwise from the link table.
+template <int NC, bool PAT, bool UNI, int Z, typename V, typename T>
+__device__ __forceinline__ void metro_sites(const V& v, int b, int cnt, int q, int colour, const T& tab, const Acc& ac,
+                                            float h, uint64_t sweep, uint32_t key0, uint32_t key1, float& dEacc,
+                                            float* dMacc) {
   typedef typename V::value_type ST;
   constexpr int G = SitesPerDraw<NC>::G;
   typename V::Site own[G];
   float s[G][3], H[G][3];
   const int32_t* row[G];
+  const GAS uint32_t* lk[G];
+  const GAS int32_t* lc[G];
   int cl[G];
   bool live[G];
 #pragma unroll
@@ -573,25 +539,34 @@ __device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, in
     const int lp = q * G + g;
     live[g] = lp < cnt;  // the last group may be short: its missing sites read the last one
     const int p = b + (G == 1 || live[g] ? lp : cnt - 1);
-    row[g] = (const int32_t*)((const char*)T.rows + __umul24((uint32_t)pat[p], (uint32_t)T.stride));
+    cl[g] = 0;
+    if constexpr (PAT) {
+      row[g] = (const int32_t*)((const char*)tab.rows + __umul24((uint32_t)tab.pat[p], (uint32_t)tab.stride));
+      lk[g] = nullptr;
+      lc[g] = nullptr;
+    } else {
+      const int z = Z > 0 ? Z : tab.zmax;
+      row[g] = nullptr;
+      lk[g] = tab.link + (uint32_t)p * (uint32_t)z;
+      lc[g] = tab.lcid ? tab.lcid + (uint32_t)p * (uint32_t)z : nullptr;
+      if (Z == 0 && !tab.one) cl[g] = tab.cls[p] * 8;
+    }
     own[g] = v.at(p);
 #pragma unroll
     for (int k = 0; k < NC; ++k) s[g][k] = v.ld(own[g], k, 0);
   }
   if constexpr (UNI && Z > 0) {
-    // every site's row, then every neighbour, then the sums
+    // every site's links, then every neighbour, then the sums
     int32_t w[G][(Z + 3) / 4 * 4];
     float t[G][Z][NC];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int u = 0; u < Z; u += 4) read_row(row[g] + u, w[g] + u);
+    for (int g = 0; g < G; ++g) link_words<PAT, Z>(tab, row[g], lk[g], 0, Z, w[g]);
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int u = 0; u < Z; ++u)
 #pragma unroll
-        for (int k = 0; k < NC; ++k) t[g][u][k] = v.ld(own[g], k, w[g][u]);
+        for (int k = 0; k < NC; ++k) t[g][u][k] = link_spin<PAT, true>(v, own[g], w[g][u], k);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       float S[3] = {t[g][0][0], NC > 1 ? t[g][0][NC > 1 ? 1 : 0] : 0.0f, NC > 2 ? t[g][0][NC > 2 ? 2 : 0] : 0.0f};
@@ -599,13 +574,13 @@ __device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, in
       for (int u = 1; u < Z; ++u)
 #pragma unroll
         for (int k = 0; k < NC; ++k) S[k] += t[g][u][k];
-      sum_field<NC>(T, S, H[g]);
+      sum_field<NC>(tab, S, H[g]);
     }
   } else {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      cl[g] = Z > 0 || T.one ? 0 : row[g][T.zmax] * 8;
-      row_field<NC, UNI, Z>(v, own[g], row[g], T, H[g]);
+      if (PAT && Z == 0 && !tab.one) cl[g] = row[g][tab.zmax] * 8;
+      site_field<NC, PAT, UNI, Z>(v, own[g], row[g], lk[g], lc[g], tab, H[g]);
     }
   }
   const u32x4 x = philox4x32_10(
@@ -617,17 +592,17 @@ __device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, in
   for (int g = 0; g < G; ++g) {
     float c[5];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) c[k] = T.cls0[k];
-    if (Z == 0 && !T.one)
+    for (int k = 0; k < 5; ++k) c[k] = tab.cls0[k];
+    if (Z == 0 && !tab.one)
 #pragma unroll
-      for (int k = 0; k < 5; ++k) c[k] = T.clsdat[cl[g] + k];
+      for (int k = 0; k < 5; ++k) c[k] = tab.clsdat[cl[g] + k];
     if constexpr (NC == 1) {
       n[g][0] = s[g][0] * c[0];  // the spin sigma*S
       acc[g] = ising_decide(n[g][0], H[g][0], h, ac, w[g], dE[g]) & live[g];
     } else {
       float r[3];
       metro_axis<NC>(NC == 3 ? w[0] : 0u, NC == 3 ? w[1] : w[2 * g], r);
-      acc[g] = metro_decide<NC>(s[g], H[g], r, ac.beta, h, T.aniso, c + 1, NC == 3 ? w[2] : w[2 * g + 1], n[g],
+      acc[g] = metro_decide<NC>(s[g], H[g], r, ac.beta, h, tab.aniso, c + 1, NC == 3 ? w[2] : w[2 * g + 1], n[g],
                                 dE[g]) & live[g];
       is2[g] = c[4];
     }
@@ -650,13 +625,13 @@ __device__ __forceinline__ void metro_rows(const V& v, int b, int cnt, int q, in
 // f(Z) with the link count a compile-time constant for graphs of one site
 // class with a common count: square (4), triangular and cubic (6) lattices,
 // honeycomb with second neighbours (9); f(0) for any other
-template <bool UNI, typename T, typename F>
+template <bool PAT, bool UNI, typename T, typename F>
 __device__ __forceinline__ void with_links(const T& t, F&& f) {
   if (UNI && t.one && t.zmax == 4)
     f(std::integral_constant<int, 4>());
-  else if (t.one && t.zmax == 6)
+  else if ((PAT || UNI) && t.one && t.zmax == 6)
     f(std::integral_constant<int, 6>());
-  else if (!UNI && t.one && t.zmax == 9)
+  else if (PAT && !UNI && t.one && t.zmax == 9)
     f(std::integral_constant<int, 9>());
   else
     f(std::integral_constant<int, 0>());
@@ -1957,13 +1932,9 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
                                               uint32_t key0, uint32_t key1, const PartInfo& pi, float& fE, float* fM,
                                               bool aniso, const PoolInfo<ST>& pl, bool pfresh) {
   constexpr int GD = SitesPerDraw<NC>::G;
-  const int zmax = G.zmax;
   const bool split = pi.np > 1;
-  RowTab<NC, const float*> T;
   beta.beta = in_vgpr(beta.beta);
   h = in_vgpr(h);
-  if constexpr (MODE == 0 || MODE == 3)
-    row_tab<NC, MODE == 3>(T, s_pat, coup, coup + (MODE == 3 ? G.ucid : 0) * COUP_LDS, clsdat, zmax, G.ncls, aniso);
   // A colour's groups are dealt out in rounds of TPR; the last, partial
   // round falls to the first lanes of the deal.  The deal starts at wave r
   // of the group, chosen so that the groups' partial rounds land on
@@ -1975,87 +1946,67 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
     lt = lt - 64 * r;
     if (lt < 0) lt += TPR;
   }
-  for (int c = 0; c < G.ncol; ++c) {
-    const int b = s_colptr[c], cnt = s_colptr[c + 1] - b;
-    const int ngrp = (cnt + GD - 1) / GD;
-    const int q0 = split ? (int)((int64_t)ngrp * pi.part / pi.np) : 0;
-    const int q1 = split ? (int)((int64_t)ngrp * (pi.part + 1) / pi.np) : ngrp;
-    const int nx = split ? pi.hx[2 * c + 1] : 0;
-    const int32_t* xl = split ? pi.halo + pi.hx[2 * c] : nullptr;
-    // A split part's recomputed groups continue the round-robin of its own
-    // groups: a thread whose own loop ends at q (the first q >= q1 of its
-    // deal) takes xl[q - q1], xl[q - q1 + TPR], ...  They fill the part's
-    // last own round: a round of them alone would cost about as much as a
-    // full one (one wave's dependent chain).
-    float xE = 0.0f, xM[3] = {0.0f, 0.0f, 0.0f};
-    if constexpr (MODE == 0 || MODE == 3) {
-      constexpr bool UNI = MODE == 3;
-      const int qm = q1 - pl.rem;  // the pool takes the last rem groups (unsplit replicas only)
-      const LdsView<NC, ST> v{sp.p, sp.n};
-      with_links<UNI>(T, [&](auto zc) {
-        constexpr int Z = decltype(zc)::value;
+  const LdsView<NC, ST> v{sp.p, sp.n};
+  auto colours = [&](auto pc, auto uc, const auto& T) {
+    constexpr bool PAT = decltype(pc)::value, UNI = decltype(uc)::value;
+    with_links<PAT, UNI>(T, [&](auto zc) {
+      constexpr int Z = decltype(zc)::value;
+      for (int c = 0; c < G.ncol; ++c) {
+        const int b = s_colptr[c], cnt = s_colptr[c + 1] - b;
+        const int ngrp = (cnt + GD - 1) / GD;
+        const int q0 = split ? (int)((int64_t)ngrp * pi.part / pi.np) : 0;
+        const int q1 = split ? (int)((int64_t)ngrp * (pi.part + 1) / pi.np) : ngrp;
+        const int qm = q1 - pl.rem;  // the pool takes the last rem groups (unsplit replicas only)
         int q = q0 + lt;
-        for (; q < qm; q += TPR)
-          metro_rows<NC, UNI, Z>(v, b, cnt, q, c, s_pid, T, beta, h, kk, key0, key1, fE, fM);
-        if (pl.pr >= 0) {
-          const float4 pv = pl.par[pl.pr];
-          float pe = 0.0f, pm[3] = {0.0f, 0.0f, 0.0f};
-          const LdsView<NC, ST> pv_s{pl.spin0 + pl.sstride * pl.pr, G.n};
-          metro_rows<NC, UNI, Z>(pv_s, b, cnt, qm + pl.pq, c, s_pid, T, beta.at(pv.x, __float_as_int(pv.w)), pv.y, kk,
-                                 key0, __float_as_uint(pv.z), pe, pm);
-          // the first pool group after a tail stores, later ones add
-          double* pp = pl.pp + threadIdx.x;
-          const bool first = pfresh && c == 0;
-          pp[0] = first ? (double)pe : pp[0] + (double)pe;
+        for (; q < qm; q += TPR) metro_sites<NC, PAT, UNI, Z>(v, b, cnt, q, c, T, beta, h, kk, key0, key1, fE, fM);
+        if constexpr (PAT) {
+          if (pl.pr >= 0) {
+            const float4 pv = pl.par[pl.pr];
+            float pe = 0.0f, pm[3] = {0.0f, 0.0f, 0.0f};
+            const LdsView<NC, ST> pv_s{pl.spin0 + pl.sstride * pl.pr, G.n};
+            metro_sites<NC, PAT, UNI, Z>(pv_s, b, cnt, qm + pl.pq, c, T, beta.at(pv.x, __float_as_int(pv.w)), pv.y, kk,
+                                         key0, __float_as_uint(pv.z), pe, pm);
+            // the first pool group after a tail stores, later ones add
+            double* pp = pl.pp + threadIdx.x;
+            const bool first = pfresh && c == 0;
+            pp[0] = first ? (double)pe : pp[0] + (double)pe;
 #pragma unroll
-          for (int k = 1; k <= NC; ++k) pp[k * pl.nr] = first ? (double)pm[k - 1] : pp[k * pl.nr] + (double)pm[k - 1];
+            for (int k = 1; k <= NC; ++k) pp[k * pl.nr] = first ? (double)pm[k - 1] : pp[k * pl.nr] + (double)pm[k - 1];
+          }
         }
-        for (int j = q - qm; j < nx; j += TPR)
-          metro_rows<NC, UNI, Z>(v, b, cnt, xl[j], c, s_pid, T, beta, h, kk, key0, key1, xE, xM);
-      });
-    } else if constexpr (MODE == 1) {
-      const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
-      if (G.ucid >= 0) {
-        const float* cp = coup + G.ucid * COUP_LDS;
-        int q = q0 + lt;
-        for (; q < q1; q += TPR)
-          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0,
-                                key1, fE, fM);
-        for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, COUP_LDS, gas(G.cls), clsdat, beta, h, kk,
-                                key0, key1, xE, xM);
-      } else {
-        int q = q0 + lt;
-        for (; q < q1; q += TPR)
-          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, coup, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0, key1,
-                          fE, fM);
-        for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, coup, COUP_LDS, gas(G.cls), clsdat, beta, h, kk, key0,
-                          key1, xE, xM);
+        if (split) {
+          // A split part's recomputed groups continue the round-robin of its
+          // own groups: a thread whose own loop ends at q (the first q >= q1
+          // of its deal) takes xl[q - q1], xl[q - q1 + TPR], ...  They fill
+          // the part's last own round: a round of them alone would cost about
+          // as much as a full one (one wave's dependent chain).
+          const int nx = pi.hx[2 * c + 1];
+          const int32_t* xl = pi.halo + pi.hx[2 * c];
+          float xE = 0.0f, xM[3] = {0.0f, 0.0f, 0.0f};
+          for (int j = q - qm; j < nx; j += TPR)
+            metro_sites<NC, PAT, UNI, Z>(v, b, cnt, xl[j], c, T, beta, h, kk, key0, key1, xE, xM);
+        }
+        __syncthreads();
       }
-    } else {
-      const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
-      const bool uni = G.ucid >= 0;
-      const GAS float* cp = gas(coup) + (uni ? G.ucid * 9 : 0);
-      if (uni) {
-        int q = q0 + lt;
-        for (; q < q1; q += TPR)
-          metro_group<NC, true>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk,
-                                key0, key1, fE, fM);
-        for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC, true>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h,
-                                kk, key0, key1, xE, xM);
-      } else {
-        int q = q0 + lt;
-        for (; q < q1; q += TPR)
-          metro_group<NC>(sp, b, cnt, q, c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk, key0,
-                          key1, fE, fM);
-        for (int j = q - q1; j < nx; j += TPR)
-          metro_group<NC>(sp, b, cnt, xl[j], c, gas(G.link), lcid, zmax, cp, 9, gas(G.cls), gas(clsdat), beta, h, kk,
-                          key0, key1, xE, xM);
-      }
-    }
-    __syncthreads();
+    });
+  };
+  typedef std::true_type Y;
+  typedef std::false_type N;
+  if constexpr (MODE == 0 || MODE == 3) {
+    constexpr bool UNI = MODE == 3;
+    colours(Y(), std::integral_constant<bool, UNI>(),
+            sweep_tab<NC, UNI>(G, s_pat, s_pid, coup, COUP_LDS, coup + (UNI ? G.ucid : 0) * COUP_LDS, clsdat, aniso));
+  } else if constexpr (MODE == 1) {
+    if (G.ucid >= 0)
+      colours(N(), Y(), sweep_tab<NC, true>(G, s_pat, s_pid, coup, COUP_LDS, coup + G.ucid * COUP_LDS, clsdat, aniso));
+    else
+      colours(N(), N(), sweep_tab<NC, false>(G, s_pat, s_pid, coup, COUP_LDS, coup, clsdat, aniso));
+  } else {
+    const GAS float* gc = gas(coup);
+    if (G.ucid >= 0)
+      colours(N(), Y(), sweep_tab<NC, true>(G, s_pat, s_pid, gc, 9, gc + G.ucid * 9, gas(clsdat), aniso));
+    else
+      colours(N(), N(), sweep_tab<NC, false>(G, s_pat, s_pid, gc, 9, gc, gas(clsdat), aniso));
   }
 }
 
@@ -2153,7 +2104,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
 
   for (int t = threadIdx.x; t < ncl * 9; t += blockDim.x) s_coup[t / 9 * COUP_LDS + t % 9] = G.coup[t];
   for (int t = threadIdx.x; t < ncs * 8; t += blockDim.x) s_clsl[t] = G.clsdat[t];
-  // does any site class carry an on-site term? (metro_core skips them if not)
+  // does any site class carry an on-site term? (the D terms are skipped if not)
   int anz = 0;
   for (int t = threadIdx.x; t < G.ncls; t += blockDim.x)
     anz |= (G.clsdat[t * 8 + 1] != 0.0f) | (G.clsdat[t * 8 + 2] != 0.0f) | (G.clsdat[t * 8 + 3] != 0.0f);
@@ -2632,8 +2583,11 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
 // groups (x * PASS_GPT + u) * 256 + t of the colour, u < PASS_GPT, so that
 // a wave touches consecutive positions and each thread's reduction is shared
 // by PASS_GPT groups.  Graphs with link patterns read their neighbours as
-// position deltas from pattern rows staged in LDS (no link-table traffic and
-// no load that waits on another); the others read the global link table.
+// position deltas from pattern rows staged in LDS (no link-table traffic); the
+// others read the global link table.  Bound: HBM traffic and the round trips
+// of one update (pattern, spins, store).  Measured on cubic 64^3 x 128 T
+// (16.8M updates, 615 MB a pass): 241 -> 160 us when the links came to be read
+// together through 32-bit offsets (2.6 -> 3.8 TB/s; a copy reaches 5.3).
 // Changes of E and M: FP32 per thread, FP64 DPP wave sums, one device
 // atomic per value per block.
 // ---------------------------------------------------------------------------
@@ -2653,6 +2607,11 @@ static constexpr int PASS_PAT_INTS = 4096;  // most LDS for pattern rows (16 KB)
 __host__ __device__ inline bool pass_patterns(const mcg_graph& G) {
   return G.npat > 0 && G.lcid == nullptr && G.npat * pat_stride(G.zmax) <= PASS_PAT_INTS;
 }
+// the pass's link mode of a graph (a compile-time argument of k_pass, so that
+// each instantiation has only its own loads in registers: together they
+// exceed the 64 that 8 waves per SIMD leave)
+enum { PASS_LINKS = 0, PASS_LINKS_UNI = 1, PASS_PAT = 2, PASS_PAT_UNI = 3, PASS_MODES = 4 };
+__host__ __device__ inline int pass_mode(const mcg_graph& G) { return (pass_patterns(G) ? 2 : 0) + (G.ucid >= 0 ? 1 : 0); }
 __host__ __device__ inline size_t pass_lds_bytes(const mcg_graph& G) {
   return pass_patterns(G) ? (size_t)G.npat * pat_stride(G.zmax) * 4 + (G.ucid >= 0 ? 0 : (size_t)G.ncoup * COUP_LDS * 4)
                           : 0;
@@ -2671,13 +2630,14 @@ __device__ __forceinline__ int xcd_item(int b, int total) {
 }
 __host__ __device__ inline int xcd_grid(int total) { return (total + NXCD - 1) / NXCD * NXCD; }
 
-// at least 8 waves per SIMD: the pass is latency-bound, and a 64-VGPR cap
-// hides more of it (measured per sweep: cubic 64^3 0.702 -> 0.648 ms,
-// triangular 128^2 0.470 -> 0.436 ms; 6 waves: 0.628 and 0.497 ms)
+// 6 waves per SIMD (80 VGPRs): with a site's links all in flight at once, more
+// waves gain nothing and 64 VGPRs spill the tensors of graphs with several
+// couplings.  Passes with 8, 6 and 5 waves: triangular 128^2 x 1024 (with its
+// frames) 1.85, 1.68, 1.68 ms; cubic 64^3 x 128 2.59, 2.55, 2.59 ms.
 #ifndef MCG_PASS_MIN_WAVES
-#define MCG_PASS_MIN_WAVES 8
+#define MCG_PASS_MIN_WAVES 6
 #endif
-template <int NC, typename ST>
+template <int NC, typename ST, int MODE>
 __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, const int32_t* __restrict__ rep_list, int colour,
                                               int64_t sweep, int nchunk, int nitems) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -2689,7 +2649,7 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
   const mcg_replica rp = B.reps[rep];
   const mcg_graph G = B.graphs[rp.graph];
   const int zmax = G.zmax;
-  const bool pats = pass_patterns(G), uni = G.ucid >= 0;
+  constexpr bool pats = MODE >= PASS_PAT, uni = (MODE & 1) != 0;
   int32_t* s_pat = (int32_t*)smem;
   float* s_coup = (float*)(s_pat + G.npat * pat_stride(zmax));
   int anz = 0;
@@ -2697,16 +2657,15 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
     for (int t = threadIdx.x; t < G.npat * (zmax + 1); t += blockDim.x) {
       const int l = t % (zmax + 1);
       const int32_t w = G.pattab[t];
-      s_pat[t / (zmax + 1) * pat_stride(zmax) + l] =
-          l == zmax ? w : uni ? row_word<true>(w, sizeof(ST)) : row_word<false>(w, sizeof(ST));
+      s_pat[t / (zmax + 1) * pat_stride(zmax) + l] = l == zmax ? w : row_word<uni>(w, sizeof(ST));
     }
     if (!uni)
       for (int t = threadIdx.x; t < G.ncoup * 9; t += blockDim.x) s_coup[t / 9 * COUP_LDS + t % 9] = G.coup[t];
-    // does any site class carry an on-site term? (the D terms are skipped if not)
-    for (int t = threadIdx.x; t < G.ncls; t += blockDim.x)
-      anz |= (G.clsdat[t * 8 + 1] != 0.0f) | (G.clsdat[t * 8 + 2] != 0.0f) | (G.clsdat[t * 8 + 3] != 0.0f);
   }
-  const bool aniso = __syncthreads_or(anz) != 0 || !pats;
+  // does any site class carry an on-site term? (the D terms are skipped if not)
+  for (int t = threadIdx.x; t < G.ncls; t += blockDim.x)
+    anz |= (G.clsdat[t * 8 + 1] != 0.0f) | (G.clsdat[t * 8 + 2] != 0.0f) | (G.clsdat[t * 8 + 3] != 0.0f);
+  const bool aniso = __syncthreads_or(anz) != 0;
   float dE = 0.0f, dM[3] = {0.0f, 0.0f, 0.0f};
   if (colour < G.ncol) {
     const int b = G.col_ptr[colour], cnt = G.col_ptr[colour + 1] - b;
@@ -2716,47 +2675,23 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
     const Acc beta = acc_of(B, in_vgpr(B.row_beta[row]), row);
     const uint32_t key1 = B.seed_hi ^ rp.serial;
     GAS ST* spins = gas((ST*)B.spins + rp.spin_off);
-    const int q0 = chunk * PASS_GPT * (int)blockDim.x + (int)threadIdx.x;
-    auto groups = [&](auto&& update) {
+    const HbmView<NC, ST> v(spins, G.n);
+    auto pass = [&](const auto& T) {
+      with_links<pats, uni>(T, [&](auto zc) {
 #pragma unroll MCG_PASS_UNROLL
-      for (int u = 0; u < PASS_GPT; ++u) {
-        const int q = q0 + u * (int)blockDim.x;
-        if (q >= ngrp) break;
-        update(q);
-      }
+        for (int u = 0; u < PASS_GPT; ++u) {
+          const int q = (chunk * PASS_GPT + u) * (int)blockDim.x + (int)threadIdx.x;
+          if (q >= ngrp) break;
+          metro_sites<NC, pats, uni, decltype(zc)::value>(v, b, cnt, q, colour, T, beta, h, (uint64_t)sweep, B.seed_lo,
+                                                          key1, dE, dM);
+        }
+      });
     };
-    if (pats) {
-      const HbmView<NC, ST> v(spins, G.n);
-      const GAS uint8_t* pat = gas(G.pat);
-      auto rows = [&](auto uc) {
-        constexpr bool UNI = decltype(uc)::value;
-        RowTab<NC, const GAS float*> T;
-        row_tab<NC, UNI>(T, s_pat, s_coup, gas(G.coup) + (UNI ? G.ucid * 9 : 0), gas(G.clsdat), zmax, G.ncls, aniso);
-        with_links<UNI>(T, [&](auto zc) {
-          groups([&](int q) {
-            metro_rows<NC, UNI, decltype(zc)::value>(v, b, cnt, q, colour, pat, T, beta, h, (uint64_t)sweep, B.seed_lo,
-                                                     key1, dE, dM);
-          });
-        });
-      };
-      if (uni)
-        rows(std::true_type());
-      else
-        rows(std::false_type());
-    } else {
-      const GSpins<ST> sp{spins, G.n};
-      const GAS int32_t* lcid = G.lcid ? gas(G.lcid) : nullptr;
-      if (uni)
-        groups([&](int q) {
-          metro_group<NC, true>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup) + G.ucid * 9, 9, gas(G.cls),
-                                gas(G.clsdat), beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
-        });
-      else
-        groups([&](int q) {
-          metro_group<NC>(sp, b, cnt, q, colour, gas(G.link), lcid, zmax, gas(G.coup), 9, gas(G.cls), gas(G.clsdat),
-                          beta, h, (uint64_t)sweep, B.seed_lo, key1, dE, dM);
-        });
-    }
+    const GAS float *gc = gas(G.coup), *uc = gc + (uni ? G.ucid * 9 : 0);
+    if constexpr (pats)
+      pass(sweep_tab<NC, uni>(G, s_pat, gas(G.pat), s_coup, COUP_LDS, uc, gas(G.clsdat), aniso));
+    else
+      pass(sweep_tab<NC, uni>(G, s_pat, gas(G.pat), gc, 9, uc, gas(G.clsdat), aniso));
   }
   // every lane reaches here: DPP sums per wave, the waves' totals through LDS
   double v[4] = {(double)dE, (double)dM[0], (double)dM[1], (double)dM[2]};
@@ -3755,16 +3690,27 @@ int check_persist(const mcg_batch* B, const mcg_plan* P, RunCtx& X, bool* ok) {
 }
 
 
+// one colour of nreps replicas (all of link mode `mode`)
 template <int NC, typename ST>
-int launch_pass(const mcg_batch* B, const int32_t* dreps, int nreps, int maxcnt, uint32_t lds, int colour, int64_t sweep,
-                hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
+int launch_pass(const mcg_batch* B, const int32_t* dreps, int nreps, int mode, int maxcnt, uint32_t lds, int colour,
+                int64_t sweep, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
   if (nreps == 0) return 0;
   const int ngrp = (maxcnt + SitesPerDraw<NC>::G - 1) / SitesPerDraw<NC>::G;
   const int chunks = std::max(1, (ngrp + 256 * PASS_GPT - 1) / (256 * PASS_GPT));
   const int64_t items = (int64_t)chunks * nreps;
   if (items > (1 << 30)) return fail("streaming pass: %lld work items", (long long)items);
-  hipExtLaunchKernelGGL((k_pass<NC, ST>), dim3((unsigned)xcd_grid((int)items)), dim3(256), lds, s, e0, e1, 0, *B, dreps,
-                        colour, sweep, chunks, (int)items);
+  auto launch = [&](auto kernel) {
+    hipExtLaunchKernelGGL(kernel, dim3((unsigned)xcd_grid((int)items)), dim3(256), lds, s, e0, e1, 0, *B, dreps, colour,
+                          sweep, chunks, (int)items);
+  };
+  if (mode == PASS_PAT_UNI)
+    launch(k_pass<NC, ST, PASS_PAT_UNI>);
+  else if (mode == PASS_PAT)
+    launch(k_pass<NC, ST, PASS_PAT>);
+  else if (mode == PASS_LINKS_UNI)
+    launch(k_pass<NC, ST, PASS_LINKS_UNI>);
+  else
+    launch(k_pass<NC, ST, PASS_LINKS>);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -3830,19 +3776,20 @@ int stream_sweeps(const mcg_batch* B, const mcg_plan* P, RunCtx& X, int64_t k0, 
   const int maxn = X.stream_maxcnt;  // largest colour class of the streamed graphs
   const int32_t* dreps = X.stream_reps;
   const int nrs = (int)X.hstream.size();
+  auto mode_of = [&](int i) { return pass_mode(B->graphs_host[B->reps_host[X.hstream[i]].graph]); };
   for (int64_t q = 0; q < nsw; ++q) {
     const int64_t k = k0 + q;
     const int64_t kk = P->sweep0 + k;
     for (int c = 0; c < ncolmax; ++c) {
-      if (plain) {
-        for (int i = 0; i < nrs; ++i) {
-          hipEvent_t e0, e1;
-          if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps + i, 1, maxn, X.stream_lds, c, kk, s, e0, e1)) return -1;
-          T.launches += 1;
-        }
-      } else {
+      // one launch per run of replicas of one link mode (hstream is sorted by
+      // it), or, plain, per replica
+      for (int i = 0, e; i < nrs; i = e) {
+        const int mode = mode_of(i);
+        for (e = i + 1; !plain && e < nrs && mode_of(e) == mode;) ++e;
         hipEvent_t e0, e1;
-        if (T.pair(&e0, &e1) || launch_pass<NC, ST>(B, dreps, nrs, maxn, X.stream_lds, c, kk, s, e0, e1)) return -1;
+        if (T.pair(&e0, &e1) ||
+            launch_pass<NC, ST>(B, dreps + i, e - i, mode, maxn, X.stream_lds, c, kk, s, e0, e1))
+          return -1;
         T.launches += 1;
       }
     }
@@ -3884,6 +3831,9 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   HIPCHK(hipDeviceGetAttribute(&X.ncu, hipDeviceAttributeMultiprocessorCount, X.device));
   const bool force_stream = P->kernel == 2 || P->kernel == 3;
   if (plan_lds(B, P, X, force_stream)) return -1;
+  std::stable_sort(X.hstream.begin(), X.hstream.end(), [&](int a, int b) {
+    return pass_mode(B->graphs_host[B->reps_host[a].graph]) < pass_mode(B->graphs_host[B->reps_host[b].graph]);
+  });
   if (P->kernel == 1 && !X.hstream.empty())
     return fail("LDS-resident kernel requested but %zu replica(s) do not fit in LDS", X.hstream.size());
   // tempering ladders (row0, rungs), each of one lattice
