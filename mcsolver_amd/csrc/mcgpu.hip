@@ -642,7 +642,7 @@ template <int NC, typename SV>
 __device__ __forceinline__ void spin_vec(const SV& sp, int i, const int32_t* __restrict__ cls, const float* clsdat,
                                          float* v) {
   if constexpr (NC == 1) {
-    v[0] = sp.get(i, 0) * clsdat[cls[i] * 8];
+    v[0] = sp.get(i, 0) * clsdat[cls ? cls[i] * 8 : 0];  // no cls: one class
     v[1] = v[2] = 0.0f;
   } else {
     v[0] = sp.get(i, 0);
@@ -701,8 +701,9 @@ __device__ __forceinline__ T dev_load(const T* p) {
 }
 __device__ __forceinline__ void dev_add(double* p, double v) { unsafeAtomicAdd(p, v); }
 
-static constexpr int RK = 8;  // values per reduction call
-static constexpr int FRM_ACC = 96;  // frame scratch: accumulator staging starts here
+static constexpr int RK = 12;  // most values per reduction call
+static constexpr int FRM_ACC = 96;       // frame scratch: accumulator staging starts here
+static constexpr int FRM = FRM_ACC + 48;  // frame scratch doubles per group: scalars, then accumulator staging
 
 // FP64 value moved across lanes by DPP (two 32-bit halves); lanes of rows
 // outside ROWMASK get 0.  With every row enabled (the quad permutes and row
@@ -738,6 +739,38 @@ __device__ __forceinline__ double wave_sum_f64(double x) {
   return x;
 }
 
+// x summed over lanes l and l ^ 16, or l and l ^ 32
+__device__ __forceinline__ double add_lane16(double x) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(x), (uint32_t)__double2loint(x), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(x), (uint32_t)__double2hiint(x), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double add_lane32(double x) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(x), (uint32_t)__double2loint(x), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(x), (uint32_t)__double2hiint(x), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// Totals of N values over the 64 lanes (every lane active): lane l gets in
+// r[j] the total of value 4 j + (l & 3).  The first two steps halve the
+// number of values with the number of lanes each still has to cover (a lane
+// keeps one of two values and sends the other), so that four values take 7
+// FP64 additions a lane instead of 24.
+template <int N>
+__device__ __forceinline__ void wave_totals(const double* v, double* r) {
+  const bool b0 = (threadIdx.x & 1) != 0, b1 = (threadIdx.x & 2) != 0;
+#pragma unroll
+  for (int j = 0; 4 * j < N; ++j) {
+    const double a = v[4 * j], b = 4 * j + 1 < N ? v[4 * j + 1] : 0.0;
+    const double c = 4 * j + 2 < N ? v[4 * j + 2] : 0.0, d = 4 * j + 3 < N ? v[4 * j + 3] : 0.0;
+    const double x = (b0 ? b : a) + dpp_f64<0xB1, 0xF>(b0 ? a : b);  // quad_perm [1,0,3,2]
+    const double y = (b0 ? d : c) + dpp_f64<0xB1, 0xF>(b0 ? c : d);
+    double t = (b1 ? y : x) + dpp_f64<0x4E, 0xF>(b1 ? x : y);  // quad_perm [2,3,0,1]
+    t += dpp_f64<0x124, 0xF>(t);                               // row_ror:4
+    t += dpp_f64<0x128, 0xF>(t);                               // row_ror:8
+    r[j] = add_lane32(add_lane16(t));
+  }
+}
+
 // lane src's value (src the same in every lane), in every lane of the wave
 __device__ __forceinline__ double lane_f64(double x, int src) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(x), src);
@@ -746,38 +779,54 @@ __device__ __forceinline__ double lane_f64(double x, int src) {
 }
 __device__ __forceinline__ double lane63(double x) { return lane_f64(x, 63); }
 
-// sum of N (<= RK) values over the TPR threads of group g (TPR a multiple of
-// 64); the result is valid in every lane of the group's first wave, so in
-// the group's first thread.  All threads call it; it ends with a workgroup
-// barrier.  Two levels of DPP wave sums: the waves' totals go through LDS
-// and the group's first wave adds them up (at most 16 waves).
-template <int N>
-__device__ __forceinline__ void group_sum(double* v, double* s_red, int g, int TPR) {
-#pragma unroll
-  for (int k = 0; k < N; ++k) v[k] = wave_sum_f64(v[k]);
+// LDS written by a wave's lanes is read by other lanes of it after this
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Totals of N (<= RK) values over the TPR threads of group g (TPR a multiple
+// of 64): sink(k, total of v[k]) is called once per value, by lane k of the
+// group's first wave, then post() by that whole wave.  All threads call it;
+// it ends with a workgroup barrier.  Each wave's totals go through LDS (lanes
+// 16 p + k of the first wave add value k of waves p, p + 4, ...).
+template <int N, typename F, typename P>
+__device__ __forceinline__ void group_add(const double* v, double* s_red, int g, int TPR, F&& sink, P&& post) {
+  constexpr int M = (N + 3) / 4;
+  double r[M];
+  wave_totals<N>(v, r);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nw = TPR >> 6;
   if (nw == 1) {  // the same for every group of the workgroup
 #pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = lane63(v[k]);
+    for (int j = 0; j < M; ++j)
+      if (lane < 4 && 4 * j + lane < N) sink(4 * j + lane, r[j]);
+    wave_lds_fence();
+    post();
     __syncthreads();
     return;
   }
-  if (lane == 63)
+  if (lane < 4)
 #pragma unroll
-    for (int k = 0; k < N; ++k) s_red[wave * RK + k] = v[k];
+    for (int j = 0; j < M; ++j) s_red[wave * RK + 4 * j + lane] = r[j];
   __syncthreads();
   const int w0 = g * nw;
-  if (wave == w0) {  // the whole wave, so that the DPP sums see every lane
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      const double x = lane < nw ? s_red[(w0 + lane) * RK + k] : 0.0;
-      v[k] = lane63(wave_sum_f64(x));
-    }
+  if (wave == w0) {
+    const int k = lane & 15;
+    double x = 0.0;
+    if (k < N)
+      for (int w = lane >> 4; w < nw; w += 4) x += s_red[(w0 + w) * RK + k];
+    x = add_lane32(add_lane16(x));
+    if (lane < N) sink(lane, x);
+    wave_lds_fence();
+    post();
   }
   __syncthreads();
 }
-__device__ __forceinline__ void group_sum8(double* v, double* s_red, int g, int TPR) { group_sum<RK>(v, s_red, g, TPR); }
+template <int N, typename F>
+__device__ __forceinline__ void group_add(const double* v, double* s_red, int g, int TPR, F&& sink) {
+  group_add<N>(v, s_red, g, TPR, sink, [] {});
+}
 
 // ---------------------------------------------------------------------------
 // measurement of one frame (all flagged observables) for one replica
@@ -790,7 +839,24 @@ struct FrameCtx {
   double* s_red;   // reduction scratch (nwaves*RK)
   double* s_frm;   // per-group frame values (>= 64 doubles per group)
   int g, lt, TPR;
+  double inv_n, inv_nlat, inv_nf;  // 1 / sites, 1 / correlation pairs (or sites), 1 / planned frames
+  int last;                        // position of the last site
+  float* blk;                      // the group's block spins (LDS, nr x NC), or nullptr
 };
+template <int NC>
+__device__ __forceinline__ void frame_consts(FrameCtx& C, const mcg_graph& G, const mcg_batch& B) {
+  C.inv_n = 1.0 / (double)G.n;
+  C.inv_nlat = 1.0 / (double)(G.nlat > 0 ? G.nlat : G.n);
+  C.inv_nf = 1.0 / (double)(B.nframes > 0 ? B.nframes : 1);
+  C.last = G.pos[G.n - 1];
+  C.blk = nullptr;
+}
+// a frame's spin-derived sums need no pass over the spins: nothing but self
+// pairs, whose sums follow from the tracked state
+__device__ __forceinline__ bool frame_light(const mcg_graph& G, int flags) {
+  return !(flags & (MCG_MEAS_Q | MCG_MEAS_RNORM | MCG_MEAS_GROUPS)) &&
+         (!(flags & MCG_MEAS_PAIRS) || G.nlat <= 0 || G.self_pairs);
+}
 
 // Frames and recomputes sit inside the sweep loop.  Left to itself the
 // compiler keeps everything they read (some 60 words of the graph, an address
@@ -810,20 +876,27 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
-// majority spin of block-spin site (heisenbergLib.c:255-267, isingLib.c:133-150)
+// majority spin of block-spin site `site`, whose cluster is row ri of rclu
+// (heisenbergLib.c:255-267, isingLib.c:133-150); cls: nullptr with one class
 template <int NC, typename SV>
-__device__ __forceinline__ void majority(const SV& sp, const mcg_graph& G, const float* clsdat, int site,
-                                         uint64_t frame, uint32_t key0, uint32_t key1, float* v) {
-  const int ri = G.rrank[site];
+__device__ __forceinline__ void majority(const SV& sp, const mcg_graph& G, const int32_t* cls, const float* clsdat,
+                                         int ri, int site, uint64_t frame, uint32_t key0, uint32_t key1, float* v) {
   float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-  for (int k = 0; k < G.nclu; ++k) {
-    float t[3];
-    spin_vec<NC>(sp, G.rclu[ri * G.nclu + k], G.cls, clsdat, t);
-    a0 += t[0];
-    a1 += t[1];
-    a2 += t[2];
+  for (int k0 = 0; k0 < G.nclu; k0 += 4) {
+    // four cluster sites at a time, all read before they are added
+    float t[4][3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      spin_vec<NC>(sp, G.rclu[ri * G.nclu + (k0 + u < G.nclu ? k0 + u : G.nclu - 1)], cls, clsdat, t[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (k0 + u >= G.nclu) break;
+      a0 += t[u][0];
+      a1 += t[u][1];
+      a2 += t[u][2];
+    }
   }
-  const float S = clsdat[G.cls[site] * 8];
+  const float S = clsdat[cls ? cls[site] * 8 : 0];
   if constexpr (NC == 1) {
     float sg;
     if (a0 > 0.0f)
@@ -848,6 +921,13 @@ __device__ __forceinline__ void majority(const SV& sp, const mcg_graph& G, const
     v[1] = a1 * S;
     v[2] = a2 * S;
   }
+}
+// the block spin of index ri computed earlier in this frame
+template <int NC>
+__device__ __forceinline__ void block_spin(const float* blk, int ri, float* v) {
+  v[0] = blk[ri * NC];
+  v[1] = NC > 1 ? blk[ri * NC + (NC > 1 ? 1 : 0)] : 0.0f;
+  v[2] = NC > 2 ? blk[ri * NC + (NC > 2 ? 2 : 0)] : 0.0f;
 }
 
 // solid angle of a spin triangle, heisenbergLib.c:114-127 (atan, +-pi branch)
@@ -895,7 +975,9 @@ __device__ __forceinline__ void flush_frame(const FrameCtx& C, const mcg_batch& 
   const int ngq = frame_groups<NC>(G, flags);
   double* A = B.acc + (size_t)row * MCG_NACC;
   const int nge = ngq > 0 ? (ngq + 1) * (ngq + 1) : 0;
-  for (int q = lt; q < MCG_NACC + MCG_NBINQ + nge; q += TPR) {
+  // from the group's last thread down: a wave's later loads wait for its
+  // atomics, and the last wave has the least of a sweep's work
+  for (int q = TPR - 1 - lt; q < MCG_NACC + MCG_NBINQ + nge; q += TPR) {
     if (q < MCG_NACC) {
       if (q != MCG_A_MPREV && Cn[q] != 0.0) dev_add(A + q, Cn[q]);  // adding 0 changes nothing
     } else if (q < MCG_NACC + MCG_NBINQ) {
@@ -914,8 +996,7 @@ __device__ __forceinline__ void flush_frame(const FrameCtx& C, const mcg_batch& 
   }
 }
 
-// the previous frame's M of a row (for <M M'>), read ahead of the frame by
-// the thread that applies it
+// the previous frame's M of a row (for <M M'>)
 __device__ __forceinline__ double frame_mprev(const mcg_batch& B, int row) {
   return dev_load(B.acc + (size_t)row * MCG_NACC + MCG_A_MPREV);
 }
@@ -925,19 +1006,23 @@ __device__ __forceinline__ double frame_mprev(const mcg_batch& B, int row) {
 // Cn for flush_frame: [0, NACC) accumulators ([MM] holds M itself until the
 // frame's M' product replaces it), [NACC, +NBINQ) the bin terms, then the bin
 // index.  st: the replica's state; F: the frame's spin-derived values.  One
-// thread per replica; every term is written (zeros included).
+// thread per replica; Cn is zero before (zero_terms).
+static constexpr int NTERMS = MCG_NACC + MCG_NBINQ + 1;
+__device__ __forceinline__ void zero_terms(double* s_frm, int R) {  // by one wave, for R groups
+  const int lane = threadIdx.x & 63;
+  for (int r = 0; r < R; ++r)
+    if (lane < NTERMS) s_frm[r * FRM + FRM_ACC + lane] = 0.0;
+  wave_lds_fence();
+}
 template <int NC>
-__device__ __forceinline__ void frame_terms(const mcg_graph& G, const mcg_batch& B, const double* st, double* F,
-                                            int flags, int64_t frame, double* Cn) {
+__device__ __forceinline__ void frame_terms(const FrameCtx& C, const mcg_graph& G, const mcg_batch& B, const double* st,
+                                            double* F, int flags, int64_t frame, double* Cn) {
   const int ngq = frame_groups<NC>(G, flags);
-  for (int q = 0; q < MCG_NACC + MCG_NBINQ + 1; ++q) Cn[q] = 0.0;
-  const double n = G.n;
-  const double nLat = G.nlat > 0 ? G.nlat : G.n;
-  const double inv_nLat = 1.0 / nLat;
+  const double inv_nLat = C.inv_nlat;
   const bool pairs = (flags & MCG_MEAS_PAIRS) && G.nlat > 0;
   double E = st[MCG_S_E];
   if (flags & MCG_ISING_RELE) E -= st[MCG_S_EREF];
-  const double e = E * (1.0 / n);
+  const double e = E * C.inv_n;
   const double M0 = st[MCG_S_M], M1 = st[MCG_S_M + 1], M2 = st[MCG_S_M + 2];
   if (pairs && G.self_pairs) {
     // pairs (i, i) over every site: sum s_i is the tracked magnetisation,
@@ -1012,7 +1097,7 @@ __device__ __forceinline__ void frame_terms(const mcg_graph& G, const mcg_batch&
   // quotient corrected to the exact integer floor
   const int64_t nf = B.nframes > 0 ? B.nframes : 1;
   const int64_t num = frame * (int64_t)B.nbins;
-  int64_t bin = (int64_t)floor((double)num * (1.0 / (double)nf));  // corrected to the exact floor below
+  int64_t bin = (int64_t)floor((double)num * C.inv_nf);  // corrected to the exact floor below
   if (bin * nf > num) --bin;
   if ((bin + 1) * nf <= num) ++bin;
   if (bin >= B.nbins) bin = B.nbins - 1;
@@ -1061,8 +1146,9 @@ __device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, cons
                            uint32_t key1, float h, int part, int np, const PartFrame* own = nullptr) {
   const mcg_graph G = fresh(C.G);
   const int lt = opaque(C.lt), TPR = C.TPR;
-  double* F = C.s_frm;  // leader-only use
+  double* F = C.s_frm;
   double v[RK];
+  const int32_t* cls = G.ncls == 1 ? nullptr : G.cls;
   const int flags = FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS);
   int lo, hi;
   // --- correlation pairs: S_i, S_j, sum s_i.s_j, last-site spin
@@ -1074,22 +1160,24 @@ __device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, cons
     for (int q = lo + lt; q < hi; q += TPR) {
       const int p = own ? own->pairs[q] : q;
       float a[3], b[3];
-      spin_vec<NC>(sp, G.pairs[2 * p], G.cls, C.clsdat, a);
-      spin_vec<NC>(sp, G.pairs[2 * p + 1], G.cls, C.clsdat, b);
+      spin_vec<NC>(sp, G.pairs[2 * p], cls, C.clsdat, a);
+      spin_vec<NC>(sp, G.pairs[2 * p + 1], cls, C.clsdat, b);
       v[0] += a[0]; v[1] += a[1]; v[2] += a[2];
       v[3] += b[0]; v[4] += b[1]; v[5] += b[2];
       v[6] += (double)(a[0] * b[0] + a[1] * b[1] + a[2] * b[2]);
     }
     if (lt == 0 && (own ? own->last : part == 0)) {
       float t[3];
-      spin_vec<NC>(sp, G.pos[G.n - 1], G.cls, C.clsdat, t);
+      spin_vec<NC>(sp, C.last, cls, C.clsdat, t);
       v[7] = t[0];
     }
     // self pairs: every other lane holds zeros, so the group reduction (a
     // microsecond of FP64 DPP steps and barriers per frame) is not needed
-    if (!G.self_pairs) group_sum8(v, C.s_red, C.g, TPR);
-    if (lt == 0)
+    if (!G.self_pairs) {
+      group_add<8>(v, C.s_red, C.g, TPR, [&](int k, double x) { F[k] = x; });
+    } else if (lt == 0) {
       for (int k = 0; k < 8; ++k) F[k] = v[k];
+    }
   }
   // --- topological charge
   if ((flags & MCG_MEAS_Q) && NC == 3 && G.ncirc > 0) {
@@ -1104,87 +1192,111 @@ __device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, cons
       const int p = own ? own->circs[q] : q;
       const int ia = G.circ[3 * p], ib = G.circ[3 * p + 1], ic = G.circ[3 * p + 2];
       float a[3], b[3], c[3];
-      spin_vec<NC>(sp, ia, G.cls, C.clsdat, a);
-      spin_vec<NC>(sp, ib, G.cls, C.clsdat, b);
-      spin_vec<NC>(sp, ic, G.cls, C.clsdat, c);
+      spin_vec<NC>(sp, ia, cls, C.clsdat, a);
+      spin_vec<NC>(sp, ib, cls, C.clsdat, b);
+      spin_vec<NC>(sp, ic, cls, C.clsdat, c);
       if (one_len)
         v[0] += (double)signed_area(a, b, c, il, il, il);
       else
         v[0] += (double)signed_area(a, b, c, inv_len(C.clsdat, G.cls, ia), inv_len(C.clsdat, G.cls, ib),
                                     inv_len(C.clsdat, G.cls, ic));
     }
-    group_sum<1>(v, C.s_red, C.g, TPR);
-    if (lt == 0) F[8] = v[0];
+    group_add<1>(v, C.s_red, C.g, TPR, [&](int, double x) { F[8] = x; });
   }
   // --- block-spin observables
   if ((flags & MCG_MEAS_RNORM) && G.nr > 0 && !own) {
     for (int k = 0; k < RK; ++k) v[k] = 0.0;
-    double w[RK];
-    for (int k = 0; k < RK; ++k) w[k] = 0.0;
+    // Every block spin is used by its own pairs and links and by its
+    // neighbours' links.  Where LDS has room each is computed once, here, and
+    // looked up below; otherwise at every use (each use waits for its rank,
+    // its cluster's sites and their spins one after another).
+    const float* blk = C.blk;
+    if (blk) {
+      for (int ri = lt; ri < G.nr; ri += TPR) {
+        float m[3];
+        majority<NC>(sp, G, cls, C.clsdat, ri, G.rorb[ri], frame, key0, key1, m);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) C.blk[ri * NC + k] = m[k];
+      }
+      __syncthreads();
+    }
+    auto block = [&](int ri, int site, float* m) {
+      if (blk)
+        block_spin<NC>(blk, ri, m);
+      else
+        majority<NC>(sp, G, cls, C.clsdat, ri, site, frame, key0, key1, m);
+    };
     slice(G.nlat, part, np, lo, hi);
     for (int p = lo + lt; p < hi; p += TPR) {
       const int ia = G.pairs[2 * p], ib = G.pairs[2 * p + 1];
-      const bool ca = G.rrank[ia] >= 0, cb = G.rrank[ib] >= 0;
+      const int ra = G.rrank[ia], rb = G.rrank[ib];
+      const bool ca = ra >= 0, cb = rb >= 0;
       float ma[3] = {0, 0, 0}, mb[3] = {0, 0, 0};
       if (ca) {
-        majority<NC>(sp, G, C.clsdat, ia, frame, key0, key1, ma);
+        block(ra, ia, ma);
         v[0] += ma[0]; v[1] += ma[1]; v[2] += ma[2];
-        w[0] += 1.0;
+        v[7] += 1.0;
       }
       if (cb) {
-        majority<NC>(sp, G, C.clsdat, ib, frame, key0, key1, mb);
+        block(rb, ib, mb);
         v[3] += mb[0]; v[4] += mb[1]; v[5] += mb[2];
-        w[1] += 1.0;
+        v[8] += 1.0;
       }
       if (ca && cb) {
         v[6] += (double)(ma[0] * mb[0] + ma[1] * mb[1] + ma[2] * mb[2]);
-        w[2] += 1.0;
+        v[9] += 1.0;
       }
     }
     slice(G.nr, part, np, lo, hi);
     for (int ri = lo + lt; ri < hi; ri += TPR) {
       const int j = G.rorb[ri];
       float m[3];
-      majority<NC>(sp, G, C.clsdat, j, frame, key0, key1, m);
+      block(G.rrank[j], j, m);
       float cc = 0.0f;
-      for (int l = 0; l < G.zmax; ++l) {
-        const uint32_t wd = G.rlink[(size_t)ri * G.zmax + l];
-        const int t = (int)(wd & 0xFFFFFFu);
-        // wide graphs: the block-spin link takes the coupling of the site's
-        // link l; a set high byte marks an absent link
-        if (G.lcid && (wd >> 24)) continue;
-        const float* J = C.coup + (G.lcid ? G.lcid[(size_t)j * G.zmax + l] : (int)(wd >> 24)) * C.cst;
-        float mt[3];
-        majority<NC>(sp, G, C.clsdat, t, frame, key0, key1, mt);
-        if constexpr (NC == 1) {
-          cc += J[1] * m[0] * mt[0];
-        } else {
-          float H0 = J[0] * mt[0] + J[1] * mt[1] + J[2] * mt[2];
-          float H1 = J[3] * mt[0] + J[4] * mt[1] + J[5] * mt[2];
-          float H2 = J[6] * mt[0] + J[7] * mt[1] + J[8] * mt[2];
-          cc += m[0] * H0 + m[1] * H1 + m[2] * H2;
+      for (int l0 = 0; l0 < G.zmax; l0 += 4) {
+        // four links at a time: their words, then their ranks, then their
+        // block spins (link order in the sum)
+        uint32_t wd[4];
+        int rt[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) wd[u] = G.rlink[(size_t)ri * G.zmax + (l0 + u < G.zmax ? l0 + u : G.zmax - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rt[u] = G.rrank[wd[u] & 0xFFFFFFu];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (l0 + u >= G.zmax) break;
+          // wide graphs: the block-spin link takes the coupling of the site's
+          // link l; a set high byte marks an absent link
+          if (G.lcid && (wd[u] >> 24)) continue;
+          const float* J =
+              C.coup + (G.lcid ? G.lcid[(size_t)j * G.zmax + l0 + u] : (int)(wd[u] >> 24)) * C.cst;
+          float mt[3];
+          block(rt[u], (int)(wd[u] & 0xFFFFFFu), mt);
+          if constexpr (NC == 1) {
+            cc += J[1] * m[0] * mt[0];
+          } else {
+            float H0 = J[0] * mt[0] + J[1] * mt[1] + J[2] * mt[2];
+            float H1 = J[3] * mt[0] + J[4] * mt[1] + J[5] * mt[2];
+            float H2 = J[6] * mt[0] + J[7] * mt[1] + J[8] * mt[2];
+            cc += m[0] * H0 + m[1] * H1 + m[2] * H2;
+          }
         }
       }
-      w[3] += (double)cc;
+      v[10] += (double)cc;
       // on-site part with the site's actual spin (heisenbergLib.c:798-800,
       // isingLib.c:390)
       float s[3];
-      spin_vec<NC>(sp, j, G.cls, C.clsdat, s);
-      const int ci = G.cls[j];
+      spin_vec<NC>(sp, j, cls, C.clsdat, s);
+      const int ci = cls ? cls[j] : 0;
       float eo;
       if constexpr (NC == 1)
         eo = -h * s[0];
       else
         eo = C.clsdat[ci * 8 + 1] * s[0] * s[0] + C.clsdat[ci * 8 + 2] * s[1] * s[1] +
              C.clsdat[ci * 8 + 3] * s[2] * s[2] - h * (NC == 3 ? s[2] : s[0]);
-      w[4] += (double)eo;
+      v[11] += (double)eo;
     }
-    group_sum<7>(v, C.s_red, C.g, TPR);
-    if (lt == 0)
-      for (int k = 0; k < 7; ++k) F[16 + k] = v[k];
-    group_sum<5>(w, C.s_red, C.g, TPR);
-    if (lt == 0)
-      for (int k = 0; k < 5; ++k) F[24 + k] = w[k];
+    group_add<12>(v, C.s_red, C.g, TPR, [&](int k, double x) { F[k < 7 ? 16 + k : 17 + k] = x; });
   }
   // --- orbital groups (heisenbergLib.c:805-830): 2 groups per reduction
   const int ng = (flags & MCG_MEAS_GROUPS) && !own ? G.ngroup : 0;
@@ -1196,64 +1308,55 @@ __device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, cons
         const int o = G.groups[(g0 + q) * G.gmax + k];
         if (o < 0) continue;
         float s[3];
-        spin_vec<NC>(sp, o, G.cls, C.clsdat, s);
+        spin_vec<NC>(sp, o, cls, C.clsdat, s);
         v[3 * q] += s[0]; v[3 * q + 1] += s[1]; v[3 * q + 2] += s[2];
       }
     }
-    group_sum<6>(v, C.s_red, C.g, TPR);
-    if (lt == 0)
-      for (int k = 0; k < 6; ++k) F[32 + 3 * g0 + k] = v[k];
+    group_add<6>(v, C.s_red, C.g, TPR, [&](int k, double x) { F[32 + 3 * g0 + k] = x; });
   }
 }
 
-// One measured frame of the group's replica at `row`: the spin-derived sums
-// (frame_sums), then frame_apply.
-template <int NC>
-__device__ __forceinline__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
-                            int flags, double mprev, bool have_prev, bool defer);
+// The frame's terms, by the group's first wave: Cn zeroed, lane 0's
+// frame_terms, <M M'> from the row's previous M in *mp (LDS), which gets this
+// frame's M.  Self pairs: the last site's spin is read here.
+template <int NC, typename SV>
+__device__ __forceinline__ void first_wave_terms(const SV& sp, const FrameCtx& C, const mcg_batch& B, const double* st,
+                                                 int64_t frame, int flags, double* mp) {
+  double* F = C.s_frm;
+  double* Cn = F + FRM_ACC;
+  zero_terms(F, 1);
+  if ((threadIdx.x & 63) == 0) {
+    const mcg_graph G = fresh(C.G);
+    if (NC == 1 && (flags & MCG_MEAS_PAIRS) && G.self_pairs) {
+      float t[3];
+      spin_vec<NC>(sp, C.last, G.ncls == 1 ? nullptr : G.cls, C.clsdat, t);
+      F[7] = t[0];
+    }
+    frame_terms<NC>(C, G, B, st, F, flags, frame, Cn);
+    const double Mf = Cn[MCG_A_MM];
+    Cn[MCG_A_MM] = *mp * Mf;
+    *mp = Mf;
+  }
+}
+// One measured frame of the group's replica at `row`, from the tracked state
+// st and the spins; *mp as above.  All threads call it; the accumulators'
+// atomics are queued, not waited for.
 template <int NC, typename SV, bool FULL = true>
 __device__ __forceinline__ void measure_frame(const SV& sp, const FrameCtx& C, const mcg_batch& B, const double* st, int row,
-                              int64_t frame, uint32_t key0, uint32_t key1, float h, double mprev = 0.0,
-                              bool have_prev = false, bool defer = false) {
-  frame_sums<NC, SV, FULL>(sp, C, B, frame, key0, key1, h, 0, 1);
-  frame_apply<NC>(C, B, st, row, frame, FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS), mprev, have_prev, defer);
-}
-
-// This frame's contribution to every FP64 accumulator of the row, from the
-// tracked state st and the spin-derived sums in C.s_frm (valid in the
-// group's first thread); called by every thread of the group.
-template <int NC>
-__device__ __forceinline__ void frame_apply(const FrameCtx& C, const mcg_batch& B, const double* st, int row, int64_t frame,
-                            int flags, double mprev, bool have_prev, bool defer) {
-  const mcg_graph G = fresh(C.G);
-  const int lt = C.lt;
-  double* F = C.s_frm;
-  // --- leader: this frame's contribution to every FP64 accumulator of the
-  //     row (isingLib.c:388-431, heisenbergLib.c:677-830 / xyLib.c:605-757),
-  //     staged in LDS; the group's threads then apply them to global memory
-  //     in parallel (one read-modify-write each instead of a serial chain)
-  double* Cn = F + FRM_ACC;  // [0, NACC) accumulators, [NACC, +NBINQ) bin, then bin index
-  const int ngq = frame_groups<NC>(G, flags);
-  if (lt == 0) frame_terms<NC>(G, B, st, F, flags, frame, Cn);
-  __syncthreads();
-  // A row's accumulators are written by whichever replica holds the row, so
-  // within one persistent launch by workgroups on different XCDs: the
-  // updates go to the device coherence point (device-scope atomics).  M' is
-  // the one value read back: its store must be complete before the row's
-  // next frame (a workgroup barrier or the launch boundary orders it).
-  if (lt == MCG_A_MM) {
-    double* A = B.acc + (size_t)row * MCG_NACC;
-    const double prev = have_prev ? mprev : dev_load(A + MCG_A_MPREV);
-    const double Mf = Cn[MCG_A_MM];
-    Cn[MCG_A_MM] = prev * Mf;
-    dev_store(A + MCG_A_MPREV, Mf);
+                                              int64_t frame, uint32_t key0, uint32_t key1, float h, double* mp) {
+  const int flags = FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS);
+  if (FULL) frame_sums<NC, SV, FULL>(sp, C, B, frame, key0, key1, h, 0, 1);
+  if (C.lt < 64) {
+    wave_lds_fence();
+    first_wave_terms<NC>(sp, C, B, st, frame, flags, mp);
   }
-  if (!defer) flush_frame<NC>(C, B, row, flags);
+  __syncthreads();
+  flush_frame<NC>(C, B, row, flags);
 }
 
-// full FP64 recomputation of one replica (group-parallel): out[0] E,
-// out[1..3] M, out[4] the summed relative spin-length deviation
-// sum_i | |s_i|^2 / S_i^2 - 1 | (0 for Ising)
+// full FP64 recomputation of one replica (group-parallel): out[0] E (out:
+// LDS, complete at return), out[1..3] M, out[4] the summed relative
+// spin-length deviation sum_i | |s_i|^2 / S_i^2 - 1 | (0 for Ising)
 static constexpr int NREC = 5;
 template <int NC, typename SV>
 __device__ __forceinline__ void recompute(const SV& sp, const mcg_graph* Gd, const float* coup, int cst, const float* clsdat, float h,
@@ -1276,9 +1379,7 @@ __device__ __forceinline__ void recompute(const SV& sp, const mcg_graph* Gd, con
       v[4] += fabs(fma(l2, (double)clsdat[G.cls[i] * 8 + 4], -1.0));
     }
   }
-  group_sum<NREC>(v, s_red, g, TPR);
-  if (lt == 0)
-    for (int k = 0; k < NREC; ++k) out[k] = v[k];
+  group_add<NREC>(v, s_red, g, TPR, [&](int k, double x) { out[k] = x; });
 }
 
 // Health checks on a recompute (called by the thread holding its result;
@@ -1360,6 +1461,7 @@ struct SweepArgs {
   int32_t fspin_n;
   int32_t max_export;
   int32_t nslots;
+  int32_t blk;               // LDS bytes per group for a frame's block spins, after the spins (0: none)
   int32_t rec_host;          // the full recompute is the host's (a launch ends at each
                              // recompute sweep, then k_measure recomputes every replica)
 };
@@ -1382,7 +1484,6 @@ __host__ __device__ inline size_t persist_lds_bytes(int nrow, int nrep) {
          align16((size_t)nrep);
 }
 
-static constexpr int FRM = 96 + 48;  // frame scratch doubles per group: scalars, then accumulator staging
 
 
 // copy one replica between HBM (16-byte aligned) and LDS in 16-byte vectors,
@@ -1421,7 +1522,7 @@ __host__ __device__ inline size_t lds_fixed_bytes(int ncoup, int ncls, int ncol,
                                                   int nwaves, int R) {
   size_t b = align16((size_t)(ncoup * COUP_LDS + ncls * 8) * 4) + align16((size_t)(ncol + 1) * 4);
   if (npat > 0) b += align16((size_t)npat * pat_stride(zmax) * 4) + align16((size_t)n);
-  return b + align16((size_t)nwaves * RK * 8) + align16((size_t)R * (MCG_NSTATE + FRM) * 8) + align16((size_t)R * 16);
+  return b + align16((size_t)nwaves * RK * 8) + align16((size_t)R * (MCG_NSTATE + FRM + 1) * 8) + align16((size_t)R * 16);
 }
 
 __host__ __device__ inline size_t lds_replica_bytes(int nc, int n, int ssize) {
@@ -1622,32 +1723,55 @@ struct PartInfo {
   const int32_t* halo = nullptr;
 };
 
-// end-of-sweep work after the state is current: full recompute (drift
-// check), energy reference at the end of thermalisation, measured frame
+// End-of-sweep work of an unsplit replica (or of the last part of a split
+// one) outside a persistent launch: the state takes the sweeps' changes dE,
+// dM (and the pool's), then full recompute (drift check), energy reference at
+// the end of thermalisation, measured frame.  With no recompute and no pass
+// over the spins the first wave does all of it between two barriers.
 template <int NC, typename ST, bool FULL, typename SV>
-__device__ __forceinline__ void tail_rest(const SV& sv, const mcg_graph& G, const mcg_batch& B, const float* s_coup,
-                                          const float* s_cls, double* s_red, double* st, FrameCtx& C, int g, int lt,
-                                          int TPR, int row, float h, int64_t k, const SweepArgs& a, bool meas,
-                                          bool therm_end, bool rec, uint32_t key0, uint32_t key1,
-                                          double mprev = 0.0, bool have_prev = false, bool defer = false) {
+__device__ __forceinline__ void lds_sweep_tail(const SV& sv, const mcg_graph& G, const mcg_batch& B, double* st,
+                                               FrameCtx& C, int row, float h, int64_t k, const SweepArgs& a, bool meas,
+                                               bool therm_end, bool rec, double& dE, double* dM, uint32_t key0,
+                                               uint32_t key1, double* mp, const PoolInfo<ST>& pl) {
+  const double v[4] = {dE, dM[0], dM[1], dM[2]};
+  const int flags = FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS);
+  const bool light = !rec && (!FULL || frame_light(G, B.meas));
+  const int64_t frame = meas ? (k - a.nthermal + 1) / a.spf - 1 + a.frame0 : 0;
+  group_add<4>(
+      v, C.s_red, C.g, C.TPR,
+      [&](int q, double x) {
+        if (pl.rem > 0 && q <= NC) {
+          double ps = 0.0;
+          for (int i = 0; i < pl.rem; ++i) ps += pl.pp[q * pl.nr + C.g * pl.rem + i];
+          x += ps;
+        }
+        st[MCG_S_E + q] += x;
+      },
+      [&] {
+        if (!light) return;
+        if (therm_end && C.lt == 0) st[MCG_S_EREF] = st[MCG_S_E];
+        if (pl.rem > 0 || !meas) return;  // with a pool, other groups' partials are in the frame area until all are read
+        first_wave_terms<NC>(sv, C, B, st, frame, flags, mp);
+      });
+  dE = 0.0;
+  dM[0] = dM[1] = dM[2] = 0.0;
+  if (light && pl.rem == 0) {
+    if (meas) flush_frame<NC>(C, B, row, flags);
+    return;
+  }
   if (rec) {
-    double r4[NREC];
-    recompute<NC>(sv, C.G, s_coup, C.cst, s_cls, h, s_red, g, lt, TPR, r4);
-    if (lt == 0) {
+    double* r4 = C.s_frm;  // the frame area
+    recompute<NC>(sv, C.G, C.coup, C.cst, C.clsdat, h, C.s_red, C.g, C.lt, C.TPR, r4);
+    if (C.lt == 0) {
       const double d = fabs(st[MCG_S_E] - r4[0]);
       if (d > st[MCG_S_DRIFT]) st[MCG_S_DRIFT] = d;
-      st[MCG_S_E] = r4[0];
-      st[MCG_S_M] = r4[1];
-      st[MCG_S_M + 1] = r4[2];
-      st[MCG_S_M + 2] = r4[3];
+      for (int q = 0; q < 4; ++q) st[MCG_S_E + q] = r4[q];
       recompute_checks<ST>(B, G, r4, d);
     }
   }
-  if (therm_end && lt == 0) st[MCG_S_EREF] = st[MCG_S_E];
+  if (therm_end && !light && C.lt == 0) st[MCG_S_EREF] = st[MCG_S_E];
   __syncthreads();
-  if (meas)
-    measure_frame<NC, SV, FULL>(sv, C, B, st, row, (k - a.nthermal + 1) / a.spf - 1 + a.frame0, key0, key1, h, mprev,
-                                have_prev, defer);
+  if (meas) measure_frame<NC, SV, FULL>(sv, C, B, st, row, frame, key0, key1, h, mp);
   __syncthreads();
 }
 
@@ -1749,12 +1873,12 @@ __device__ __forceinline__ double frame_mprev3(const SweepArgs& a, int64_t f, in
   return dev_load(a.mprev3 + (size_t)((f + 2) % 3) * nrow + row);
 }
 template <int NC>
-__device__ __forceinline__ void take_frame(const mcg_graph* Gd, const mcg_batch& B, const SweepArgs& a, double* s_st,
+__device__ __forceinline__ void take_frame(const FrameCtx& C, const mcg_batch& B, const SweepArgs& a, double* s_st,
                                            double* s_frm, int lane, int64_t f, int row, int nrow, double mp,
                                            int flags) {
   double* F = s_frm + lane * FRM;
   double* Cn = F + FRM_ACC;
-  frame_terms<NC>(fresh(Gd), B, s_st + lane * MCG_NSTATE, F, flags, f, Cn);
+  frame_terms<NC>(C, fresh(C.G), B, s_st + lane * MCG_NSTATE, F, flags, f, Cn);
   const double Mf = Cn[MCG_A_MM];
   Cn[MCG_A_MM] = mp * Mf;
   dev_store(a.mprev3 + (size_t)(f % 3) * nrow + row, Mf);
@@ -1813,113 +1937,70 @@ __device__ __forceinline__ bool gather_frame_sums(const SweepArgs& a, const mcg_
   return true;
 }
 
-// End of a persistent sweep for a workgroup of unsplit replicas: the state
-// update (and published energy) of every replica is done by the
-// workgroup's first wave, lane g for group g, so that this serial
-// per-replica work runs once per workgroup instead of once in every group.
-// The sums are group_sum's (each wave's DPP total, then the same DPP steps
-// over a group's waves).  rep_l: lane g's replica; eslot_par: the energy
-// slots of this sweep's parity, or nullptr to publish nothing.  Called by
-// every thread; ends with a workgroup barrier.
-// Pool partials (PoolInfo): thread t's ΔE, ΔM of its pool groups are kept
-// in pp[k*nr + t] (nr = R*rem, k < NC+1; pp is the frame area, free between
-// a sweep's frames and the next tail); pool_sums gives replica g the sum of
-// its rem entries in thread order.
-template <int NC>
-__device__ __forceinline__ void pool_sums(const double* pp, int nr, int rem, int g, double* out) {
-  for (int k = 0; k <= NC; ++k) {
-    double x = 0.0;
-    for (int i = 0; i < rem; ++i) x += pp[k * nr + g * rem + i];
-    out[k] = x;
-  }
-}
-
-// The sweep's ΔE, ΔM of every group, in the first wave: lane g gets group
-// g's totals in t (the other waves get zeros).  The sums are group_sum's
-// (each wave's DPP total, then the same DPP steps over a group's waves).
+// Totals of every group's changes v[0..NC] (E, M) over its waves, in the
+// workgroup's first wave: sink(g, k, total) by one lane per group and value.
 // Called by every thread; s_red is free again only after the caller's next
 // workgroup barrier.
-template <int NC>
-__device__ __forceinline__ void wave0_sums(double* s_red, int TPR, float fE, const float* fM, double* t) {
-  constexpr int NV = NC + 1;  // E and the spin components (the rest stay 0)
-  double v[4] = {(double)fE, (double)fM[0], (double)fM[1], (double)fM[2]};
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = wave_sum_f64(v[k]);
+template <int NC, typename F>
+__device__ __forceinline__ void wave0_add(double* s_red, int TPR, const double* v, F&& sink) {
+  double r[1];
+  wave_totals<NC + 1>(v, r);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 63)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) s_red[wave * RK + k] = v[k];
+  if (lane < 4) s_red[wave * RK + lane] = r[0];
   __syncthreads();
-  t[0] = t[1] = t[2] = t[3] = 0.0;
   if (wave == 0) {
     const int nw = TPR >> 6, nwaves = (int)blockDim.x >> 6;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      double x = lane < nwaves ? s_red[lane * RK + k] : 0.0;
-      if (nw >= 2) x += dpp_f64<0xB1, 0xF>(x);   // quad_perm [1,0,3,2]
-      if (nw >= 4) x += dpp_f64<0x4E, 0xF>(x);   // quad_perm [2,3,0,1]
-      if (nw >= 8) x += dpp_f64<0x141, 0xF>(x);  // row_half_mirror
-      if (nw >= 16) x += dpp_f64<0x140, 0xF>(x); // row_mirror
-      t[k] = bperm_f64(x, lane * nw);
+    const int k = lane & 3;
+    double x = 0.0;
+    if (nw == 8 || nw == 16) {
+      // lane 4 w + k holds wave w's value k
+      x = (lane >> 2) < nwaves ? s_red[(lane >> 2) * RK + k] : 0.0;
+      x += dpp_f64<0x124, 0xF>(x);  // row_ror:4
+      x += dpp_f64<0x128, 0xF>(x);  // row_ror:8
+      x = add_lane16(x);
+      if (nw == 16) x = add_lane32(x);
+      const int g = (lane >> 2) / nw;
+      if ((lane >> 2) == g * nw && g * nw < nwaves && k <= NC) sink(g, k, x);
+    } else {
+      const int g = lane >> 2;  // at most 16 groups
+      if (g * nw < nwaves && k <= NC) {
+        for (int w = 0; w < nw; ++w) x += s_red[(g * nw + w) * RK + k];
+        sink(g, k, x);
+      }
     }
   }
 }
 
+// End of a persistent sweep for a workgroup of unsplit replicas: the state
+// update (and published energy) of every replica is done by the workgroup's
+// first wave, so that this serial per-replica work runs once per workgroup
+// instead of once in every group.  rep_l: lane g's replica; eslot_par: the
+// energy slots of this sweep's parity, or nullptr to publish nothing.  Called
+// by every thread; ends with a workgroup barrier.  Pool partials (PoolInfo):
+// thread t's changes are kept in pp[k*nr + t] (nr = R*rem, k < NC+1; pp is the
+// frame area, free between a sweep's frames and the next tail); replica g
+// adds its rem entries in thread order.
 template <int NC>
-__device__ __forceinline__ void tail_wave0(const mcg_batch& B, double* s_red, double* s_st, int R, int TPR, float fE,
-                                           const float* fM, bool therm_end, int rep_l, double* eslot_par,
-                                           const double* pp, int prem) {
-  constexpr int NV = NC + 1;
-  double t[4];
-  wave0_sums<NC>(s_red, TPR, fE, fM, t);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave == 0) {
+__device__ __forceinline__ void tail_wave0(double* s_red, double* s_st, int R, int TPR, const double* v, bool therm_end,
+                                           int rep_l, double* eslot_par, const double* pp, int prem) {
+  wave0_add<NC>(s_red, TPR, v, [&](int g, int k, double x) {
     if (prem > 0) {
-      // a replica's sweep change: its groups' sum plus its pool groups' sum
-      // (pool_sums' order); lane 16k+g adds term k of replica g, R <= 16
-      const int gk = lane & 15, kk = lane >> 4;
-      double x = 0.0;
-      if (gk < R && kk < NV)
-        for (int i = 0; i < prem; ++i) x += pp[kk * R * prem + gk * prem + i];
-#pragma unroll
-      for (int k = 0; k < NV; ++k) t[k] += bperm_f64(x, 16 * k + (lane & 15));
+      double ps = 0.0;
+      for (int i = 0; i < prem; ++i) ps += pp[k * R * prem + g * prem + i];
+      x += ps;
     }
+    s_st[g * MCG_NSTATE + MCG_S_E + k] += x;
+  });
+  if (threadIdx.x < 64) {
+    wave_lds_fence();
+    const int lane = threadIdx.x;
     if (lane < R) {
       double* st = s_st + lane * MCG_NSTATE;
-#pragma unroll
-      for (int k = 0; k < NV; ++k) st[MCG_S_E + k] += t[k];
       if (therm_end) st[MCG_S_EREF] = st[MCG_S_E];
       if (eslot_par) dev_store(eslot_par + (size_t)rep_l * MAX_PARTS, st[MCG_S_E]);
     }
   }
   __syncthreads();
-}
-
-template <int NC, typename ST, bool FULL, typename SV>
-__device__ __forceinline__ void lds_sweep_tail(const SV& sv, const mcg_graph& G, const mcg_batch& B, const float* s_coup,
-                                               const float* s_cls, double* s_red, double* st, FrameCtx& C, int g,
-                                               int lt, int TPR, int row, float h, int64_t k, const SweepArgs& a,
-                                               bool meas, bool therm_end, bool rec, double& dE, double* dM,
-                                               uint32_t key0, uint32_t key1, double mprev, bool have_prev,
-                                               const PoolInfo<ST>& pl) {
-  double v[RK] = {dE, dM[0], dM[1], dM[2], 0, 0, 0, 0};
-  group_sum<4>(v, s_red, g, TPR);
-  if (lt == 0) {
-    if (pl.rem > 0) {
-      double ps[4];
-      pool_sums<NC>(pl.pp, pl.nr, pl.rem, g, ps);
-      for (int k = 0; k <= NC; ++k) v[k] += ps[k];
-    }
-    st[MCG_S_E] += v[0];
-    st[MCG_S_M] += v[1];
-    st[MCG_S_M + 1] += v[2];
-    st[MCG_S_M + 2] += v[3];
-  }
-
-  dE = 0.0;
-  dM[0] = dM[1] = dM[2] = 0.0;
-  tail_rest<NC, ST, FULL>(sv, G, B, s_coup, s_cls, s_red, st, C, g, lt, TPR, row, h, k, a, meas, therm_end, rec, key0,
-                          key1, mprev, have_prev);
 }
 
 // one sweep of a workgroup's replica group: every colour class in turn,
@@ -2019,10 +2100,9 @@ template <int NC, typename ST, int MODE, bool FULL>
 __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& B, const SweepArgs& a,
                                            const Spins<ST>& sp, const float* coup,
                                            const float* clsdat, const int32_t* s_colptr, const uint8_t* s_pid,
-                                           const int32_t* s_pat, double* s_red, double* st, FrameCtx& C, int g,
-                                           int lt, int TPR, int row, float beta, float h, uint32_t key0,
-                                           uint32_t key1, const PartInfo& pi, double& dE, double* dM, bool aniso,
-                                           const PoolInfo<ST>& pl) {
+                                           const int32_t* s_pat, double* st, FrameCtx& C, int lt, int TPR, int row,
+                                           float beta, float h, uint32_t key0, uint32_t key1, const PartInfo& pi,
+                                           double& dE, double* dM, bool aniso, const PoolInfo<ST>& pl, double* mp) {
   const bool split = pi.np > 1;
   dE = 0.0;
   dM[0] = dM[1] = dM[2] = 0.0;
@@ -2031,12 +2111,9 @@ __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& 
     const int64_t k = a.k_begin + s;
     const uint64_t kk = (uint64_t)(a.philox_base + k);
     const bool meas = k >= a.nthermal && ((k - a.nthermal + 1) % a.spf) == 0;
-    double mprev = 0.0;  // read ahead, so that the frame does not wait for it
-    if (meas && !split && lt == MCG_A_MM) mprev = frame_mprev(B, row);
     float fE = 0.0f, fM[3] = {0.0f, 0.0f, 0.0f};  // this sweep's accepted changes
     sweep_colours<NC, ST, MODE>(G, sp, coup, clsdat, s_colptr, s_pid, s_pat, lt, TPR, acc_of(B, beta, row), h, kk, key0,
-                                key1, pi, fE,
-                                fM, aniso, pl, pfresh);
+                                key1, pi, fE, fM, aniso, pl, pfresh);
     pfresh = false;
     dE += (double)fE;
     dM[0] += (double)fM[0];
@@ -2046,8 +2123,7 @@ __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& 
     const bool therm_end = (k + 1 == a.nthermal);
     const bool rec = recompute_due(B, a.philox_base + k);
     if (meas || therm_end || rec || s == a.nsweeps - 1) {
-      lds_sweep_tail<NC, ST, FULL>(sp, G, B, coup, clsdat, s_red, st, C, g, lt, TPR, row, h, k, a, meas, therm_end,
-                                   rec, dE, dM, key0, key1, mprev, true, pl);
+      lds_sweep_tail<NC, ST, FULL>(sp, G, B, st, C, row, h, k, a, meas, therm_end, rec, dE, dM, key0, key1, mp, pl);
       pfresh = true;
     }
   }
@@ -2095,7 +2171,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   off += align16((size_t)nwaves * RK * 8);
   double* s_st = (double*)(smem + off);  // R * NSTATE
   double* s_frm = s_st + R * MCG_NSTATE;  // R * FRM
-  off += align16((size_t)R * (MCG_NSTATE + FRM) * 8);
+  double* s_mp = s_frm + R * FRM;         // the rows' previous M
+  off += align16((size_t)R * (MCG_NSTATE + FRM + 1) * 8);
   float4* s_par = (float4*)(smem + off);  // per group: beta, h, key1 bits (the pool's parameters)
   off += align16((size_t)R * 16);
   unsigned char* s_pers = smem + off;  // tempering state of a persistent launch
@@ -2159,6 +2236,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
     pi.halo = a.halo;
   }
   FrameCtx C{B.graphs + w.graph, wide ? G.coup : s_coup, wide ? 9 : COUP_LDS, wide ? G.clsdat : s_clsl, s_red, s_frm + g * FRM, g, lt, TPR};
+  frame_consts<NC>(C, G, B);
+  if (FULL && a.blk && w.nparts <= 1) C.blk = (float*)((unsigned char*)s_spin + R * lds_replica_bytes(NC, n, sizeof(ST)) + g * a.blk);
   if constexpr (PERSIST) {
     // Persistent launch: many sweeps with the replicas in LDS.  After each
     // sweep every replica's energy is published at the device coherence
@@ -2242,18 +2321,39 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       const double m0 = B.acc[(size_t)r * MCG_NACC + MCG_A_MPREV];
       for (int q = 0; q < 3; ++q) dev_store(a.mprev3 + (size_t)q * nrow + r, m0);
     }
+    // The sweeps' changes are added up (FP64, per thread) until a sweep needs
+    // the energies: a frame, a swap pass, a recompute, the end.  Sweeps in
+    // between end without the reduction over the workgroup.
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    bool vfresh = true;
+    // sweeps until the next frame, swap pass and recompute (each event's
+    // period, 0: never), so that no sweep divides 64-bit indices
+    const int64_t gs0 = a.philox_base + a.k_begin;
+    const int rec_every = a.rec_host ? 0 : B.recompute_every;
+    auto until = [&](int every) {  // sweeps from gs0 on until one with (index + 1) % every == 0
+      if (every <= 0) return 0;
+      const int m = (int)(gs0 % every);
+      return m < 0 ? -m : every - m;
+    };
+    int to_pt = until(a.pt_every), to_rec = until(rec_every);
+    int64_t fcur = a.k_begin > a.nthermal ? (a.k_begin - a.nthermal) / a.spf + a.frame0 : a.frame0;  // next frame
+    int64_t to_frame = a.k_begin > a.nthermal ? a.spf - (a.k_begin - a.nthermal) % a.spf
+                                              : (int64_t)a.nthermal - a.k_begin + a.spf;
     for (int s = 0; s < a.nsweeps; ++s) {
       const int64_t k = a.k_begin + s;
       const uint64_t kk = (uint64_t)(a.philox_base + k);
       const int par = (int)(k & 1);
       const int rowg = wave_uniform(ir.row0 + s_rung[rep]);
       const float bg = wave_uniform(s_beta[rowg]), hg = wave_uniform(s_h[rowg]);
-      const bool meas = k >= a.nthermal && ((k - a.nthermal + 1) % a.spf) == 0;
+      const bool meas = --to_frame == 0;
       const bool therm_end = (k + 1 == a.nthermal);
-      const bool rec = !a.rec_host && recompute_due(B, a.philox_base + k);
-      const bool pt_now = a.pt_every > 0 && ((a.philox_base + k + 1) % a.pt_every) == 0;
+      const bool rec = --to_rec == 0;
+      const bool pt_now = --to_pt == 0;
+      if (meas) to_frame = a.spf;
+      if (rec) to_rec = rec_every;
+      if (pt_now) to_pt = a.pt_every;
+      const bool need = meas || therm_end || rec || pt_now || s == a.nsweeps - 1;
       const int rowg_l = row0_l + s_rung[rep_l];
-      const int64_t fcur = (k - a.nthermal + 1) / a.spf - 1 + a.frame0;
       if (pl.rem > 0) {  // the pool's parameters of this sweep (rows move with tempering)
         if (lt == 0) s_par[g] = make_float4(bg, hg, __uint_as_float(key1), __int_as_float(rowg));
         __syncthreads();
@@ -2261,17 +2361,25 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       float fE = 0.0f, fM[3] = {0.0f, 0.0f, 0.0f};
       sweep_colours<NC, ST, MODE>(G, sp, C.coup, C.clsdat, s_colptr, s_pid, s_pat, lt, TPR, acc_of(B, bg, rowg), hg, kk,
                                   key0, key1, pi,
-                                  fE, fM, aniso, pl, true);
-      double v[RK] = {(double)fE, (double)fM[0], (double)fM[1], (double)fM[2], 0.0, 0.0, 0.0, 0.0};
+                                  fE, fM, aniso, pl, vfresh);
+      vfresh = false;
+      v[0] += (double)fE;
+      v[1] += (double)fM[0];
+      v[2] += (double)fM[1];
+      v[3] += (double)fM[2];
       double* es = a.eslot + ((size_t)par * nrepb + rep) * MAX_PARTS;
       double* ms = a.mslot + ((size_t)par * nrepb + rep) * MAX_PARTS * 3;
       if (pi.np == 1) {
         // state update and published energy before the barrier (with a full
         // recompute due, the recomputed state is published instead)
-        tail_wave0<NC>(B, s_red, s_st, R, TPR, fE, fM, therm_end && !rec, rep_l,
-                       rec ? nullptr : a.eslot + (size_t)par * nrepb * MAX_PARTS, s_frm, pl.rem);
+        if (need) {
+          tail_wave0<NC>(s_red, s_st, R, TPR, v, therm_end && !rec, rep_l,
+                         rec ? nullptr : a.eslot + (size_t)par * nrepb * MAX_PARTS, s_frm, pl.rem);
+          vfresh = true;
+          v[0] = v[1] = v[2] = v[3] = 0.0;
+        }
         if (rec) {
-          double r4[NREC];
+          double* r4 = C.s_frm;
           recompute<NC>(sp, C.G, C.coup, C.cst, C.clsdat, hg, s_red, g, lt, TPR, r4);
           if (lt == 0) {
             const double d = fabs(st[MCG_S_E] - r4[0]);
@@ -2286,14 +2394,22 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
         if constexpr (FULL) {
           // the spin-derived sums of every group's frame, from its LDS
           // replica (the frame area is free after the tail)
-          if (meas) frame_sums<NC, Spins<ST>, true>(sp, C, B, fcur, key0, key1, hg, 0, 1);
+          if (meas) {
+            frame_sums<NC, Spins<ST>, true>(sp, C, B, fcur, key0, key1, hg, 0, 1);
+            if (!frames_after) __syncthreads();  // the first wave takes every group's frame
+          }
         }
       } else {
-        // one replica: lane 0 of the first wave gets the part's sums
-        wave0_sums<NC>(s_red, TPR, fE, fM, v);
-        if (threadIdx.x == 0) {
-          dev_store(es + pi.part, (pi.part == 0 ? st[MCG_S_E] : 0.0) + v[0]);
-          for (int q = 0; q < 3; ++q) dev_store(ms + pi.part * 3 + q, v[1 + q]);
+        // one replica: the part's sums, published and kept in LDS
+        if (need) {
+          wave0_add<NC>(s_red, TPR, v, [&](int, int q, double x) {
+            if (q == 0)
+              dev_store(es + pi.part, (pi.part == 0 ? st[MCG_S_E] : 0.0) + x);
+            else
+              dev_store(ms + pi.part * 3 + (q - 1), x);
+            s_frm[FRM - 4 + q] = x;
+          });
+          v[0] = v[1] = v[2] = v[3] = 0.0;
         }
         const int32_t* ex = a.halo + pi.hx[2 * G.ncol];
         const int nex = pi.hx[2 * G.ncol + 1];
@@ -2317,8 +2433,9 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
                              NC, s_colptr, G.ncol, GD, pi.part, pi.np, lt, TPR);
         }
       }
+      if (meas && threadIdx.x < 64 && nfr > 0) zero_terms(s_frm, nfr);
       if (meas && l_grp && !frames_after) {
-        take_frame<NC>(C.G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, frame_mprev3<NC>(a, fcur, rowg_l, nrow),
+        take_frame<NC>(C, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, frame_mprev3<NC>(a, fcur, rowg_l, nrow),
                        fflags);
         last_row = rowg_l;
       }
@@ -2346,7 +2463,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       if (meas && l_grp && frames_after) mp = frame_mprev3<NC>(a, fcur, rowg_l, nrow);
       if (pi.np > 1) {
         // part 0 reads part p's sums in lane p, overlapping the import
-        const bool w0 = pi.part == 0 && threadIdx.x < 64;
+        const bool w0 = need && pi.part == 0 && threadIdx.x < 64;
         double pe = 0.0, pm[3] = {0.0, 0.0, 0.0};
         if (w0 && lane >= 1 && lane < pi.np) {
           pe = dev_load(es + lane);
@@ -2381,7 +2498,8 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
                            a.max_export, a.halo, pi.hx, DS, G.ncol, pi.part, pi.np, lraw, n, lt, TPR);
         }
         if (w0) {
-          double E = st[MCG_S_E] + v[0], dm[3] = {v[1], v[2], v[3]};
+          const double* own = s_frm + FRM - 4;  // this part's sums
+          double E = st[MCG_S_E] + own[0], dm[3] = {own[1], NC > 1 ? own[2] : 0.0, NC > 2 ? own[3] : 0.0};
           for (int p = 1; p < pi.np; ++p) {
             E += lane_f64(pe, p);
             for (int q = 0; q < 3; ++q) dm[q] += lane_f64(pm[q], p);
@@ -2427,7 +2545,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       // the frame of every replica (first wave, lane g), while the other
       // waves run the tempering pass
       if (meas && l_grp && frames_after) {
-        take_frame<NC>(C.G, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, mp, fflags);
+        take_frame<NC>(C, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, mp, fflags);
         last_row = rowg_l;
       }
       if (pt_now) {
@@ -2488,6 +2606,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
         __syncthreads();
         if (g < nfr) flush_frame<NC>(C, B, rowg, fflags);
       }
+      if (meas) ++fcur;
     }
     __syncthreads();
     if (last_row >= 0) {
@@ -2515,19 +2634,15 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
     return;
   } else {
   double dE, dM[3];
-  if constexpr (MODE == 0 || MODE == 3)
-    lds_sweeps<NC, ST, MODE, FULL>(G, B, a, sp, s_coup, s_clsl, s_colptr, s_pid, s_pat, s_red, st, C, g, lt, TPR, row,
-                                   beta, h, key0, key1, pi, dE, dM, aniso, pl);
-  else if constexpr (MODE == 1)
-    lds_sweeps<NC, ST, 1, FULL>(G, B, a, sp, s_coup, s_clsl, s_colptr, s_pid, s_pat, s_red, st, C, g, lt, TPR, row,
-                                beta, h, key0, key1, pi, dE, dM, aniso, pl);
-  else
-    lds_sweeps<NC, ST, 2, FULL>(G, B, a, sp, G.coup, G.clsdat, s_colptr, s_pid, s_pat, s_red, st, C, g, lt, TPR,
-                                row, beta, h, key0, key1, pi, dE, dM, aniso, pl);
+  double* mp = s_mp + g;
+  if (lt == 0) *mp = B.acc[(size_t)row * MCG_NACC + MCG_A_MPREV];  // read by the same thread
+  lds_sweeps<NC, ST, MODE, FULL>(G, B, a, sp, C.coup, C.clsdat, s_colptr, s_pid, s_pat, st, C, lt, TPR, row, beta, h,
+                                 key0, key1, pi, dE, dM, aniso, pl, mp);
   __syncthreads();
   if (pi.np == 1) {
     stage<ST, false>(my, gsp, NC * n, lt, TPR);
     if (lt < MCG_NSTATE) B.state[(size_t)rep * MCG_NSTATE + lt] = st[lt];
+    if (lt == 0 && a.k_begin + a.nsweeps > a.nthermal) B.acc[(size_t)row * MCG_NACC + MCG_A_MPREV] = *mp;
     return;
   }
   // split replica (one workgroup per part, R = 1): write back own sites,
@@ -2545,10 +2660,12 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   uint32_t* ctr = a.sync + (size_t)w.slot * SYNC_STRIDE;
   double* xp = a.xpart + (size_t)w.slot * MAX_PARTS * 4;
   part_copy<ST, true>(my, gsp, n, NC, s_colptr, G.ncol, GD, pi.part, pi.np, lt, TPR);
-  double v[RK] = {dE, dM[0], dM[1], dM[2], 0.0, 0.0, 0.0, 0.0};
-  group_sum<4>(v, s_red, g, TPR);
-  if (lt == 0)
-    for (int q = 0; q < 4; ++q) dev_store(xp + pi.part * 4 + q, v[q]);
+  const double v[4] = {dE, dM[0], dM[1], dM[2]};
+  double* tot = s_frm;  // this part's sums (the frame area)
+  group_add<4>(v, s_red, g, TPR, [&](int q, double x) {
+    tot[q] = x;
+    dev_store(xp + pi.part * 4 + q, x);
+  });
   stores_done();
   __syncthreads();
   int* s_last = (int*)s_red;
@@ -2567,12 +2684,14 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   double tE = 0.0, tM[3] = {0.0, 0.0, 0.0};
   if (lt == 0)
     for (int p = 0; p < pi.np; ++p) {
-      tE += p == pi.part ? v[0] : dev_load(xp + p * 4);
-      for (int q = 0; q < 3; ++q) tM[q] += p == pi.part ? v[1 + q] : dev_load(xp + p * 4 + 1 + q);
+      tE += p == pi.part ? tot[0] : dev_load(xp + p * 4);
+      for (int q = 0; q < 3; ++q) tM[q] += p == pi.part ? tot[1 + q] : dev_load(xp + p * 4 + 1 + q);
     }
+  if (lt == 0) *mp = frame_mprev(B, row);  // an earlier launch's last part stored it
   __syncthreads();
-  lds_sweep_tail<NC, ST, FULL>(sp, G, B, C.coup, C.clsdat, s_red, st, C, g, lt, TPR, row, h, k, a, meas, therm_end,
-                               rec, tE, tM, key0, key1, 0.0, false, PoolInfo<ST>{});
+  lds_sweep_tail<NC, ST, FULL>(sp, G, B, st, C, row, h, k, a, meas, therm_end, rec, tE, tM, key0, key1, mp,
+                               PoolInfo<ST>{});
+  if (meas && lt == 0) dev_store(B.acc + (size_t)row * MCG_NACC + MCG_A_MPREV, *mp);
   if (lt < MCG_NSTATE) B.state[(size_t)rep * MCG_NSTATE + lt] = st[lt];
   }
 }
@@ -2728,7 +2847,7 @@ __global__ __launch_bounds__(1024) void k_measure(mcg_batch B, const int32_t* __
   if (threadIdx.x < MCG_NSTATE) st[threadIdx.x] = B.state[(size_t)rep * MCG_NSTATE + threadIdx.x];
   __syncthreads();
   if (mode & 1) {
-    double r4[NREC];
+    double* r4 = s_frm;
     recompute<NC>(sp, B.graphs + rp.graph, G.coup, 9, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r4);
     if (threadIdx.x == 0) {
       double d = 0.0;
@@ -2747,7 +2866,11 @@ __global__ __launch_bounds__(1024) void k_measure(mcg_batch B, const int32_t* __
   __syncthreads();
   if (mode & 4) {
     FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
-    measure_frame<NC>(sp, C, B, st, row, frame, B.seed_lo, B.seed_hi ^ rp.serial, h);
+    frame_consts<NC>(C, G, B);
+    __shared__ double mp;
+    if (threadIdx.x == 0) mp = frame_mprev(B, row);
+    measure_frame<NC>(sp, C, B, st, row, frame, B.seed_lo, B.seed_hi ^ rp.serial, h, &mp);
+    if (threadIdx.x == 0) B.acc[(size_t)row * MCG_NACC + MCG_A_MPREV] = mp;
   }
   __syncthreads();
   if (threadIdx.x < MCG_NSTATE) B.state[(size_t)rep * MCG_NSTATE + threadIdx.x] = st[threadIdx.x];
@@ -2778,20 +2901,20 @@ __global__ __launch_bounds__(256) void k_frame_part(mcg_batch B, const int32_t* 
   const int part = item % np;
   double* out = fsum + (size_t)rep * FSLOTS;
   if (mode & 1) {
-    double r[NREC];
+    double* r = s_frm;
     recompute<NC>(sp, B.graphs + rp.graph, G.coup, 9, G.clsdat, h, s_red, 0, threadIdx.x, blockDim.x, r, part, np);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < NREC; ++k)
-        if (r[k] != 0.0) atomicAdd(out + FSUMS + k, r[k]);
+    if (threadIdx.x < NREC && r[threadIdx.x] != 0.0) atomicAdd(out + FSUMS + threadIdx.x, r[threadIdx.x]);
+    __syncthreads();
   }
   if (mode & 4) {
     for (int t = threadIdx.x; t < FSUMS; t += blockDim.x) s_frm[t] = 0.0;
     __syncthreads();
     FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, (int)threadIdx.x, (int)blockDim.x};
+    frame_consts<NC>(C, G, B);
     frame_sums<NC>(sp, C, B, frame, B.seed_lo, B.seed_hi ^ rp.serial, h, part, np);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < FSUMS; ++k)
-        if (s_frm[k] != 0.0) atomicAdd(out + k, s_frm[k]);
+    __syncthreads();  // F is written by the first wave (or thread)
+    for (int k = threadIdx.x; k < FSUMS; k += blockDim.x)
+      if (s_frm[k] != 0.0) atomicAdd(out + k, s_frm[k]);
   }
 }
 
@@ -2825,7 +2948,18 @@ __global__ __launch_bounds__(64) void k_frame_end(mcg_batch B, const int32_t* __
   __syncthreads();
   if (mode & 4) {
     FrameCtx C{B.graphs + rp.graph, G.coup, 9, G.clsdat, s_red, s_frm, 0, lt, (int)blockDim.x};
-    frame_apply<NC>(C, B, st, row, frame, B.meas, 0.0, false, false);
+    frame_consts<NC>(C, G, B);
+    zero_terms(s_frm, 1);
+    if (lt == 0) {
+      double* Cn = s_frm + FRM_ACC;
+      frame_terms<NC>(C, G, B, st, s_frm, B.meas, frame, Cn);
+      double* mprev = B.acc + (size_t)row * MCG_NACC + MCG_A_MPREV;
+      const double Mf = Cn[MCG_A_MM];
+      Cn[MCG_A_MM] = *mprev * Mf;
+      *mprev = Mf;
+    }
+    __syncthreads();
+    flush_frame<NC>(C, B, row, B.meas);
   }
   __syncthreads();
   for (int t = lt; t < FSLOTS; t += blockDim.x) in[t] = 0.0;
@@ -3180,6 +3314,7 @@ struct RunCtx {
   int ncu = 0;
   int nslots = 0;  // split replicas (arrival counters)
   int max_export = 0;  // longest export list of a part
+  int blk = 0;  // LDS bytes per replica for a frame's block spins (0: looked up at every use)
   bool persist = false;  // persistent launches (barrier + tempering inside)
   int mode_begin[5] = {0, 0, 0, 0, 0};  // work items of link mode m: [mode_begin[m], mode_begin[m+1])
   size_t lds_max = 0;
@@ -3596,7 +3731,7 @@ size_t lds_bytes_for(const mcg_batch* B, const RunCtx& X, int i0, int i1) {
     const bool wide = G.lcid != nullptr || G.ncls > 256;
     const size_t b = lds_fixed_bytes(wide ? 0 : G.ncoup, wide ? 0 : G.ncls, G.ncol, G.npat, G.zmax, G.n, nwaves,
                                      w.nrep) +
-                     w.nrep * lds_replica_bytes(NC, G.n, sizeof(ST));
+                     w.nrep * (lds_replica_bytes(NC, G.n, sizeof(ST)) + (w.nparts > 1 ? 0 : (size_t)X.blk));
     mx = std::max(mx, b);
   }
   return mx;
@@ -3648,6 +3783,21 @@ int launch_lds(const mcg_batch* B, RunCtx& X, const SweepArgs& a, hipStream_t s,
     T.launches += 1;
   }
   return 0;
+}
+
+// Room for a frame's block spins in LDS (X.blk): taken when the workgroups
+// still fit, and as many of them per CU as without it.
+template <int NC, typename ST>
+void plan_block_spins(const mcg_batch* B, RunCtx& X) {
+  X.blk = 0;
+  if (!(B->meas & MCG_MEAS_RNORM) || X.hitems.empty()) return;
+  const int ni = (int)X.hitems.size();
+  const size_t pers = persist_lds_bytes(B->nrow, B->nrep);
+  const size_t without = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
+  for (const WorkItem& w : X.hitems)
+    X.blk = std::max(X.blk, (int)align16((size_t)B->graphs_host[w.graph].nr * NC * 4));
+  const size_t with = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
+  if (with > X.lds_max || (ni > X.ncu && X.lds_max / with != X.lds_max / without)) X.blk = 0;
 }
 
 // Can this run use a persistent launch?  All replicas on the LDS path, one
@@ -3885,6 +4035,7 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   X.lds_updates_per_sweep = 0;
   for (const WorkItem& w : X.hitems)
     if (w.part == 0) X.lds_updates_per_sweep += (double)w.nrep * B->graphs_host[w.graph].n;
+  plan_block_spins<NC, ST>(B, X);
   // persistent launches when possible (P->no_persist turns them off)
   X.persist = false;
   if (P->algorithm == MCG_METROPOLIS && !P->no_persist && !force_stream && check_persist<NC, ST>(B, P, X, &X.persist))
@@ -4104,6 +4255,7 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
     const bool rec_host = X.persist && X.nslots > 0 && B->recompute_every > 0;
     if (rec_host) ns = std::min<int64_t>(ns, B->recompute_every - (P->sweep0 + k) % B->recompute_every);
     SweepArgs a{k, P->sweep0, (int32_t)ns, (int32_t)nth, spf, P->frame0, X.sync, X.xpart, X.halo};
+    a.blk = X.blk;
     if (X.persist) {
       a.bar = X.bar;
       a.bar_base = (int32_t)bar_base;
