@@ -12,12 +12,12 @@
 //                     and part exchange inside the kernel.  HBM traffic per
 //                     sweep ~1 MB of bookkeeping; bound by VALU issue and the
 //                     per-sweep synchronisation.
-//   k_pass<NC,ST>     streaming colour pass over all replicas (spins in HBM /
+//   k_pass<NC,ST,..>  streaming colour pass over all replicas (spins in HBM /
 //                     L2), for lattices too large for LDS; also the "plain"
 //                     one-launch-per-replica-per-colour baseline.
 //   k_measure<NC,ST>  one workgroup per replica: FP64 full-Hamiltonian
 //                     recomputation and/or one measured frame.
-//   k_wolff<NC,ST>    one workgroup per replica: level-synchronous frontier
+//   k_wolff<NC,ST,..> one workgroup per replica: level-synchronous frontier
 //                     BFS Wolff clusters (embedded-spin for O(n)).
 //   k_pt              parallel-tempering swaps of temperature rows.
 //
@@ -3005,10 +3005,28 @@ __global__ void k_pt(mcg_batch B, const int32_t* __restrict__ ladder_row0, const
 }
 
 // ---------------------------------------------------------------------------
-// k_wolff: one 1024-thread block per replica, ncl clusters, frontier BFS in
-// global memory with one work item per (frontier site, link)
+// k_wolff: one 1024-thread block per replica, ncl clusters, level-synchronous
+// frontier BFS with one work item per (frontier site, link)
 // (heisenbergLib.c:310-439, xyLib.c:256-380, isingLib.c:165-236)
+//
+// A cluster is a chain of levels, each of which waits for its slowest item.
+// Everything an item needs but the neighbour's spin is therefore in LDS: the
+// frontier (site, pattern and projection, computed when the site was added),
+// the pattern rows, r.J.r per coupling, and the members as one bit per site
+// (BITS; graphs too large for that use stamps in global memory, as before).
+// An item then makes one round trip to L2, and the draw runs while it waits;
+// reading frontier entry, link word, stamp, both spins and exchanging the
+// stamp in global memory made five.  Cubic 64^3 at T_c, 16 replicas (clusters
+// of 6,000 spins on average): 447 -> 270 us a cluster; 8 ordered replicas of a
+// few thousand sites gain 1.5x, clusters of a few spins 1.2x to 1.3x.  What is
+// left is one CU's gathers (a cache line per lane) and draws per replica.
 // ---------------------------------------------------------------------------
+static constexpr int WOLFF_FRONT = 2048;  // frontier entries in LDS (a level's others are read from the member list)
+static constexpr int WOLFF_RJR = 256;     // couplings whose r.J.r is kept
+__host__ __device__ inline size_t wolff_lds_bytes(const mcg_graph& G, bool bits) {
+  return (size_t)2 * WOLFF_FRONT * 8 + WOLFF_RJR * 4 +
+         (pass_patterns(G) ? (size_t)G.npat * pat_stride(G.zmax) * 4 : 0) + (bits ? ((size_t)G.n + 127) / 128 * 16 : 0);
+}
 // accesses to a workgroup's private scratch in global memory (Wolff stamps
 // and cluster lists): ordered among the workgroup's threads only
 template <typename T>
@@ -3020,23 +3038,35 @@ __device__ __forceinline__ void wg_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <int NC, typename ST>
+template <int NC, typename ST, bool BITS>
 __global__ __launch_bounds__(1024) void k_wolff(mcg_batch B, const int32_t* __restrict__ rep_list, int64_t cl0,
                                                 int ncl) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint2* s_front = (uint2*)smem;  // [2][WOLFF_FRONT]: site | pattern << 24, projection (Ising: spin)
+  float* s_rjr = (float*)(s_front + 2 * WOLFF_FRONT);
+  int32_t* s_rows = (int32_t*)(s_rjr + WOLFF_RJR);
   const int rep = rep_list[blockIdx.x];
   const mcg_replica rp = B.reps[rep];
   const mcg_graph G = B.graphs[rp.graph];
-  const Spins<ST> sp{(ST*)B.spins + rp.spin_off, G.n};
+  const GSpins<ST> sp{gas((ST*)B.spins + rp.spin_off), G.n};
   uint32_t* stamp = B.wstamp + rp.site_off;
   int32_t* mem = B.wlist + rp.site_off;
   const int row = rp.row0 + B.rung[rep];
   const float beta = B.row_beta[row], h = B.row_h[row];
   const uint32_t key0 = B.seed_lo, key1 = B.seed_hi ^ rp.serial;
-  __shared__ int s_nc[3], s_seed;
-  __shared__ float s_r[3];
+  __shared__ int s_nc[3];
   __shared__ double s_red[16];
   __shared__ int s_acc;
   const int tid = threadIdx.x;
+  const bool pats = pass_patterns(G), wide = G.lcid != nullptr;
+  const int pstride = pat_stride(G.zmax);
+  uint32_t* s_bits = (uint32_t*)(s_rows + (pats ? G.npat * pstride : 0));
+  if (pats)
+    for (int t = tid; t < G.npat * (G.zmax + 1); t += blockDim.x) {
+      const int l = t % (G.zmax + 1);
+      const int32_t w = G.pattab[t];
+      s_rows[t / (G.zmax + 1) * pstride + l] = l == G.zmax ? w : row_word<false>(w, sizeof(ST));
+    }
   // isotropic exchange (every tensor c*I on the spin components) and no
   // single-ion term: with h = 0 the cluster's acceptance energy
   // (heisenbergLib.c:403-423) is zero in exact arithmetic, so the cluster is
@@ -3052,84 +3082,128 @@ __global__ __launch_bounds__(1024) void k_wolff(mcg_batch B, const int32_t* __re
       for (int k = 0; k < NC; ++k) iso_ok = iso_ok && G.clsdat[c * 8 + 1 + k] == 0.0f;
   }
   const bool skip_acc = __syncthreads_and(iso_ok ? 1 : 0) != 0 && h == 0.0f;
+  const uint32_t zl = (uint32_t)G.zmax, zmagic = zl > 0 ? 0xFFFFFFFFu / zl : 0u;
+  double grown = 0.0, flipped = 0.0;  // sites grown and flipped (first thread)
+  auto clear_bits = [&] {
+    if (BITS)
+      for (int w = tid; w < (G.n + 127) / 128; w += blockDim.x) ((uint4*)s_bits)[w] = make_uint4(0u, 0u, 0u, 0u);
+  };
+  clear_bits();
+  __syncthreads();
 
   for (int c = 0; c < ncl; ++c) {
     const uint64_t cl = (uint64_t)(cl0 + c);
     const uint32_t cur = (uint32_t)(cl & 0x7FFFFFFFu) * 2u + 1u;  // odd: never 0
+    // every thread draws the seed and the direction: no broadcast to wait for
+    const u32x4 x0 = philox4x32_10(u32x4{0u, (uint32_t)cl, (uint32_t)(cl >> 32), TAG_WOLFF}, key0, key1);
+    const int seed = (int)(((uint64_t)x0.x * (uint64_t)G.n) >> 32);
+    float r0 = 0.0f, r1 = 0.0f, r2 = 0.0f;
+    if constexpr (NC == 3) {
+      r2 = fmaf(u24(x0.y), 2.0f, -1.0f);
+      const float rho = unit_rho(r2);
+      float cc, sn;
+      sincos_turn(x0.z, &cc, &sn);
+      r0 = rho * cc;
+      r1 = rho * sn;
+    } else if constexpr (NC == 2) {
+      sincos_turn(x0.y, &r0, &r1);
+    }
+    auto rjr = [&](const float* J) {
+      return r0 * (J[0] * r0 + J[1] * r1 + J[2] * r2) + r1 * (J[3] * r0 + J[4] * r1 + J[5] * r2) +
+             r2 * (J[6] * r0 + J[7] * r1 + J[8] * r2);
+    };
+    // the projection of a site (Ising: its spin), as used by its links
+    auto project = [&](int i) {
+      float v[3];
+      spin_vec<NC>(sp, i, G.cls, G.clsdat, v);
+      return NC == 1 ? v[0] : -(v[0] * r0 + v[1] * r1 + v[2] * r2);
+    };
+    auto entry = [&](int i, float pj) {
+      return make_uint2((uint32_t)i | (pats ? (uint32_t)gas(G.pat)[i] << 24 : 0u), __float_as_uint(pj));
+    };
+    if (!wide)
+      for (int q = tid; q < G.ncoup; q += blockDim.x) s_rjr[q] = NC == 1 ? G.coup[q * 9] : rjr(G.coup + q * 9);
     if (tid == 0) {
-      const u32x4 x = philox4x32_10(u32x4{0u, (uint32_t)cl, (uint32_t)(cl >> 32), TAG_WOLFF}, key0, key1);
-      const int seed = (int)(((uint64_t)x.x * (uint64_t)G.n) >> 32);
-      float rx = 0, ry = 0, rz = 0;
-      if constexpr (NC == 3) {
-        rz = fmaf(u24(x.y), 2.0f, -1.0f);
-        const float rho = sqrtf(fmaxf(fmaf(-rz, rz, 1.0f), 0.0f));
-        float cc, sn;
-        sincos_turn(x.z, &cc, &sn);
-        rx = rho * cc;
-        ry = rho * sn;
-      } else if constexpr (NC == 2) {
-        sincos_turn(x.y, &rx, &ry);
-      }
-      s_r[0] = rx; s_r[1] = ry; s_r[2] = rz;
-      s_seed = seed;
-      wg_store(stamp + seed, cur);
+      const uint2 e0 = entry(seed, project(seed));
+      if (BITS)
+        s_bits[seed >> 5] = 1u << (seed & 31);
+      else
+        wg_store(stamp + seed, cur);
+      s_front[0] = e0;
       wg_store(mem, seed);
       s_nc[0] = s_nc[1] = s_nc[2] = 0;
-      // cluster accept draw: x.w
-      s_acc = (int)(x.w >> 8);
     }
     __syncthreads();
-    const float r0 = s_r[0], r1 = s_r[1], r2 = s_r[2];
     // Level-synchronous growth, one workgroup barrier per level: the sites
-    // level k adds go to mem[hi + s_nc[k % 3]++], so the frontier of level
-    // k+1 is [hi, hi + s_nc[k % 3]).  During level k the first thread clears
-    // the counter of level k+1, last read (level k-2's) before the barrier
-    // that ended level k-1.  One workgroup owns the cluster, so the stamps
-    // and the list need workgroup scope only: their accesses stay in the
-    // CU's caches.
+    // level k adds go to entry s_nc[k % 3]++ of the next frontier and to the
+    // member list behind it.  During level k the first thread clears the
+    // counter of level k+1, last read (level k-2's) before the barrier that
+    // ended level k-1.
     int lo = 0, hi = 1, cnt = 1;
     for (int k = 0;; ++k) {
-      // one work item per (frontier site, link): every item is one short
-      // dependent chain (stamp test, bond draw, stamp exchange)
-      const uint32_t zl = (uint32_t)G.zmax;
+      const uint2* front = s_front + (k & 1) * WOLFF_FRONT;
+      uint2* next = s_front + ((k + 1) & 1) * WOLFF_FRONT;
       const uint32_t nitem = (uint32_t)(hi - lo) * zl;
       for (uint32_t it = tid; it < nitem; it += blockDim.x) {
-        const uint32_t fq = it / zl;
+        uint32_t fq = __umulhi(it, zmagic);  // it / zl, or a little less
+        while (it - fq * zl >= zl) ++fq;
         const int l = (int)(it - fq * zl);
-        const int o = wg_load(mem + lo + (int)fq);
-        float so[3];
-        spin_vec<NC>(sp, o, G.cls, G.clsdat, so);
-        const float sdo = -(so[0] * r0 + so[1] * r1 + so[2] * r2);
-        {
-          const uint32_t wd = G.link[(size_t)o * G.zmax + l];
-          const int t = (int)(wd & 0xFFFFFFu);
-          if (t == o) continue;
-          if (wg_load(stamp + t) == cur) continue;
-          const uint32_t cw = G.lcid ? (uint32_t)G.lcid[(size_t)o * G.zmax + l] : (wd >> 24);
-          const float* J = G.coup + cw * 9;
+        uint2 e;
+        if (fq < (uint32_t)WOLFF_FRONT) {
+          e = front[fq];
+        } else {
+          const int o = wg_load(mem + lo + (int)fq);
+          e = entry(o, project(o));
+        }
+        const int o = (int)(e.x & 0xFFFFFFu);
+        const float pjo = __uint_as_float(e.y);
+        int t;
+        uint32_t cw;
+        if (pats) {
+          const int32_t wd = s_rows[(e.x >> 24) * pstride + l];
+          t = o + (wd >> 8);
+          cw = (uint32_t)wd & 0xFFu;
+        } else {
+          const uint32_t wd = gas(G.link)[(size_t)o * G.zmax + l];
+          t = (int)(wd & 0xFFFFFFu);
+          cw = wide ? (uint32_t)gas(G.lcid)[(size_t)o * G.zmax + l] : (wd >> 24);
+        }
+        bool add = false;
+        uint2 en = make_uint2(0u, 0u);
+        const bool member = t == o || (BITS ? (s_bits[t >> 5] >> (t & 31) & 1u) != 0u : wg_load(stamp + t) == cur);
+        if (!member) {
+          const float pjt = project(t);
+          en = entry(t, pjt);
+          const float rj = !wide ? s_rjr[cw] : NC == 1 ? G.coup[cw * 9] : rjr(G.coup + cw * 9);
+          const u32x4 x = philox4x32_10(
+              u32x4{(uint32_t)(o * G.zmax + l), (uint32_t)cl, (uint32_t)(cl >> 32), TAG_BOND}, key0, key1);
           float corr;
           if constexpr (NC == 1) {
-            corr = (J[0] * sp.get(t, 0)) * so[0] * beta;  // J*S_t*sigma_t * s_o
-            corr = 2.0f * corr;                            // add if J s s < 0, p = 1-exp(2 corr)
+            corr = (rj * sp.get(t, 0)) * pjo * beta;  // J*S_t*sigma_t * s_o
+            corr = 2.0f * corr;                        // add if J s s < 0, p = 1-exp(2 corr)
           } else {
-            float st3[3];
-            spin_vec<NC>(sp, t, G.cls, G.clsdat, st3);
-            const float sdt = -(st3[0] * r0 + st3[1] * r1 + st3[2] * r2);
-            const float rJr = r0 * (J[0] * r0 + J[1] * r1 + J[2] * r2) + r1 * (J[3] * r0 + J[4] * r1 + J[5] * r2) +
-                              r2 * (J[6] * r0 + J[7] * r1 + J[8] * r2);
-            corr = 2.0f * sdo * sdt * rJr * beta;
+            corr = 2.0f * pjo * pjt * rj * beta;
           }
-          if (corr < 0.0f) {
-            const u32x4 x = philox4x32_10(
-                u32x4{(uint32_t)(o * G.zmax + l), (uint32_t)cl, (uint32_t)(cl >> 32), TAG_BOND}, key0, key1);
-            if (1.0f - exp_neg(corr) > u24(x.x)) {
-              const uint32_t old = __hip_atomic_exchange(stamp + t, cur, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
-              if (old != cur) {
-                const int pos = hi + atomicAdd(&s_nc[k % 3], 1);
-                wg_store(mem + pos, t);
-              }
+          if (corr < 0.0f && 1.0f - exp_neg(corr) > u24(x.x)) {
+            if (BITS) {
+              const uint32_t bit = 1u << (t & 31);
+              add = (atomicOr(s_bits + (t >> 5), bit) & bit) == 0u;
+            } else {
+              add = __hip_atomic_exchange(stamp + t, cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != cur;
             }
+          }
+        }
+        // one counter update per wave for its new members
+        const uint64_t who = __ballot(add);
+        if (who) {
+          int base = 0;
+          const int first = __ffsll((unsigned long long)who) - 1, lane = tid & 63;
+          if (lane == first) base = atomicAdd(&s_nc[k % 3], __popcll(who));
+          base = __builtin_amdgcn_readlane(base, first);
+          if (add) {
+            const int pos = base + __popcll(who & ((1ull << lane) - 1ull));
+            if (pos < WOLFF_FRONT) next[pos] = en;
+            wg_store(mem + hi + pos, t);
           }
         }
       }
@@ -3175,7 +3249,7 @@ __global__ __launch_bounds__(1024) void k_wolff(mcg_batch B, const int32_t* __re
                                    r1 * (J[3] * pt[0] + J[4] * pt[1] + J[5] * pt[2]) +
                                    r2 * (J[6] * pt[0] + J[7] * pt[1] + J[8] * pt[2]));
           d += (double)src;
-          if (wg_load(stamp + t) == cur)
+          if (BITS ? (s_bits[t >> 5] >> (t & 31) & 1u) != 0u : wg_load(stamp + t) == cur)
             d += (double)(sdt * (pb[0] * (J[0] * r0 + J[1] * r1 + J[2] * r2) +
                                  pb[1] * (J[3] * r0 + J[4] * r1 + J[5] * r2) +
                                  pb[2] * (J[6] * r0 + J[7] * r1 + J[8] * r2)));
@@ -3196,22 +3270,25 @@ __global__ __launch_bounds__(1024) void k_wolff(mcg_batch B, const int32_t* __re
         }
       }
     }
-    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
-    if ((tid & 63) == 0) s_red[tid >> 6] = d;
-    __syncthreads();
-    if (tid == 0) {
-      double t = 0.0;
-      for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
-      const float db = (float)(t * (double)beta);
-      const float u = (float)s_acc * 0x1p-24f;
-      s_acc = (db <= 0.0f || u < exp_neg(-db)) ? 1 : 0;
-      // cluster statistics: sites flipped and sites grown
-      double* st = B.state + (size_t)rep * MCG_NSTATE;
-      if (s_acc) st[MCG_S_ACC] += (double)cnt;
-      st[MCG_S_TRY] += (double)cnt;
+    bool flip = true;
+    if (!skip_acc) {
+      for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+      if ((tid & 63) == 0) s_red[tid >> 6] = d;
+      __syncthreads();
+      if (tid == 0) {
+        double t = 0.0;
+        for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
+        const float db = (float)(t * (double)beta);
+        s_acc = (db <= 0.0f || u24(x0.w) < exp_neg(-db)) ? 1 : 0;  // x0.w: the cluster's acceptance draw
+      }
+      __syncthreads();
+      flip = s_acc != 0;
     }
-    __syncthreads();
-    if (s_acc) {
+    clear_bits();  // for the next cluster
+    // cluster statistics: sites flipped and sites grown
+    if (flip) flipped += (double)cnt;
+    grown += (double)cnt;
+    if (flip) {
       for (int f = tid; f < cnt; f += blockDim.x) {
         const int b = wg_load(mem + f);
         if constexpr (NC == 1) {
@@ -3230,6 +3307,11 @@ __global__ __launch_bounds__(1024) void k_wolff(mcg_batch B, const int32_t* __re
       }
     }
     __syncthreads();
+  }
+  if (tid == 0) {
+    double* st = B.state + (size_t)rep * MCG_NSTATE;
+    st[MCG_S_ACC] += flipped;
+    st[MCG_S_TRY] += grown;
   }
 }
 
@@ -4215,12 +4297,30 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
       wmax = std::max<int64_t>(wmax, (int64_t)B->graphs_host[gi].n * (B->graphs_host[gi].zmax + 1));
     }
     if (wmax >= ((int64_t)1 << 32)) return fail("Wolff: sites x (links + 1) must stay below 2^32");
+    // members as bits in LDS where every graph's fit
+    bool bits = true;
+    size_t wolff_lds = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+      wolff_lds = 0;
+      for (int gi = 0; gi < B->ngraph; ++gi) wolff_lds = std::max(wolff_lds, wolff_lds_bytes(B->graphs_host[gi], bits));
+      if (wolff_lds + 1024 <= X.lds_max) break;  // 1024: the kernel's other LDS
+      bits = false;
+    }
+    (void)hipFuncSetAttribute(bits ? (const void*)k_wolff<NC, ST, true> : (const void*)k_wolff<NC, ST, false>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)wolff_lds);
+    (void)hipGetLastError();
     for (int64_t k = 0; k < total; ++k) {
       const int64_t kk = P->sweep0 + k;
       // clusters per sweep: plan value or n of the replica's graph (use max n)
       const int ncl = P->clusters_per_sweep > 0 ? P->clusters_per_sweep : (int)nmax;
-      hipLaunchKernelGGL((k_wolff<NC, ST>), dim3((unsigned)nall), dim3(1024), 0, s, *B, X.all_reps,
-                         kk * (int64_t)ncl, ncl);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nall), dim3(1024), (uint32_t)wolff_lds, s, *B, X.all_reps,
+                           kk * (int64_t)ncl, ncl);
+      };
+      if (bits)
+        launch(k_wolff<NC, ST, true>);
+      else
+        launch(k_wolff<NC, ST, false>);
       HIPCHK(hipGetLastError());
       const bool meas = k >= nth && ((k - nth + 1) % spf) == 0;
       const bool therm_end = (k + 1 == nth);
