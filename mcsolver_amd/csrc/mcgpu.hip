@@ -8,10 +8,9 @@
 //                     workgroups), stages their spins in LDS once, runs many
 //                     graph-coloured Metropolis sweeps with in-kernel fused
 //                     measurement, writes spins back once.  PERSIST: every
-//                     workgroup resident, a grid barrier per sweep, tempering
-//                     and part exchange inside the kernel.  HBM traffic per
-//                     sweep ~1 MB of bookkeeping; bound by VALU issue and the
-//                     per-sweep synchronisation.
+//                     workgroup resident; tempering and part exchange inside
+//                     the kernel.  HBM traffic per sweep ~1 MB of bookkeeping;
+//                     bound by VALU issue and the per-sweep exchanges.
 //   k_pass<NC,ST,..>  streaming colour pass over all replicas (spins in HBM /
 //                     L2), for lattices too large for LDS; also the "plain"
 //                     one-launch-per-replica-per-colour baseline.
@@ -150,6 +149,9 @@ static constexpr double REF_PI = 3.1415926535;  // heisenbergLib.c:6
 // a value that is the same in every active lane, as a scalar
 __device__ __forceinline__ int wave_uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ float wave_uniform(float x) { return __int_as_float(wave_uniform(__float_as_int(x))); }
+__device__ __forceinline__ double wave_uniform(double x) {
+  return __hiloint2double(wave_uniform(__double2hiint(x)), wave_uniform(__double2loint(x)));
+}
 // a wave-uniform value kept in a vector register: FP32 adds, products and
 // FMAs whose operands are all vector registers issue at 2.8-3.2 cycles per
 // SIMD on gfx950, those with a scalar operand at 4.4 (measured, 4 waves)
@@ -739,6 +741,15 @@ __device__ __forceinline__ double wave_sum_f64(double x) {
   return x;
 }
 
+// The thread's index, read anew: the reductions and frames sit inside the
+// sweep loop, and what the compiler derives from the plain index (addresses,
+// masks) it computes before the loop and keeps, spilled, across the sweeps.
+__device__ __forceinline__ int tid() {
+  int x = (int)threadIdx.x;
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // x summed over lanes l and l ^ 16, or l and l ^ 32
 __device__ __forceinline__ double add_lane16(double x) {
   const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(x), (uint32_t)__double2loint(x), false, false);
@@ -757,7 +768,8 @@ __device__ __forceinline__ double add_lane32(double x) {
 // FP64 additions a lane instead of 24.
 template <int N>
 __device__ __forceinline__ void wave_totals(const double* v, double* r) {
-  const bool b0 = (threadIdx.x & 1) != 0, b1 = (threadIdx.x & 2) != 0;
+  const int tx = tid();
+  const bool b0 = (tx & 1) != 0, b1 = (tx & 2) != 0;
 #pragma unroll
   for (int j = 0; 4 * j < N; ++j) {
     const double a = v[4 * j], b = 4 * j + 1 < N ? v[4 * j + 1] : 0.0;
@@ -795,7 +807,7 @@ __device__ __forceinline__ void group_add(const double* v, double* s_red, int g,
   constexpr int M = (N + 3) / 4;
   double r[M];
   wave_totals<N>(v, r);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tx = tid(), lane = tx & 63, wave = tx >> 6;
   const int nw = TPR >> 6;
   if (nw == 1) {  // the same for every group of the workgroup
 #pragma unroll
@@ -845,9 +857,10 @@ struct FrameCtx {
 };
 template <int NC>
 __device__ __forceinline__ void frame_consts(FrameCtx& C, const mcg_graph& G, const mcg_batch& B) {
-  C.inv_n = 1.0 / (double)G.n;
-  C.inv_nlat = 1.0 / (double)(G.nlat > 0 ? G.nlat : G.n);
-  C.inv_nf = 1.0 / (double)(B.nframes > 0 ? B.nframes : 1);
+  // (scalars: they live across the sweeps)
+  C.inv_n = wave_uniform(1.0 / (double)G.n);
+  C.inv_nlat = wave_uniform(1.0 / (double)(G.nlat > 0 ? G.nlat : G.n));
+  C.inv_nf = wave_uniform(1.0 / (double)(B.nframes > 0 ? B.nframes : 1));
   C.last = G.pos[G.n - 1];
   C.blk = nullptr;
 }
@@ -1009,7 +1022,7 @@ __device__ __forceinline__ double frame_mprev(const mcg_batch& B, int row) {
 // thread per replica; Cn is zero before (zero_terms).
 static constexpr int NTERMS = MCG_NACC + MCG_NBINQ + 1;
 __device__ __forceinline__ void zero_terms(double* s_frm, int R) {  // by one wave, for R groups
-  const int lane = threadIdx.x & 63;
+  const int lane = tid() & 63;
   for (int r = 0; r < R; ++r)
     if (lane < NTERMS) s_frm[r * FRM + FRM_ACC + lane] = 0.0;
   wave_lds_fence();
@@ -1020,27 +1033,36 @@ __device__ __forceinline__ void frame_terms(const FrameCtx& C, const mcg_graph& 
   const int ngq = frame_groups<NC>(G, flags);
   const double inv_nLat = C.inv_nlat;
   const bool pairs = (flags & MCG_MEAS_PAIRS) && G.nlat > 0;
+  const bool charge = (flags & MCG_MEAS_Q) && NC == 3 && G.ncirc > 0;
+  const bool blocks = (flags & MCG_MEAS_RNORM) && G.nr > 0;
+  // everything is read before the first term is stored: reads and stores of
+  // the same memory stay in order, and one lane would wait for each in turn
   double E = st[MCG_S_E];
-  if (flags & MCG_ISING_RELE) E -= st[MCG_S_EREF];
-  const double e = E * C.inv_n;
+  const double Eref = st[MCG_S_EREF];
   const double M0 = st[MCG_S_M], M1 = st[MCG_S_M + 1], M2 = st[MCG_S_M + 2];
+  double P[8];  // the pairs' sums
+#pragma unroll
+  for (int k = 0; k < 8; ++k) P[k] = pairs ? F[k] : 0.0;
+  const double q8 = charge ? F[8] : 0.0;
+  if (flags & MCG_ISING_RELE) E -= Eref;
+  const double e = E * C.inv_n;
   if (pairs && G.self_pairs) {
     // pairs (i, i) over every site: sum s_i is the tracked magnetisation,
     // sum s_i.s_i the sum of the squared spin lengths
-    F[0] = F[3] = M0;
-    F[1] = F[4] = M1;
-    F[2] = F[5] = M2;
-    F[6] = G.pair_s2;
+    P[0] = P[3] = M0;
+    P[1] = P[4] = M1;
+    P[2] = P[5] = M2;
+    P[6] = G.pair_s2;
   }
   double Mf;
-  const int ax = NC == 3 ? 2 : 0;
+  constexpr int ax = NC == 3 ? 2 : 0;
   if constexpr (NC == 1) {
-    Mf = (pairs ? F[0] : M0) * inv_nLat;
+    Mf = (pairs ? P[0] : M0) * inv_nLat;
     if (pairs) {
-      Cn[MCG_A_SI] = fabs(F[0]) * inv_nLat;
-      Cn[MCG_A_SJ] = fabs(F[3]) * inv_nLat;
-      Cn[MCG_A_SIJ] = F[6] * inv_nLat;
-      Cn[MCG_A_LAST] = F[7];
+      Cn[MCG_A_SI] = fabs(P[0]) * inv_nLat;
+      Cn[MCG_A_SJ] = fabs(P[3]) * inv_nLat;
+      Cn[MCG_A_SIJ] = P[6] * inv_nLat;
+      Cn[MCG_A_LAST] = P[7];
     }
     Cn[MCG_A_TOT] = M0;
   } else {
@@ -1048,39 +1070,45 @@ __device__ __forceinline__ void frame_terms(const FrameCtx& C, const mcg_graph& 
     double dir[3] = {Mv[0], Mv[1], Mv[2]};
     const double ml = sqrt(dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2]);
     if (ml >= 1e-5) {
-      dir[0] /= ml; dir[1] /= ml;
-      if constexpr (NC == 3) dir[2] /= ml;  // XY: 0 / ml = 0
+      const double il = 1.0 / ml;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) dir[k] *= il;
     }
     if (NC == 3 || !pairs)
       Mf = ml * inv_nLat;
     else
-      Mf = sqrt(F[0] * F[0] + F[1] * F[1]) * inv_nLat;
+      Mf = sqrt(P[0] * P[0] + P[1] * P[1]) * inv_nLat;
     if (pairs) {
+#pragma unroll
       for (int k = 0; k < NC; ++k) {
-        Cn[MCG_A_SI + k] = fabs(F[k] * inv_nLat);
-        Cn[MCG_A_SJ + k] = fabs(F[3 + k] * inv_nLat);
+        Cn[MCG_A_SI + k] = fabs(P[k] * inv_nLat);
+        Cn[MCG_A_SJ + k] = fabs(P[3 + k] * inv_nLat);
       }
-      Cn[MCG_A_SIJ] = F[6] * inv_nLat;
-      Cn[MCG_A_ZI] = (dir[0] * F[0] + dir[1] * F[1] + dir[2] * F[2]) * inv_nLat;
-      Cn[MCG_A_ZJ] = (dir[0] * F[3] + dir[1] * F[4] + dir[2] * F[5]) * inv_nLat;
-      Cn[MCG_A_HI] = F[ax] * inv_nLat;
-      Cn[MCG_A_HJ] = F[3 + ax] * inv_nLat;
+      Cn[MCG_A_SIJ] = P[6] * inv_nLat;
+      Cn[MCG_A_ZI] = (dir[0] * P[0] + dir[1] * P[1] + dir[2] * P[2]) * inv_nLat;
+      Cn[MCG_A_ZJ] = (dir[0] * P[3] + dir[1] * P[4] + dir[2] * P[5]) * inv_nLat;
+      Cn[MCG_A_HI] = P[ax] * inv_nLat;
+      Cn[MCG_A_HJ] = P[3 + ax] * inv_nLat;
     }
     Cn[MCG_A_ZT] = (dir[0] * Mv[0] + dir[1] * Mv[1] + dir[2] * Mv[2]) * inv_nLat;
     Cn[MCG_A_HT] = Mv[ax] * inv_nLat;
-    if ((flags & MCG_MEAS_Q) && NC == 3 && G.ncirc > 0) Cn[MCG_A_Q] = F[8] / REF_PI / 4;
-    if ((flags & MCG_MEAS_RNORM) && G.nr > 0) {
+    if (charge) Cn[MCG_A_Q] = q8 / REF_PI / 4;
+    if (blocks) {
+      double R[11];
+#pragma unroll
+      for (int k = 0; k < 11; ++k) R[k] = F[16 + k];
+#pragma unroll
       for (int k = 0; k < NC; ++k) {
-        Cn[MCG_A_SIR + k] = fabs(F[16 + k] / F[24]);
-        Cn[MCG_A_SJR + k] = fabs(F[19 + k] / F[25]);
+        Cn[MCG_A_SIR + k] = fabs(R[k] / R[8]);
+        Cn[MCG_A_SJR + k] = fabs(R[3 + k] / R[9]);
       }
-      Cn[MCG_A_SIJR] = F[22] / F[26];
+      Cn[MCG_A_SIJR] = R[6] / R[10];
     }
     // groups: the total (all sites / nLat) is group ng
     if (ngq > 0)
       for (int k = 0; k < 3; ++k) F[32 + 3 * ngq + k] = Mv[k] * inv_nLat;
   }
-  if ((flags & MCG_MEAS_RNORM) && G.nr > 0) {
+  if (blocks) {
     const double er = (F[27] / 2 + F[28]) / G.nr;
     Cn[MCG_A_ER] = er;
     Cn[MCG_A_ER2] = er * er;
@@ -1325,7 +1353,7 @@ __device__ __forceinline__ void first_wave_terms(const SV& sp, const FrameCtx& C
   double* F = C.s_frm;
   double* Cn = F + FRM_ACC;
   zero_terms(F, 1);
-  if ((threadIdx.x & 63) == 0) {
+  if ((tid() & 63) == 0) {
     const mcg_graph G = fresh(C.G);
     if (NC == 1 && (flags & MCG_MEAS_PAIRS) && G.self_pairs) {
       float t[3];
@@ -1420,7 +1448,7 @@ struct WorkItem {
 // that staging starts one dependent load after the work item
 struct ItemRep {
   int64_t spin_off;
-  int32_t rep, serial, row0, pad;
+  int32_t rep, serial, row0, nrung, ladder, pad;  // nrung 0: no tempering ladder
 };
 
 static constexpr int MAX_PARTS = 4;
@@ -1439,21 +1467,16 @@ struct SweepArgs {
   double* xpart;        // split replicas: per-part (dE, dM) partial sums
   const int32_t* halo;  // split replicas: extra-group tables
   // persistent launches (many sweeps, tempering inside the kernel)
-  uint32_t* bar;             // grid barrier counter, zero at run start
-  int32_t bar_base;          // barriers passed before this launch
+  int32_t sync_base;         // exchanges (of parts or ladders) before this launch in the run
   int32_t pt_every;          // tempering period in sweeps (0: none)
   int32_t has_split;         // the launch holds split replicas
-  int32_t nladder;
-  const int32_t* lad_row0;
-  const int32_t* lad_n;
-  const int32_t* blk_lad;    // per workgroup: [nblocks+1] offsets, then ladder
-                             // indices (bit 31: the workgroup owns the ladder)
-  const uint8_t* rep_np;     // parts of each replica (1: whole)
-  double* eslot;             // [2][nrep][MAX_PARTS] published energies
-  double* mslot;             // [2][nrep][MAX_PARTS][3] published magnetisation changes
+  int32_t nrow_parts;        // parts a row has words for in rowslot: the most of any replica
+  uint64_t* rowslot;         // [4][nrow][nrow_parts][2] energies published for tempering (tagged words)
+  uint64_t* pslot;           // [2][nslots][MAX_PARTS][2] energies of a split replica's parts (tagged words)
+  double* mslot;             // [2][nslots][MAX_PARTS-1][3] published magnetisation changes of parts 1, ...
   void* xbuf;                // [2][nslots][MAX_PARTS][max_export][NC] exported sites
-  double* mprev3;            // [3][nrow] M' of each row's last frames (frame f in slot f % 3)
-  double* fpart;             // [nslots][MAX_PARTS][FSUMS] split replicas' partial frame sums
+  uint64_t* mprev;           // [2][nrow][2] M' of each row's last frames (tagged words, by the tag's parity)
+  double* fpart;             // [2][nslots][MAX_PARTS-1][FSUMS] split replicas' partial frame sums
                              // (spin-derived observables); their arrival count is sync[slot]
   void* fspin;               // [2][nslots][NC][fspin_n] split replicas' sites as published for a
                              // frame, by sweep parity: the next sweep's publication must not
@@ -1475,20 +1498,16 @@ __host__ __device__ inline bool recompute_due(const mcg_batch& B, int64_t global
 }
 
 // LDS of the tempering state a persistent launch keeps in every workgroup:
-// who and accepted-swap counts per row, rung per replica, beta and h per row
-// (and the workgroup's ladder list: at most one ladder per replica, so at
-// most MAX_LADW entries of (ladder | owner bit, first row, rungs))
-static constexpr int MAX_LADW = 16;
-__host__ __device__ inline size_t persist_lds_bytes(int nrow, int nrep) {
-  return align16((size_t)(2 * nrow + nrep) * 4) + align16((size_t)2 * nrow * 4) + align16((size_t)MAX_LADW * 3 * 4) +
-         align16((size_t)nrep);
+// beta and h per row; per group its row, and its ladder's first row and rungs;
+// the flag of a wait that timed out
+static constexpr int MAX_GROUPS = 16;  // replicas per workgroup (1024 threads, a wave each)
+__host__ __device__ inline size_t persist_lds_bytes(int nrow) {
+  return align16((size_t)2 * nrow * 4) + (size_t)MAX_GROUPS * 12 + 16;
 }
 
-
-
+typedef unsigned int v4u32 __attribute__((ext_vector_type(4)));
 // copy one replica between HBM (16-byte aligned) and LDS in 16-byte vectors,
 // four in flight per thread
-typedef unsigned int v4u32 __attribute__((ext_vector_type(4)));
 
 template <typename ST, bool IN>
 __device__ __forceinline__ void stage(ST* lds, ST* g, int count, int lt, int TPR) {
@@ -1563,53 +1582,56 @@ __device__ __forceinline__ void stores_done() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// Grid-wide barrier of a persistent launch (every workgroup resident), in
-// two levels, because arrivals on one counter serialise at its memory
-// channel (256 workgroups on one counter: ~3.9 us per barrier on MI355X;
-// 16 counters of 16 plus a top counter: ~1.6 us).  Workgroup b counts in
-// on group counter b % BAR_GROUPS; the group's last arrival counts in on the
-// top counter; the last of those writes the barrier's epoch (its index,
-// from 1) to every group's release word, which the group's workgroups poll.
-// All words sit in their own 128-byte lines.  Bounded: on time-out bit 16
-// of the error flag is raised and false returned, and the caller leaves the
-// kernel.
-static constexpr int BAR_GROUPS = 16;
-static constexpr int BAR_LINE = 32;  // uint32 per line
-static constexpr int BAR_WORDS = (1 + 2 * BAR_GROUPS) * BAR_LINE;
-// (grid_arrive then grid_wait: work placed between them overlaps the wait)
-__device__ __forceinline__ void grid_arrive(uint32_t* bar, uint32_t epoch) {
-  stores_done();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int nb = (int)gridDim.x;
-    const int grp = (int)blockIdx.x % BAR_GROUPS;
-    const int ngrp = nb < BAR_GROUPS ? nb : BAR_GROUPS;
-    const uint32_t gsz = (uint32_t)((nb - grp + BAR_GROUPS - 1) / BAR_GROUPS);
-    uint32_t* gc = bar + (1 + grp) * BAR_LINE;
-    const uint32_t old = __hip_atomic_fetch_add(gc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old + 1 == epoch * gsz) {
-      const uint32_t o2 = __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (o2 + 1 == epoch * (uint32_t)ngrp)
-        for (int q = 0; q < ngrp; ++q) dev_store(bar + (1 + BAR_GROUPS + q) * BAR_LINE, epoch);
-    }
-  }
+// A published FP64 value: two words, each with half of its bits and the tag
+// of the event it belongs to, in device-coherent stores.  A reader that sees
+// its tag in both words has the value: the store needs no acknowledgement, no
+// counter and no release word, and the reader no second trip for the data.
+// Tags only grow during a run, and every run starts with zeroed words.
+__device__ __forceinline__ void tag_store(uint64_t* w, uint32_t tag, double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x), t = (uint64_t)tag << 32;
+  dev_store(w, t | (u & 0xFFFFFFFFu));
+  dev_store(w + 1, t | (u >> 32));
 }
-__device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t epoch, int32_t* err, int* s_flag) {
-  if (threadIdx.x == 0) {
-    uint32_t* rel = bar + (1 + BAR_GROUPS + (int)blockIdx.x % BAR_GROUPS) * BAR_LINE;
-    int ok = 1;
-    uint32_t it = 0;
-    while ((int32_t)(dev_load(rel) - epoch) < 0) {
-      if (++it > (1u << 22)) {
-        atomicOr(err, MCG_ERR_BARRIER);
-        ok = 0;
-        break;
-      }
-    }
-    *s_flag = ok;
+struct Tagged {
+  uint64_t a = 0, b = 0;
+  // both words in one 16-byte load (with the wait: its registers are not free
+  // before), half the requests of two loads
+  __device__ __forceinline__ void load(const uint64_t* w) {
+    v4u32 u;
+    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(u) : "v"(w) : "memory");
+    a = (uint64_t)u.y << 32 | u.x;
+    b = (uint64_t)u.w << 32 | u.z;
   }
-  __syncthreads();
-  return *s_flag != 0;
+  __device__ __forceinline__ void load_ahead(const uint64_t* w) {  // not waited for here
+    a = dev_load(w);
+    b = dev_load(w + 1);
+  }
+  // the tag, but for the bits in `any`
+  __device__ __forceinline__ bool has(uint32_t tag, uint32_t any = 0u) const {
+    return ((((uint32_t)(a >> 32) ^ tag) | ((uint32_t)(b >> 32) ^ tag)) & ~any) == 0u;
+  }
+  __device__ __forceinline__ double value() const {
+    return __hiloint2double((int)(uint32_t)b, (int)(uint32_t)a);
+  }
+};
+// Waits are bounded: on time-out bit 16 of the error flag is raised and the
+// workgroup's flag cleared, and the workgroup leaves the kernel.
+static constexpr uint32_t WAIT_POLLS = 1u << 22;
+__device__ __forceinline__ void wait_failed(int32_t* err, int* s_flag) {
+  atomicOr(err, MCG_ERR_BARRIER);
+  *s_flag = 0;
+}
+// the value of tag `tag` at w (t: words read ahead)
+__device__ __forceinline__ double tag_wait(const uint64_t* w, Tagged t, uint32_t tag, int32_t* err, int* s_flag) {
+  uint32_t it = 0;
+  while (!t.has(tag)) {
+    t.load(w);
+    if (++it > WAIT_POLLS) {
+      wait_failed(err, s_flag);
+      break;
+    }
+  }
+  return t.value();
 }
 
 template <int S>
@@ -1655,7 +1677,7 @@ __device__ __forceinline__ void part_copy(ST* lds_s, ST* gsp, int n, int nc, con
 // the sites of part p (every colour) from LDS (component stride n) to a
 // copy of the replica in global memory (component stride dn) with
 // device-scope stores, so that any workgroup of the launch can read them
-// (DevSpins) after the next grid barrier.  The copy is not the replica's
+// (DevSpins) after the parts' next exchange.  The copy is not the replica's
 // spin array: other parts still stage from that at the launch start.
 template <typename ST>
 __device__ __forceinline__ void part_publish(const ST* lds_s, typename RawBits<sizeof(ST)>::T* dst, int n, int dn, int nc,
@@ -1775,13 +1797,6 @@ __device__ __forceinline__ void lds_sweep_tail(const SV& sv, const mcg_graph& G,
   __syncthreads();
 }
 
-// FP64 value of lane src (any lane) in every lane
-__device__ __forceinline__ double bperm_f64(double x, int src) {
-  const int lo = __builtin_amdgcn_ds_bpermute(src << 2, __double2loint(x));
-  const int hi = __builtin_amdgcn_ds_bpermute(src << 2, __double2hiint(x));
-  return __hiloint2double(hi, lo);
-}
-
 // One exported site of a split replica: its NC components (raw bits, SoA in
 // LDS) as one device-scope store when they fill 4 or 8 bytes, else one per
 // component.
@@ -1805,8 +1820,8 @@ __device__ __forceinline__ void export_site(U* dst, const U* lraw, int n, int si
 // 0..np-1 (its own list has no entries here), so that it imports about
 // (sites of all lists) / TPR sites in all instead of working through every
 // part's list in turn, one device-scope round trip per list.  K sites are
-// loaded before any is stored (K = 1 measured faster than 4 on the
-// honeycomb set).  xs: part 0's export area of this replica and sweep
+// loaded before any is stored (honeycomb 64^2 x 64, 50 sweeps: one 916 us,
+// two 906).  xs: part 0's export area of this replica and sweep
 // parity; parts are max_export * NC words apart.  dsc: this part's
 // descriptor; part p's is (p - part) * ds ints away.
 template <int NC, typename U>
@@ -1815,7 +1830,7 @@ __device__ __forceinline__ void import_parts(const U* xs, int max_export, const 
   constexpr int W = NC * (int)sizeof(U);
   constexpr bool PACKED = W == 8 || W == 4;
   typedef typename std::conditional<W == 8, uint64_t, uint32_t>::type P;
-  constexpr int K = 1;
+  constexpr int K = 2;
   int ofs[MAX_PARTS], lst[MAX_PARTS], tot = 0;
 #pragma unroll
   for (int p = 0; p < MAX_PARTS; ++p) {
@@ -1865,68 +1880,46 @@ __device__ __forceinline__ void import_parts(const U* xs, int max_export, const 
   }
 }
 
-// Frame f of the replica of lane g (persistent launches): its terms are
-// staged for flush_frame; mp is the row's previous M', slot (f-1) % 3 of
-// a.mprev3 (frame_mprev3), and the frame's own M goes to slot f % 3.
-template <int NC>
-__device__ __forceinline__ double frame_mprev3(const SweepArgs& a, int64_t f, int row, int nrow) {
-  return dev_load(a.mprev3 + (size_t)((f + 2) % 3) * nrow + row);
-}
-template <int NC>
-__device__ __forceinline__ void take_frame(const FrameCtx& C, const mcg_batch& B, const SweepArgs& a, double* s_st,
-                                           double* s_frm, int lane, int64_t f, int row, int nrow, double mp,
-                                           int flags) {
-  double* F = s_frm + lane * FRM;
-  double* Cn = F + FRM_ACC;
-  frame_terms<NC>(C, fresh(C.G), B, s_st + lane * MCG_NSTATE, F, flags, f, Cn);
-  const double Mf = Cn[MCG_A_MM];
-  Cn[MCG_A_MM] = mp * Mf;
-  dev_store(a.mprev3 + (size_t)(f % 3) * nrow + row, Mf);
-}
-
 // Split replica, measured frame with spin-derived observables: each part's
 // share F[0, FSUMS) of the sums (frame_sums) goes to a.fpart and counts in
 // on the replica's counter a.sync[slot]; part 0 waits for the other parts of
 // this frame (the counter counts from the run's first frame, a.frame0), then
 // adds their sums to its own in part order, so the result does not depend on
-// arrival order.  Bounded like the grid barrier.  Called by every thread of
-// the part's workgroup; false: time-out (the caller leaves the kernel).
-// A part overwrites its slot only after the next grid barrier, which part 0
-// passes after reading it.
+// arrival order.  Called by every thread of the part's workgroup; false:
+// time-out (the caller leaves the kernel).  A part overwrites its slot only
+// after the parts' next exchange, which part 0 joins after reading it.
 __device__ __forceinline__ bool gather_frame_sums(const SweepArgs& a, const mcg_batch& B, double* F, int slot, int part, int np,
                                   int64_t frame, int* s_flag) {
-  double* fp = a.fpart + (size_t)slot * MAX_PARTS * FSUMS;
+  double* fp = a.fpart + (size_t)slot * (MAX_PARTS - 1) * FSUMS;  // part p at p - 1
   uint32_t* cnt = a.sync + (size_t)slot * SYNC_STRIDE;
+  const int tx = tid();
   __syncthreads();  // F is written by the first thread
   if (part != 0) {
-    if (threadIdx.x < 64)
-      for (int q = threadIdx.x; q < FSUMS; q += 64) dev_store(fp + (size_t)part * FSUMS + q, F[q]);
+    if (tx < 64)
+      for (int q = tx; q < FSUMS; q += 64) dev_store(fp + (size_t)(part - 1) * FSUMS + q, F[q]);
     stores_done();
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tx == 0) __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
   }
-  if (threadIdx.x == 0) {
+  if (tx == 0) {
     const uint32_t want = (uint32_t)((frame - a.frame0 + 1) * (int64_t)(np - 1));
-    int ok = 1;
     uint32_t it = 0;
     while ((int32_t)(dev_load(cnt) - want) < 0) {
-      if (++it > (1u << 22)) {
-        atomicOr(B.err, MCG_ERR_BARRIER);
-        ok = 0;
+      if (++it > WAIT_POLLS) {
+        wait_failed(B.err, s_flag);
         break;
       }
     }
-    *s_flag = ok;
   }
   __syncthreads();
   if (!*s_flag) return false;
-  if (threadIdx.x < 64)
-    for (int q = threadIdx.x; q < FSUMS; q += 64) {
+  if (tx < 64)
+    for (int q = tx; q < FSUMS; q += 64) {
       // the parts' values loaded together, then added in part order
       double y[MAX_PARTS];
 #pragma unroll
-      for (int p = 1; p < MAX_PARTS; ++p) y[p] = p < np ? dev_load(fp + (size_t)p * FSUMS + q) : 0.0;
+      for (int p = 1; p < MAX_PARTS; ++p) y[p] = p < np ? dev_load(fp + (size_t)(p - 1) * FSUMS + q) : 0.0;
       double x = F[q];
 #pragma unroll
       for (int p = 1; p < MAX_PARTS; ++p)
@@ -1938,17 +1931,21 @@ __device__ __forceinline__ bool gather_frame_sums(const SweepArgs& a, const mcg_
 }
 
 // Totals of every group's changes v[0..NC] (E, M) over its waves, in the
-// workgroup's first wave: sink(g, k, total) by one lane per group and value.
-// Called by every thread; s_red is free again only after the caller's next
-// workgroup barrier.
+// workgroup's first wave and in wave `also`, each for itself: sink(g, k, total)
+// by lane group_lane(g) + k.  Called by every thread; s_red is free again only
+// after the caller's next workgroup barrier.
+__device__ __forceinline__ int group_lane_stride(int TPR) {
+  const int nw = TPR >> 6;
+  return nw == 8 || nw == 16 ? 4 * nw : 4;
+}
 template <int NC, typename F>
-__device__ __forceinline__ void wave0_add(double* s_red, int TPR, const double* v, F&& sink) {
+__device__ __forceinline__ void wave0_add(double* s_red, int TPR, const double* v, int also, F&& sink) {
   double r[1];
   wave_totals<NC + 1>(v, r);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tx = tid(), lane = tx & 63, wave = tx >> 6;
   if (lane < 4) s_red[wave * RK + lane] = r[0];
   __syncthreads();
-  if (wave == 0) {
+  if (wave == 0 || wave == also) {
     const int nw = TPR >> 6, nwaves = (int)blockDim.x >> 6;
     const int k = lane & 3;
     double x = 0.0;
@@ -1974,33 +1971,36 @@ __device__ __forceinline__ void wave0_add(double* s_red, int TPR, const double* 
 // End of a persistent sweep for a workgroup of unsplit replicas: the state
 // update (and published energy) of every replica is done by the workgroup's
 // first wave, so that this serial per-replica work runs once per workgroup
-// instead of once in every group.  rep_l: lane g's replica; eslot_par: the
-// energy slots of this sweep's parity, or nullptr to publish nothing.  Called
-// by every thread; ends with a workgroup barrier.  Pool partials (PoolInfo):
-// thread t's changes are kept in pp[k*nr + t] (nr = R*rem, k < NC+1; pp is the
-// frame area, free between a sweep's frames and the next tail); replica g
-// adds its rem entries in thread order.
+// instead of once in every group.  es_l: lane g's words to publish its energy
+// in, with tag `tag`, or nullptr.  Called by every thread; the state and s_red
+// are the first wave's until the caller's next workgroup barrier.  Pool
+// partials (PoolInfo): thread t's changes are kept in pp[k*nr + t] (nr =
+// R*rem, k < NC+1; pp is the frame area, free between a sweep's frames and the
+// next tail); replica g adds its rem entries in thread order.  Wave pw, which
+// decides the swaps, keeps the energies for itself (e_pw, of the lane's group).
 template <int NC>
 __device__ __forceinline__ void tail_wave0(double* s_red, double* s_st, int R, int TPR, const double* v, bool therm_end,
-                                           int rep_l, double* eslot_par, const double* pp, int prem) {
-  wave0_add<NC>(s_red, TPR, v, [&](int g, int k, double x) {
+                                           uint64_t* es_l, uint32_t tag, const double* pp, int prem, int pw,
+                                           double& e_pw) {
+  const int tx = tid();
+  wave0_add<NC>(s_red, TPR, v, pw, [&](int g, int k, double x) {
     if (prem > 0) {
       double ps = 0.0;
       for (int i = 0; i < prem; ++i) ps += pp[k * R * prem + g * prem + i];
       x += ps;
     }
-    s_st[g * MCG_NSTATE + MCG_S_E + k] += x;
+    if (k == 0) e_pw += x;
+    if (tx < 64) s_st[g * MCG_NSTATE + MCG_S_E + k] += x;
   });
-  if (threadIdx.x < 64) {
+  if (tx < 64) {
     wave_lds_fence();
-    const int lane = threadIdx.x;
+    const int lane = tx;
     if (lane < R) {
       double* st = s_st + lane * MCG_NSTATE;
+      if (es_l) tag_store(es_l, tag, st[MCG_S_E]);
       if (therm_end) st[MCG_S_EREF] = st[MCG_S_E];
-      if (eslot_par) dev_store(eslot_par + (size_t)rep_l * MAX_PARTS, st[MCG_S_E]);
     }
   }
-  __syncthreads();
 }
 
 // one sweep of a workgroup's replica group: every colour class in turn,
@@ -2129,14 +2129,33 @@ __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& 
   }
 }
 
+// The kernel's arguments, and the same read again from the kernel's argument
+// memory: the persistent loop's parts read what they use where they use it (a
+// few scalar loads), so that some 60 words of arguments do not live, spilled,
+// across the sweeps.
+struct LdsArgs {
+  mcg_batch B;
+  const WorkItem* items;
+  const ItemRep* recs;
+  SweepArgs a;
+};
+__device__ __forceinline__ const LdsArgs& args_again() {
+  uint64_t x = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(x));
+  return *(const LdsArgs*)(const __attribute__((address_space(4))) LdsArgs*)x;
+}
+
 // MODE: link mode of every graph of the launch (0 pattern, 1 global links
 // with LDS tables, 2 wide); FULL: spin-derived observables are measured.
 // Both are compile-time so that each instantiation carries only the code it
 // runs (instruction-cache misses dominate the per-launch cost otherwise).
 // PERSIST: a persistent launch (every workgroup resident, see below).
 template <int NC, typename ST, int MODE, bool FULL, bool PERSIST>
-__global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __restrict__ items,
-                                              const ItemRep* __restrict__ recs, SweepArgs a) {
+__global__ __launch_bounds__(1024) void k_lds(LdsArgs A) {
+  const mcg_batch& B = A.B;
+  const SweepArgs& a = A.a;
+  const WorkItem* __restrict__ items = A.items;
+  const ItemRep* __restrict__ recs = A.recs;
   const WorkItem w = items[blockIdx.x];
   const mcg_graph G = B.graphs[w.graph];
   const int R = w.nrep;
@@ -2176,7 +2195,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   float4* s_par = (float4*)(smem + off);  // per group: beta, h, key1 bits (the pool's parameters)
   off += align16((size_t)R * 16);
   unsigned char* s_pers = smem + off;  // tempering state of a persistent launch
-  if (PERSIST) off += persist_lds_bytes(B.nrow, B.nrep);
+  if (PERSIST) off += persist_lds_bytes(B.nrow);
   ST* s_spin = (ST*)(smem + off);
 
   for (int t = threadIdx.x; t < ncl * 9; t += blockDim.x) s_coup[t / 9 * COUP_LDS + t % 9] = G.coup[t];
@@ -2239,93 +2258,115 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
   frame_consts<NC>(C, G, B);
   if (FULL && a.blk && w.nparts <= 1) C.blk = (float*)((unsigned char*)s_spin + R * lds_replica_bytes(NC, n, sizeof(ST)) + g * a.blk);
   if constexpr (PERSIST) {
-    // Persistent launch: many sweeps with the replicas in LDS.  After each
-    // sweep every replica's energy is published at the device coherence
-    // point (double-buffered by sweep parity); split parts publish their
-    // partial sums and the sites another part reads (export lists).  A grid
-    // barrier follows whenever tempering is due or parts must exchange.
-    // Then every workgroup computes the swap decisions of the ladders its
-    // replicas belong to itself, on its own copy of who/rung (identical in
-    // all workgroups that share a ladder: same energies, same Philox words),
-    // so no second barrier is needed: a workgroup can get at most one sweep
-    // ahead, and the parity buffers keep what the slower ones still read.
-    // Each ladder's owner writes its tables back at the end.
+    // Persistent launch: many sweeps with the replicas in LDS.  Nothing waits
+    // for the whole grid, or for a whole ladder: where tempering is due a
+    // replica's energy is published under its row (tagged words), and the
+    // workgroup reads the energy published under the partner row and decides
+    // the swap itself, as the partner's workgroup does (same energies, same
+    // Philox word).  A row's words are written in turn to four slots: a slot
+    // is written again four events later, by a workgroup that has got there
+    // through the event two before, which has the same pairs, and so after the
+    // reader of the slot had gone on (pairs alternate, or never change).
+    // The parts of a split replica exchange sites after every sweep: a part
+    // publishes its sums and the sites another part reads (export lists), waits
+    // for these stores, then publishes its energy, whose tag the other parts
+    // wait for; a part is at most one sweep ahead of the others, and the
+    // parity buffers keep what the slower ones still read.
+    // Measured against one barrier of all workgroups per event (two-level
+    // counters, after the stores' acknowledgement and before the loads of every
+    // energy of the ladder), with the end of a sweep on two waves and no
+    // scratch: XY 48^2 x 48 rungs 8.2 -> 6.0 us a sweep, 96^2 x 256 rungs
+    // 12.2 -> 9.8, 16^2 x 1024 rungs 9.1 -> 5.4; honeycomb 64^2 x 64 in four
+    // parts each 20 -> 18.
     typedef typename RawBits<sizeof(ST)>::T U;
     constexpr int GD = SitesPerDraw<NC>::G;
-    const int nrow = B.nrow, nrepb = B.nrep;
-    int32_t* s_who = (int32_t*)s_pers;
-    int32_t* s_ptacc = s_who + nrow;
-    int32_t* s_rung = s_ptacc + nrow;
-    float* s_beta = (float*)(s_pers + align16((size_t)(2 * nrow + nrepb) * 4));
+    const int nrow = B.nrow;
+    float* s_beta = (float*)s_pers;
     float* s_h = s_beta + nrow;
-    int32_t* s_lad = (int32_t*)(s_pers + align16((size_t)(2 * nrow + nrepb) * 4) + align16((size_t)2 * nrow * 4));
-    uint8_t* s_np = (uint8_t*)s_lad + align16((size_t)MAX_LADW * 3 * 4);  // parts of each replica
+    int32_t* s_row = (int32_t*)(s_pers + align16((size_t)2 * nrow * 4));
+    int2* s_lad = (int2*)(s_row + MAX_GROUPS);  // first row, rungs (0: no ladder)
+    int* s_flag = (int*)(s_lad + MAX_GROUPS);
     for (int t = threadIdx.x; t < nrow; t += blockDim.x) {
-      s_who[t] = B.who[t];
-      s_ptacc[t] = 0;
       s_beta[t] = B.row_beta[t];
       s_h[t] = B.row_h[t];
     }
-    for (int t = threadIdx.x; t < nrepb; t += blockDim.x) {
-      s_rung[t] = B.rung[t];
-      s_np[t] = a.rep_np[t];
+    if (lt == 0) {
+      s_row[g] = row;
+      s_lad[g] = make_int2(ir.row0, ir.nrung);
     }
-    // this workgroup's ladders, kept in LDS (read every tempering pass)
-    const int nlad = min(a.blk_lad[blockIdx.x + 1] - a.blk_lad[blockIdx.x], MAX_LADW);
-    if ((int)threadIdx.x < nlad) {
-      const int e = a.blk_lad[a.blk_lad[blockIdx.x] + threadIdx.x];
-      const int L = e & 0x7FFFFFFF;
-      s_lad[3 * threadIdx.x] = e;
-      s_lad[3 * threadIdx.x + 1] = a.lad_row0[L];
-      s_lad[3 * threadIdx.x + 2] = a.lad_n[L];
-    }
+    if (threadIdx.x == 0) *s_flag = 1;  // cleared by a wait that times out
     __syncthreads();
     U* lraw = (U*)my;
     U* xb = (U*)a.xbuf;
     const int DS = halo_desc_ints(G.ncol);
-    int* s_flag = (int*)s_red;
-    int nbar = 0;
+    uint32_t epoch = (uint32_t)a.sync_base;
     // Lane g of the first wave stands for group g (unsplit replicas) or for
     // the replica (part 0 of a split one) in the end-of-sweep work.  M' of a
-    // row (for <M M'>) passes from frame to frame through slot f % 3 of
-    // a.mprev3: frame f of a row is taken after the barrier of its sweep (or
-    // before it, see frames_after), reads slot (f-1) % 3 and writes slot
-    // f % 3; the writer of frame f-1 stored before it arrived at a barrier
-    // the reader has passed, and a workgroup is never more than one sweep
-    // ahead, so three slots never collide.  A[MPREV] seeds the slots of the
+    // row (for <M M'>) passes from frame to frame, and from workgroup to
+    // workgroup where the row moves, in tagged words: a frame reads the words
+    // of the last one's tag, then writes its own to the other slot, whose
+    // reader wrote the words it has just read.  A[MPREV] seeds the words of the
     // rows held at the start and takes the last frame's M'.
     const int lane = threadIdx.x & 63;
     const int nfr = pi.np == 1 ? R : pi.part == 0 ? 1 : 0;  // groups whose frames this workgroup takes
     const bool l_grp = threadIdx.x < 64 && lane < nfr;
-    const int pt0 = blockDim.x >= 128 ? 64 : 0;  // tempering on the waves after the first
-    // Frames are taken after the barrier when every sweep has one (split
-    // replicas, tempering every sweep); otherwise before it, so that a
-    // barrier always separates two frames of a row taken by different
-    // workgroups.
-    const bool frames_after = a.has_split || a.pt_every == 1;
+    // Swaps are the second wave's, so that the first wave's sums and frame and
+    // the second's draw, wait and decision run side by side (each is a chain of
+    // dependent instructions of one wave: 2,300 and 3,400 cycles).
+    const int pw = blockDim.x >= 128 ? 1 : 0;
+    const int gl = lane / group_lane_stride(TPR);
+    const bool l_lad = (int)threadIdx.x >> 6 == pw && lane % group_lane_stride(TPR) == 0 && gl < R;
+    double e_pw = 0.0;  // energy of the lane's replica (unsplit)
+    if (l_lad) e_pw = s_st[gl * MCG_NSTATE + MCG_S_E];
     const int fflags = FULL ? B.meas : (B.meas & ~MEAS_SPIN_OBS);  // what a frame measures
     // A split part measures the pairs and circuits whose first site it owns
-    // from its own copy before the grid barrier, when none of them has
+    // from its own copy before the parts' exchange, when none of them has
     // sites of two parts and no block spins or orbital groups are measured;
-    // its sums reach part 0 through the barrier (a.fpart, by sweep parity).
-    // Otherwise every part publishes its sites and, after the barrier, sums
+    // its sums reach part 0 through the exchange (a.fpart, by sweep parity).
+    // Otherwise every part publishes its sites and, after the exchange, sums
     // its share over the published copy; part 0 waits for the others' sums.
     const bool own_frame = FULL && pi.np > 1 && !(B.meas & (MCG_MEAS_RNORM | MCG_MEAS_GROUPS)) &&
                            pi.hx[2 * G.ncol + 7] != 0;
-    int rep_l = 0, row0_l = 0, last_row = -1;
+    int64_t fcur = a.k_begin > a.nthermal ? (a.k_begin - a.nthermal) / a.spf + a.frame0 : a.frame0;  // next frame
+    uint32_t ftag = (uint32_t)(fcur - a.frame0) + 1u;  // tag of the last frame's M'
+    auto mprev_at = [&](uint32_t tag, int r) { return a.mprev + ((size_t)(tag & 1u) * nrow + r) * 2; };
+    const int ladder_l = l_lad ? recs[w.off + gl].ladder : 0;
+    int frow_l = -1;  // the row of the lane's last frame, whose M is in s_mp
     if (l_grp) {
-      const ItemRep irl = recs[w.off + lane];
-      rep_l = irl.rep;
-      row0_l = irl.row0;
-      const int r = row0_l + s_rung[rep_l];
-      const double m0 = B.acc[(size_t)r * MCG_NACC + MCG_A_MPREV];
-      for (int q = 0; q < 3; ++q) dev_store(a.mprev3 + (size_t)q * nrow + r, m0);
+      const int r = s_row[lane];
+      tag_store(mprev_at(ftag, r), ftag, B.acc[(size_t)r * MCG_NACC + MCG_A_MPREV]);
+    }
+    uint32_t ev = 0;  // tempering events of this launch
+    // the thread's first exported site, and (two parts) its first imported one
+    int ex0 = 0, im0 = 0;
+    if (pi.np > 1 && lt < pi.hx[2 * G.ncol + 1]) ex0 = a.halo[pi.hx[2 * G.ncol] + lt];
+    if (pi.np == 2) {
+      const int32_t* hq = pi.hx + (1 - 2 * pi.part) * DS;
+      if (lt < hq[2 * G.ncol + 1]) im0 = a.halo[hq[2 * G.ncol] + lt];
     }
     // The sweeps' changes are added up (FP64, per thread) until a sweep needs
     // the energies: a frame, a swap pass, a recompute, the end.  Sweeps in
     // between end without the reduction over the workgroup.
     double v[4] = {0.0, 0.0, 0.0, 0.0};
     bool vfresh = true;
+    auto stage_frame = [&](const mcg_batch& B, const SweepArgs& a, int64_t f, uint32_t tag, int row_l, int lane) {
+      const bool l_grp = lane < nfr;
+      // frame f, by the first wave; tag: of the frame before; M' is read ahead
+      Tagged mpw;
+      const uint64_t* w = a.mprev + ((size_t)(tag & 1u) * nrow + row_l) * 2;
+      if (l_grp) mpw.load_ahead(w);
+      zero_terms(s_frm, nfr);
+      if (l_grp) {
+        double* F = s_frm + lane * FRM;
+        frame_terms<NC>(C, fresh(C.G), B, s_st + lane * MCG_NSTATE, F, fflags, f, F + FRM_ACC);
+        double* mm = F + FRM_ACC + MCG_A_MM;  // holds the frame's M
+        const double m = *mm;
+        s_mp[lane] = m;
+        frow_l = row_l;
+        tag_store(a.mprev + ((size_t)((tag + 1u) & 1u) * nrow + row_l) * 2, tag + 1u, m);
+        *mm = tag_wait(w, mpw, tag, B.err, s_flag) * m;
+      }
+    };
     // sweeps until the next frame, swap pass and recompute (each event's
     // period, 0: never), so that no sweep divides 64-bit indices
     const int64_t gs0 = a.philox_base + a.k_begin;
@@ -2336,24 +2377,29 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       return m < 0 ? -m : every - m;
     };
     int to_pt = until(a.pt_every), to_rec = until(rec_every);
-    int64_t fcur = a.k_begin > a.nthermal ? (a.k_begin - a.nthermal) / a.spf + a.frame0 : a.frame0;  // next frame
     int64_t to_frame = a.k_begin > a.nthermal ? a.spf - (a.k_begin - a.nthermal) % a.spf
                                               : (int64_t)a.nthermal - a.k_begin + a.spf;
-    for (int s = 0; s < a.nsweeps; ++s) {
-      const int64_t k = a.k_begin + s;
-      const uint64_t kk = (uint64_t)(a.philox_base + k);
-      const int par = (int)(k & 1);
-      const int rowg = wave_uniform(ir.row0 + s_rung[rep]);
+    const int nsweeps = a.nsweeps;
+    const int64_t k_begin = a.k_begin;
+    const uint64_t philox_base = (uint64_t)a.philox_base;
+    const int spf = a.spf, pt_every = a.pt_every;
+    const int64_t nthermal = a.nthermal;
+    const bool has_split = a.has_split != 0;
+    for (int s = 0; s < nsweeps; ++s) {
+      const int64_t k = k_begin + s;
+      const uint64_t kk = philox_base + (uint64_t)k;
+      const int rowg = wave_uniform(s_row[g]);
       const float bg = wave_uniform(s_beta[rowg]), hg = wave_uniform(s_h[rowg]);
       const bool meas = --to_frame == 0;
-      const bool therm_end = (k + 1 == a.nthermal);
+      const bool therm_end = (k + 1 == nthermal);
       const bool rec = --to_rec == 0;
       const bool pt_now = --to_pt == 0;
-      if (meas) to_frame = a.spf;
+      if (meas) to_frame = spf;
       if (rec) to_rec = rec_every;
-      if (pt_now) to_pt = a.pt_every;
-      const bool need = meas || therm_end || rec || pt_now || s == a.nsweeps - 1;
-      const int rowg_l = row0_l + s_rung[rep_l];
+      if (pt_now) to_pt = pt_every;
+      const bool need = meas || therm_end || rec || pt_now || s == nsweeps - 1;
+      if (pt_now || has_split) ++epoch;
+      const int par = (int)(epoch & 1u);
       if (pl.rem > 0) {  // the pool's parameters of this sweep (rows move with tempering)
         if (lt == 0) s_par[g] = make_float4(bg, hg, __uint_as_float(key1), __int_as_float(rowg));
         __syncthreads();
@@ -2367,18 +2413,56 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
       v[1] += (double)fM[0];
       v[2] += (double)fM[1];
       v[3] += (double)fM[2];
-      double* es = a.eslot + ((size_t)par * nrepb + rep) * MAX_PARTS;
-      double* ms = a.mslot + ((size_t)par * nrepb + rep) * MAX_PARTS * 3;
+      const LdsArgs& A = args_again();
+      const mcg_batch& B = A.B;
+      const SweepArgs& a = A.a;
+      const int tx = tid(), lane = tx & 63, lt = tx - g * TPR;
+      const bool wave0 = tx < 64, l_grp = wave0 && lane < nfr;
+      const int gl = lane / group_lane_stride(TPR);
+      const bool l_lad = tx >> 6 == pw && lane == gl * group_lane_stride(TPR) && gl < R;
+      // words of the row's energy (part `part`) in this event; the tag also
+      // says how many parts the row's replica has
+      auto row_words = [&](int r, int part) {
+        return a.rowslot + ((((size_t)(ev & 3u) * nrow + r) * a.nrow_parts) + part) * 2;
+      };
+      const uint32_t rtag = epoch << 2;
+      double e_l = 0.0;  // the lane's replica's energy
+      // The swap of the lane's replica: first the draw, which does not depend
+      // on the energies, then the partner's words, then the decision
+      const int row_l = wave0 && lane < R ? s_row[lane] : 0;  // the frame's
+      const int row_p = l_lad ? s_row[gl] : 0;
+      int rb = -1;     // the partner row, if the lane's replica has one
+      int t0 = 0;      // row of the pair's lower rung
+      float pu = 0.0f;
+      Tagged ew;
+      auto swap_draw = [&] {
+        if (!pt_now || !l_lad) return;
+        const int2 ld = s_lad[gl];
+        const int pp = (int)(kk & 1), t = row_p - ld.x;
+        const bool low = ((t - pp) & 1) == 0;  // the lower rung of its pair
+        const int tl = low ? t : t - 1;
+        if (tl < pp || tl + 1 >= ld.y) return;
+        const u32x4 x = philox4x32_10(u32x4{(uint32_t)tl, (uint32_t)kk, (uint32_t)(kk >> 32), TAG_PT}, B.seed_lo,
+                                      B.seed_hi ^ (0x80000000u | (uint32_t)ladder_l));
+        pu = u24(x.x);
+        t0 = ld.x + tl;
+        rb = low ? row_p + 1 : row_p - 1;
+      };
+      auto swap_read = [&] {
+        if (rb >= 0) ew.load_ahead(row_words(rb, 0));
+      };
       if (pi.np == 1) {
-        // state update and published energy before the barrier (with a full
-        // recompute due, the recomputed state is published instead)
+        // state update and published energy (with a full recompute due, the
+        // recomputed state is published instead)
         if (need) {
-          tail_wave0<NC>(s_red, s_st, R, TPR, v, therm_end && !rec, rep_l,
-                         rec ? nullptr : a.eslot + (size_t)par * nrepb * MAX_PARTS, s_frm, pl.rem);
+          tail_wave0<NC>(s_red, s_st, R, TPR, v, therm_end && !rec,
+                         pt_now && !rec && wave0 && lane < R && s_lad[lane].y > 0 ? row_words(row_l, 0) : nullptr,
+                         rtag, s_frm, pl.rem, pw, e_pw);
           vfresh = true;
           v[0] = v[1] = v[2] = v[3] = 0.0;
         }
         if (rec) {
+          __syncthreads();
           double* r4 = C.s_frm;
           recompute<NC>(sp, C.G, C.coup, C.cst, C.clsdat, hg, s_red, g, lt, TPR, r4);
           if (lt == 0) {
@@ -2387,26 +2471,32 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
             recompute_checks<ST>(B, G, r4, d);
             for (int q = 0; q < 4; ++q) st[MCG_S_E + q] = r4[q];
             if (therm_end) st[MCG_S_EREF] = st[MCG_S_E];
-            dev_store(es, st[MCG_S_E]);
+            if (pt_now && ir.nrung > 0) tag_store(row_words(rowg, 0), rtag, st[MCG_S_E]);
           }
           __syncthreads();
+          if (l_lad) e_pw = s_st[gl * MCG_NSTATE + MCG_S_E];
         }
         if constexpr (FULL) {
           // the spin-derived sums of every group's frame, from its LDS
-          // replica (the frame area is free after the tail)
+          // replica (the frame area is free after the tail); the first wave
+          // takes every group's frame
           if (meas) {
+            __syncthreads();
             frame_sums<NC, Spins<ST>, true>(sp, C, B, fcur, key0, key1, hg, 0, 1);
-            if (!frames_after) __syncthreads();  // the first wave takes every group's frame
+            __syncthreads();
           }
         }
+        swap_draw();
+        swap_read();
       } else {
         // one replica: the part's sums, published and kept in LDS
+        double* ms = a.mslot + ((size_t)par * a.nslots + w.slot) * (MAX_PARTS - 1) * 3;
         if (need) {
-          wave0_add<NC>(s_red, TPR, v, [&](int, int q, double x) {
-            if (q == 0)
-              dev_store(es + pi.part, (pi.part == 0 ? st[MCG_S_E] : 0.0) + x);
-            else
-              dev_store(ms + pi.part * 3 + (q - 1), x);
+          wave0_add<NC>(s_red, TPR, v, 0, [&](int, int q, double x) {
+            if (q > 0 && pi.part > 0) dev_store(ms + (pi.part - 1) * 3 + (q - 1), x);
+            if (q == 0 && pi.part == 0) x += st[MCG_S_E];
+            if (q == 0 && pt_now && ir.nrung > 0)
+              tag_store(row_words(rowg, pi.part), rtag | (uint32_t)(pi.np - 1), x);
             s_frm[FRM - 4 + q] = x;
           });
           v[0] = v[1] = v[2] = v[3] = 0.0;
@@ -2414,17 +2504,18 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
         const int32_t* ex = a.halo + pi.hx[2 * G.ncol];
         const int nex = pi.hx[2 * G.ncol + 1];
         U* xo = xb + (((size_t)par * a.nslots + w.slot) * MAX_PARTS + pi.part) * (size_t)a.max_export * NC;
-        for (int i = lt; i < nex; i += TPR)
-          export_site<NC>(xo + (size_t)i * NC, lraw, n, ex[i]);
+        if (lt < nex) export_site<NC>(xo + (size_t)lt * NC, lraw, n, ex0);
+        for (int i = lt + TPR; i < nex; i += TPR) export_site<NC>(xo + (size_t)i * NC, lraw, n, ex[i]);
         if constexpr (FULL) {
           if (meas && own_frame) {
+            __syncthreads();  // s_red
             const int32_t* d = pi.hx + 2 * G.ncol;
             const PartFrame pf{a.halo + d[2], a.halo + d[4], d[3], d[5], d[6] != 0};
             frame_sums<NC, Spins<ST>, true>(sp, C, B, fcur, key0, key1, hg, pi.part, pi.np, &pf);
             if (pi.part != 0) {
               __syncthreads();  // F is written by the first thread
-              double* fp = a.fpart + (((size_t)par * a.nslots + w.slot) * MAX_PARTS + pi.part) * FSUMS;
-              if ((int)threadIdx.x < FSUMS_PQ) dev_store(fp + threadIdx.x, s_frm[threadIdx.x]);
+              double* fp = a.fpart + (((size_t)par * a.nslots + w.slot) * (MAX_PARTS - 1) + pi.part - 1) * FSUMS;
+              if (tx < FSUMS_PQ) dev_store(fp + tx, s_frm[tx]);
             }
           }
           // the frame reads every part's sites: publish this part's own
@@ -2432,43 +2523,40 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
             part_publish<ST>(my, (U*)a.fspin + ((size_t)par * a.nslots + w.slot) * NC * a.fspin_n, n, a.fspin_n,
                              NC, s_colptr, G.ncol, GD, pi.part, pi.np, lt, TPR);
         }
-      }
-      if (meas && threadIdx.x < 64 && nfr > 0) zero_terms(s_frm, nfr);
-      if (meas && l_grp && !frames_after) {
-        take_frame<NC>(C, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, frame_mprev3<NC>(a, fcur, rowg_l, nrow),
-                       fflags);
-        last_row = rowg_l;
-      }
-      // the swap words of the first ladder are drawn while the barrier
-      // completes (they do not depend on the energies)
-      float pt_u0 = 0.0f;
-      if (a.has_split || pt_now) {
-        const uint32_t epoch = (uint32_t)(a.bar_base + nbar + 1);
-        grid_arrive(a.bar, epoch);
-        if (pt_now && nlad > 0) {
-          const int64_t swap = a.philox_base + k;
-          const int i = (int)threadIdx.x - pt0;
-          const int t = (int)(swap & 1) + 2 * i;
-          if (i >= 0 && t + 1 < s_lad[2]) {
-            const u32x4 x = philox4x32_10(u32x4{(uint32_t)t, (uint32_t)swap, (uint32_t)((uint64_t)swap >> 32), TAG_PT},
-                                          B.seed_lo, B.seed_hi ^ (0x80000000u | (uint32_t)(s_lad[0] & 0x7FFFFFFF)));
-            pt_u0 = u24(x.x);
+        // the energy last: its tag says that everything above has arrived
+        stores_done();
+        __syncthreads();
+        uint64_t* ps = a.pslot + ((size_t)par * a.nslots + w.slot) * MAX_PARTS * 2;
+        const double own_e = need ? s_frm[FRM - 4] : 0.0;  // part 0: with the replica's energy before
+        if (tx == 0) tag_store(ps + pi.part * 2, epoch, own_e);
+        swap_draw();
+        // the other parts' tags, lane p for part p, by the waves that need their
+        // energies (every wave for itself: 3 % slower on honeycomb 64^2 x 64)
+        Tagged pw;
+        {
+          uint32_t it = 0;
+          bool ok = !(tx < 128 && lane < pi.np && lane != pi.part);
+          while (!ok) {
+            pw.load(ps + lane * 2);
+            ok = pw.has(epoch);
+            if (!ok && ++it > WAIT_POLLS) {
+              wait_failed(B.err, s_flag);
+              break;
+            }
           }
         }
-        if (!grid_wait(a.bar, epoch, B.err, s_flag)) return;
-        ++nbar;
-      }
-      // M' of the frame's row, read first so that it overlaps the import
-      double mp = 0.0;
-      if (meas && l_grp && frames_after) mp = frame_mprev3<NC>(a, fcur, rowg_l, nrow);
-      if (pi.np > 1) {
+        __syncthreads();
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
         // part 0 reads part p's sums in lane p, overlapping the import
-        const bool w0 = need && pi.part == 0 && threadIdx.x < 64;
-        double pe = 0.0, pm[3] = {0.0, 0.0, 0.0};
+        const bool w0 = need && pi.part == 0 && wave0;
+        const double pe = lane == pi.part ? own_e : pw.value();
+        double pm[3] = {0.0, 0.0, 0.0};
         if (w0 && lane >= 1 && lane < pi.np) {
-          pe = dev_load(es + lane);
-          for (int q = 0; q < 3; ++q) pm[q] = dev_load(ms + lane * 3 + q);
+          for (int q = 0; q < NC; ++q) pm[q] = dev_load(ms + (lane - 1) * 3 + q);
         }
+        swap_read();
+        double Esum = lane_f64(pe, 0);  // the replica's energy: its parts', in part order
+        for (int p = 1; p < pi.np; ++p) Esum += lane_f64(pe, p);
         if (pi.np == 2) {
           // the other part's list directly (measured faster than the flat
           // round-robin on the XY scan's two-part replicas)
@@ -2480,7 +2568,7 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
             const U* xi = xb + (((size_t)par * a.nslots + w.slot) * MAX_PARTS + p) * (size_t)a.max_export * NC;
             for (int i = lt; i < nex; i += TPR) {
               const U* src = xi + (size_t)i * NC;
-              const int site = ex[i];
+              const int site = i < TPR ? im0 : ex[i];
               constexpr int W = NC * (int)sizeof(U);
               if constexpr (W == 8 || W == 4) {
                 typedef typename std::conditional<W == 8, uint64_t, uint32_t>::type P;
@@ -2497,23 +2585,24 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
           import_parts<NC>(xb + ((size_t)par * a.nslots + w.slot) * MAX_PARTS * (size_t)a.max_export * NC,
                            a.max_export, a.halo, pi.hx, DS, G.ncol, pi.part, pi.np, lraw, n, lt, TPR);
         }
+        e_l = Esum;
         if (w0) {
           const double* own = s_frm + FRM - 4;  // this part's sums
-          double E = st[MCG_S_E] + own[0], dm[3] = {own[1], NC > 1 ? own[2] : 0.0, NC > 2 ? own[3] : 0.0};
-          for (int p = 1; p < pi.np; ++p) {
-            E += lane_f64(pe, p);
+          double dm[3] = {own[1], NC > 1 ? own[2] : 0.0, NC > 2 ? own[3] : 0.0};
+          for (int p = 1; p < pi.np; ++p)
             for (int q = 0; q < 3; ++q) dm[q] += lane_f64(pm[q], p);
-          }
           if (lane == 0) {
-            st[MCG_S_E] = E;
+            st[MCG_S_E] = Esum;
             for (int q = 0; q < 3; ++q) st[MCG_S_M + q] += dm[q];
             if (therm_end) st[MCG_S_EREF] = st[MCG_S_E];
           }
         }
-        // the imported sites are read by other threads: by the frame, and by
-        // the next sweep's first colour when no frame or tempering pass
-        // (which end with a workgroup barrier) comes between
-        __syncthreads();
+        // the imported sites are read by other threads: by the frame's sums
+        // over the spins, and by the next sweep's first colour
+        if (FULL && meas) {
+          __syncthreads();
+          if (*s_flag == 0) return;
+        }
       }
       if constexpr (FULL) {
         if (meas && pi.np > 1) {
@@ -2522,16 +2611,16 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
           if (own_frame) {
             // the other parts' sums, stored before the barrier, added in
             // part order
-            if (pi.part == 0 && (int)threadIdx.x < FSUMS_PQ) {
-              const double* fp = a.fpart + ((size_t)par * a.nslots + w.slot) * MAX_PARTS * FSUMS + threadIdx.x;
+            if (pi.part == 0 && tx < FSUMS_PQ) {
+              const double* fp = a.fpart + ((size_t)par * a.nslots + w.slot) * (MAX_PARTS - 1) * FSUMS + tx;
               double y[MAX_PARTS];
 #pragma unroll
-              for (int p = 1; p < MAX_PARTS; ++p) y[p] = p < pi.np ? dev_load(fp + (size_t)p * FSUMS) : 0.0;
-              double x = s_frm[threadIdx.x];
+              for (int p = 1; p < MAX_PARTS; ++p) y[p] = p < pi.np ? dev_load(fp + (size_t)(p - 1) * FSUMS) : 0.0;
+              double x = s_frm[tx];
 #pragma unroll
               for (int p = 1; p < MAX_PARTS; ++p)
                 if (p < pi.np) x += y[p];
-              s_frm[threadIdx.x] = x;
+              s_frm[tx] = x;
             }
             __syncthreads();
           } else {
@@ -2542,94 +2631,56 @@ __global__ __launch_bounds__(1024) void k_lds(mcg_batch B, const WorkItem* __res
           }
         }
       }
-      // the frame of every replica (first wave, lane g), while the other
-      // waves run the tempering pass
-      if (meas && l_grp && frames_after) {
-        take_frame<NC>(C, B, a, s_st, s_frm, lane, fcur, rowg_l, nrow, mp, fflags);
-        last_row = rowg_l;
+      // the frame of every replica (first wave, lane g)
+      if (meas) {
+        if (wave0 && nfr > 0) stage_frame(B, a, fcur, ftag, row_l, lane);
+        ++ftag;
+        ++fcur;
       }
       if (pt_now) {
-        // the swaps of the ladders this workgroup's replicas belong to (the
-        // other ladders' rows are never read here)
-        const int64_t swap = a.philox_base + k;
-        const int pp = (int)(swap & 1);
-        for (int li = 0; li < nlad; ++li) {
-        const int L = s_lad[3 * li] & 0x7FFFFFFF;
-        const int r0 = s_lad[3 * li + 1];
-        const int npairs = max(0, (s_lad[3 * li + 2] - pp) / 2);
-        for (int i = (int)threadIdx.x - pt0; i < npairs; i += (int)blockDim.x - pt0) {
-          if (i < 0) break;
-          const int t = pp + 2 * i;
-          const int ra = s_who[r0 + t], rb = s_who[r0 + t + 1];
-          const double* ea = a.eslot + ((size_t)par * nrepb + ra) * MAX_PARTS;
-          const double* eb = a.eslot + ((size_t)par * nrepb + rb) * MAX_PARTS;
-          // the parts' slots at once (a replica's energy is the sum of its
-          // parts' slots, in part order)
-          const int npa = s_np[ra], npb = s_np[rb];
-          double xa[MAX_PARTS], xb[MAX_PARTS];
-#pragma unroll
-          for (int q = 0; q < MAX_PARTS; ++q) {
-            xa[q] = q < npa ? dev_load(ea + q) : 0.0;
-            xb[q] = q < npb ? dev_load(eb + q) : 0.0;
-          }
-          double Ea = xa[0], Eb = xb[0];
-#pragma unroll
-          for (int q = 1; q < MAX_PARTS; ++q) {
-            Ea += xa[q];
-            Eb += xb[q];
-          }
-          const double ba = s_beta[r0 + t], bb = s_beta[r0 + t + 1];
-          const double d = (ba - bb) * (Ea - Eb);
-          bool acc = d >= 0.0;
-          if (!acc) {
-            float u = pt_u0;  // drawn during the barrier for the first ladder
-            if (li > 0 || i >= (int)blockDim.x - pt0) {
-              const u32x4 x =
-                  philox4x32_10(u32x4{(uint32_t)t, (uint32_t)swap, (uint32_t)((uint64_t)swap >> 32), TAG_PT},
-                                B.seed_lo, B.seed_hi ^ (0x80000000u | (uint32_t)L));
-              u = u24(x.x);
+        // the swaps of the workgroup's replicas
+        if (rb >= 0) {
+          double eb = 0.0;
+          uint32_t it = 0;
+          for (int q = 0, np = 1; q < np;) {
+            if (ew.has(rtag, 3u)) {
+              np = (int)((uint32_t)(ew.a >> 32) & 3u) + 1;
+              eb = q ? eb + ew.value() : ew.value();  // in part order
+              if (++q == np) break;
+            } else if (++it > WAIT_POLLS) {
+              wait_failed(B.err, s_flag);
+              break;
             }
-            acc = u < exp_neg((float)d);
+            ew.load(row_words(rb, q));
           }
-          if (acc) {
-            s_who[r0 + t] = rb;
-            s_who[r0 + t + 1] = ra;
-            s_rung[ra] = t + 1;
-            s_rung[rb] = t;
-            s_ptacc[r0 + t] += 1;
+          const bool low = rb > row_p;
+          const double ea = pi.np == 1 ? e_pw : e_l;
+          const double ba = s_beta[t0], bb = s_beta[t0 + 1];
+          const double d = (ba - bb) * (low ? ea - eb : eb - ea);
+          if (d >= 0.0 || pu < exp_neg((float)d)) {
+            if (low && pi.part == 0) atomicAdd(B.pt_acc + t0, 1);
+            s_row[gl] = rb;
           }
         }
-        }
-        __syncthreads();
+        ++ev;
       }
-      if (meas && nfr > 0) {
+      if (pt_now || meas || pi.np > 1) {
         __syncthreads();
-        if (g < nfr) flush_frame<NC>(C, B, rowg, fflags);
+        if (*s_flag == 0) return;
       }
-      if (meas) ++fcur;
+      if (meas && g < nfr) flush_frame<NC>(C, B, rowg, fflags);
     }
     __syncthreads();
-    if (last_row >= 0) {
-      const int64_t fl = (a.k_begin + a.nsweeps - a.nthermal) / a.spf - 1 + a.frame0;  // last frame
-      B.acc[(size_t)last_row * MCG_NACC + MCG_A_MPREV] = dev_load(a.mprev3 + (size_t)(fl % 3) * nrow + last_row);
-    }
+    if (frow_l >= 0) B.acc[(size_t)frow_l * MCG_NACC + MCG_A_MPREV] = s_mp[lane];
     if (pi.np == 1)
       stage<ST, false>(my, gsp, NC * n, lt, TPR);
     else
       part_copy<ST, true>(my, gsp, n, NC, s_colptr, G.ncol, GD, pi.part, pi.np, lt, TPR);
     if (pi.part == 0 && lt < MCG_NSTATE) B.state[(size_t)rep * MCG_NSTATE + lt] = st[lt];
-    // each ladder's state goes back from its owner (flag bit 31 of the
-    // workgroup's ladder entry): the first workgroup holding one of its
-    // replicas
-    for (int li = 0; li < nlad; ++li) {
-      if (!(s_lad[3 * li] & 0x80000000)) continue;
-      const int r0 = s_lad[3 * li + 1];
-      for (int t = threadIdx.x; t < s_lad[3 * li + 2]; t += blockDim.x) {
-        const int r = s_who[r0 + t];
-        B.who[r0 + t] = r;
-        B.pt_acc[r0 + t] += s_ptacc[r0 + t];
-        B.rung[r] = s_rung[r];
-      }
+    if (l_grp && s_lad[lane].y > 0) {  // every row is held by one replica
+      const int r = s_row[lane], q = recs[w.off + lane].rep;
+      B.who[r] = q;
+      B.rung[q] = r - s_lad[lane].x;
     }
     return;
   } else {
@@ -2816,7 +2867,7 @@ __global__ __launch_bounds__(256, MCG_PASS_MIN_WAVES) void k_pass(mcg_batch B, c
   double v[4] = {(double)dE, (double)dM[0], (double)dM[1], (double)dM[2]};
 #pragma unroll
   for (int k = 0; k < 4; ++k) v[k] = wave_sum_f64(v[k]);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tx = tid(), lane = tx & 63, wave = tx >> 6;
   if (lane == 63)
 #pragma unroll
     for (int k = 0; k < 4; ++k) s_red[wave * 4 + k] = v[k];
@@ -3017,9 +3068,9 @@ __global__ void k_pt(mcg_batch B, const int32_t* __restrict__ ladder_row0, const
 // An item then makes one round trip to L2, and the draw runs while it waits;
 // reading frontier entry, link word, stamp, both spins and exchanging the
 // stamp in global memory made five.  Cubic 64^3 at T_c, 16 replicas (clusters
-// of 6,000 spins on average): 447 -> 270 us a cluster; 8 ordered replicas of a
-// few thousand sites gain 1.5x, clusters of a few spins 1.2x to 1.3x.  What is
-// left is one CU's gathers (a cache line per lane) and draws per replica.
+// of 6,000 spins on average): 447 -> 270 us a cluster; smaller lattices gain 1.5x
+// to 1.66x, clusters of a few spins 1.2x to 1.3x.  What is left is one CU's
+// gathers (a cache line per lane) and draws per replica.
 // ---------------------------------------------------------------------------
 static constexpr int WOLFF_FRONT = 2048;  // frontier entries in LDS (a level's others are read from the member list)
 static constexpr int WOLFF_RJR = 256;     // couplings whose r.J.r is kept
@@ -3416,17 +3467,18 @@ struct RunCtx {
   size_t dev_bytes = 0, tab_bytes = 0, reset_off = 0, reset_bytes = 0;
   std::vector<unsigned char> hstage;  // the tables as uploaded
   // offsets of the pieces, then their device addresses
-  size_t o_items = 0, o_item_reps = 0, o_stream = 0, o_all = 0, o_lrow0 = 0, o_ln = 0, o_halo = 0, o_repnp = 0,
-         o_blklad = 0, o_sync = 0, o_xpart = 0, o_bar = 0, o_eslot = 0, o_mslot = 0, o_xbuf = 0, o_mprev3 = 0,
+  size_t o_items = 0, o_item_reps = 0, o_stream = 0, o_all = 0, o_lrow0 = 0, o_ln = 0, o_halo = 0,
+         o_sync = 0, o_xpart = 0, o_rowslot = 0, o_pslot = 0, o_mslot = 0, o_xbuf = 0, o_mprev = 0,
          o_fsum = 0, o_fpart = 0, o_fspin = 0;
   int fspin_n = 0;  // component stride of the published-site copies
+  int max_np = 1;   // most parts of a replica
   const WorkItem* items = nullptr;
   const ItemRep* item_reps = nullptr;
   const int32_t *stream_reps = nullptr, *all_reps = nullptr, *lad_row0 = nullptr, *lad_n = nullptr,
-                *halo = nullptr, *blk_lad = nullptr;
-  const uint8_t* rep_np = nullptr;
-  uint32_t *sync = nullptr, *bar = nullptr;
-  double *xpart = nullptr, *eslot = nullptr, *mslot = nullptr, *mprev3 = nullptr;
+                *halo = nullptr;
+  uint32_t* sync = nullptr;
+  uint64_t *rowslot = nullptr, *pslot = nullptr, *mprev = nullptr;
+  double *xpart = nullptr, *mslot = nullptr;
   double* fsum = nullptr;  // split measurement: FSLOTS per replica, zero between frames
   double* fpart = nullptr;  // persistent split replicas: partial frame sums of each part
   void* fspin = nullptr;    // persistent split replicas: sites published for a frame
@@ -3823,10 +3875,10 @@ template <int NC, typename ST, int MODE, bool FULL, bool PERSIST>
 int launch_lds_range(const mcg_batch* B, RunCtx& X, const SweepArgs& a, hipStream_t s, int i0, int i1, hipEvent_t e0,
                      hipEvent_t e1) {
   size_t bytes = lds_bytes_for<NC, ST>(B, X, i0, i1);
-  if (PERSIST) bytes += persist_lds_bytes(B->nrow, B->nrep);
+  if (PERSIST) bytes += persist_lds_bytes(B->nrow);
   set_lds_attr<NC, ST, MODE, FULL, PERSIST>(bytes);
   hipExtLaunchKernelGGL((k_lds<NC, ST, MODE, FULL, PERSIST>), dim3((unsigned)(i1 - i0)), dim3(X.block),
-                        (uint32_t)bytes, s, e0, e1, 0, *B, X.items + i0, X.item_reps, a);
+                        (uint32_t)bytes, s, e0, e1, 0, LdsArgs{*B, X.items + i0, X.item_reps, a});
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -3874,7 +3926,7 @@ void plan_block_spins(const mcg_batch* B, RunCtx& X) {
   X.blk = 0;
   if (!(B->meas & MCG_MEAS_RNORM) || X.hitems.empty()) return;
   const int ni = (int)X.hitems.size();
-  const size_t pers = persist_lds_bytes(B->nrow, B->nrep);
+  const size_t pers = persist_lds_bytes(B->nrow);
   const size_t without = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
   for (const WorkItem& w : X.hitems)
     X.blk = std::max(X.blk, (int)align16((size_t)B->graphs_host[w.graph].nr * NC * 4));
@@ -3899,7 +3951,7 @@ int check_persist(const mcg_batch* B, const mcg_plan* P, RunCtx& X, bool* ok) {
   if (full && m != 0 && m != 3) return 0;
   const bool pt = P->pt_every > 0 && !X.hl_row0.empty();
   if (!pt && X.nslots == 0) return 0;
-  const size_t bytes = lds_bytes_for<NC, ST>(B, X, 0, (int)X.hitems.size()) + persist_lds_bytes(B->nrow, B->nrep);
+  const size_t bytes = lds_bytes_for<NC, ST>(B, X, 0, (int)X.hitems.size()) + persist_lds_bytes(B->nrow);
   if (bytes > X.lds_max) return 0;
   const void* f = full ? (m == 0 ? (const void*)k_lds<NC, ST, 0, true, true> : (const void*)k_lds<NC, ST, 3, true, true>)
                   : m == 0 ? (const void*)k_lds<NC, ST, 0, false, true>
@@ -4122,41 +4174,16 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   X.persist = false;
   if (P->algorithm == MCG_METROPOLIS && !P->no_persist && !force_stream && check_persist<NC, ST>(B, P, X, &X.persist))
     return -1;
-  // workgroup ladder lists of a persistent launch: the ladders of each
-  // workgroup's replicas; the first workgroup of a ladder owns it
-  std::vector<int32_t> bl;
-  std::vector<uint8_t> np;
-  if (X.persist) {
-    np.assign(B->nrep, 1);
-    for (const WorkItem& w : X.hitems)
-      if (w.nparts > 1) np[X.hitem_reps[w.off]] = w.nparts;
-    std::vector<int32_t> lad_of_row(B->nrow, -1);
-    for (size_t L = 0; L < X.hl_row0.size(); ++L) lad_of_row[X.hl_row0[L]] = (int32_t)L;
-    const size_t nb = X.hitems.size();
-    bl.assign(nb + 1, 0);
-    std::vector<char> owned(X.hl_row0.size(), 0);
-    for (size_t i = 0; i < nb; ++i) {
-      const WorkItem& w = X.hitems[i];
-      std::vector<int32_t> ls;
-      for (int q = 0; q < w.nrep; ++q) {
-        const mcg_replica& R = B->reps_host[X.hitem_reps[w.off + q]];
-        const int L = R.ladder >= 0 && R.nrung >= 2 ? lad_of_row[R.row0] : -1;
-        if (L >= 0 && std::find(ls.begin(), ls.end(), L) == ls.end()) ls.push_back(L);
-      }
-      std::sort(ls.begin(), ls.end());
-      if (ls.size() > (size_t)MAX_LADW) return fail("internal: more than %d ladders in one workgroup", MAX_LADW);
-      for (int32_t L : ls) {
-        bl.push_back(owned[L] ? L : (int32_t)(L | 0x80000000u));
-        owned[L] = 1;
-      }
-      bl[i + 1] = (int32_t)(bl.size() - (nb + 1));
-    }
-    for (size_t i = 0; i <= nb; ++i) bl[i] += (int32_t)(nb + 1);
-  }
+  std::vector<int32_t> lad_of_row(B->nrow, -1);
+  for (size_t L = 0; L < X.hl_row0.size(); ++L) lad_of_row[X.hl_row0[L]] = (int32_t)L;
+  X.max_np = 1;
+  for (const WorkItem& w : X.hitems) X.max_np = std::max(X.max_np, (int)w.nparts);
   std::vector<ItemRep> recs(X.hitem_reps.size());
   for (size_t i = 0; i < recs.size(); ++i) {
     const mcg_replica& R = B->reps_host[X.hitem_reps[i]];
-    recs[i] = ItemRep{R.spin_off, X.hitem_reps[i], (int32_t)R.serial, R.row0, 0};
+    const bool lad = R.ladder >= 0 && R.nrung >= 2;
+    recs[i] = ItemRep{R.spin_off, X.hitem_reps[i], (int32_t)R.serial, R.row0, lad ? R.nrung : 0,
+                      lad ? lad_of_row[R.row0] : -1, 0};
   }
   // layout: tables first, then the state every run clears
   size_t off = 0;
@@ -4167,20 +4194,18 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   X.o_lrow0 = take(&off, X.hl_row0.size() * 4);
   X.o_ln = take(&off, X.hl_n.size() * 4);
   X.o_halo = take(&off, X.hhalo.size() * 4);
-  X.o_repnp = take(&off, np.size());
-  X.o_blklad = take(&off, bl.size() * 4);
   X.tab_bytes = off;
   X.reset_off = off;
   X.o_fsum = take(&off, (size_t)B->nrep * FSLOTS * 8);
   X.o_sync = take(&off, (size_t)X.nslots * SYNC_STRIDE * 4);
   X.o_xpart = take(&off, (size_t)X.nslots * MAX_PARTS * 4 * 8);
   if (X.persist) {
-    X.o_bar = take(&off, (size_t)BAR_WORDS * 4);
-    X.o_eslot = take(&off, (size_t)2 * B->nrep * MAX_PARTS * 8);
-    X.o_mslot = take(&off, (size_t)2 * B->nrep * MAX_PARTS * 3 * 8);
+    X.o_rowslot = take(&off, (size_t)4 * B->nrow * X.max_np * 16);
+    X.o_pslot = take(&off, (size_t)2 * X.nslots * MAX_PARTS * 16);
+    X.o_mslot = take(&off, (size_t)2 * X.nslots * (MAX_PARTS - 1) * 3 * 8);
     X.o_xbuf = take(&off, (size_t)2 * std::max(X.nslots, 1) * MAX_PARTS * std::max(X.max_export, 1) * NC * sizeof(ST));
-    X.o_mprev3 = take(&off, (size_t)3 * B->nrow * 8);
-    X.o_fpart = take(&off, (size_t)2 * std::max(X.nslots, 1) * MAX_PARTS * FSUMS * 8);
+    X.o_mprev = take(&off, (size_t)2 * B->nrow * 16);
+    X.o_fpart = take(&off, (size_t)2 * std::max(X.nslots, 1) * (MAX_PARTS - 1) * FSUMS * 8);
   }
   X.reset_bytes = off - X.reset_off;
   if (X.persist && X.nslots > 0 && (B->meas & MEAS_SPIN_OBS)) {
@@ -4202,8 +4227,6 @@ int prepare_typed(const mcg_batch* B, const mcg_plan* P, RunCtx& X) {
   put(X.o_lrow0, X.hl_row0.data(), X.hl_row0.size() * 4);
   put(X.o_ln, X.hl_n.data(), X.hl_n.size() * 4);
   put(X.o_halo, X.hhalo.data(), X.hhalo.size() * 4);
-  put(X.o_repnp, np.data(), np.size());
-  put(X.o_blklad, bl.data(), bl.size() * 4);
   // the key
   X.k_kernel = P->kernel;
   X.k_block = P->block;
@@ -4237,15 +4260,13 @@ int bind_region(RunCtx& X, unsigned char* dev, hipStream_t s) {
   X.lad_row0 = (const int32_t*)at(X.o_lrow0);
   X.lad_n = (const int32_t*)at(X.o_ln);
   X.halo = (const int32_t*)at(X.o_halo);
-  X.rep_np = (const uint8_t*)at(X.o_repnp);
-  X.blk_lad = (const int32_t*)at(X.o_blklad);
   X.sync = (uint32_t*)at(X.o_sync);
   X.xpart = (double*)at(X.o_xpart);
-  X.bar = (uint32_t*)at(X.o_bar);
-  X.eslot = (double*)at(X.o_eslot);
+  X.rowslot = (uint64_t*)at(X.o_rowslot);
+  X.pslot = (uint64_t*)at(X.o_pslot);
   X.mslot = (double*)at(X.o_mslot);
   X.xbuf = at(X.o_xbuf);
-  X.mprev3 = (double*)at(X.o_mprev3);
+  X.mprev = (uint64_t*)at(X.o_mprev);
   X.fsum = (double*)at(X.o_fsum);
   X.fpart = (double*)at(X.o_fpart);
   X.fspin = at(X.o_fspin);
@@ -4345,7 +4366,7 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
   // finish every launch (one sweep per launch) and tempering needs a launch
   // boundary every pt_every sweeps
   const int64_t chunk = X.persist ? 4096 : X.nslots > 0 ? 1 : P->pt_every > 0 ? P->pt_every : total;
-  int64_t bar_base = 0;
+  int64_t sync_base = 0;  // exchanges of parts and ladders before a launch
   for (int64_t k = 0; k < total;) {
     int64_t ns = std::min<int64_t>(chunk, total - k);
     if (!X.persist && X.nslots == 0 && P->pt_every > 0)  // launches end where swaps are due
@@ -4357,19 +4378,15 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
     SweepArgs a{k, P->sweep0, (int32_t)ns, (int32_t)nth, spf, P->frame0, X.sync, X.xpart, X.halo};
     a.blk = X.blk;
     if (X.persist) {
-      a.bar = X.bar;
-      a.bar_base = (int32_t)bar_base;
+      a.sync_base = (int32_t)sync_base;
       a.pt_every = pt_on ? P->pt_every : 0;
       a.has_split = X.nslots > 0;
-      a.nladder = (int32_t)X.hl_row0.size();
-      a.lad_row0 = X.lad_row0;
-      a.lad_n = X.lad_n;
-      a.blk_lad = X.blk_lad;
-      a.rep_np = X.rep_np;
-      a.eslot = X.eslot;
+      a.nrow_parts = X.max_np;
+      a.rowslot = X.rowslot;
+      a.pslot = X.pslot;
       a.mslot = X.mslot;
       a.xbuf = X.xbuf;
-      a.mprev3 = X.mprev3;
+      a.mprev = X.mprev;
       a.fpart = X.fpart;
       a.fspin = X.fspin;
       a.fspin_n = X.fspin_n;
@@ -4377,9 +4394,9 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
       a.nslots = std::max(X.nslots, 1);
       a.rec_host = rec_host ? 1 : 0;
       for (int64_t q = k; q < k + ns; ++q)
-        if (X.nslots > 0 || (pt_on && ((P->sweep0 + q + 1) % P->pt_every) == 0)) ++bar_base;
-      if (bar_base * (int64_t)std::max<size_t>(X.hitems.size(), BAR_GROUPS) >= ((int64_t)1 << 31))
-        return fail("too many barriers in one call (%lld); split the call", (long long)bar_base);
+        if (X.nslots > 0 || (pt_on && ((P->sweep0 + q + 1) % P->pt_every) == 0)) ++sync_base;
+      if (sync_base * (int64_t)std::max<size_t>(X.hitems.size(), 16) >= ((int64_t)1 << 31))
+        return fail("too many barriers in one call (%lld); split the call", (long long)sync_base);
     }
     if (!X.hitems.empty()) {
       if (launch_lds<NC, ST>(B, X, a, s, T)) return -1;
