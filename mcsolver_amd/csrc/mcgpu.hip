@@ -356,6 +356,14 @@ struct HbmView {
   }
   __device__ __forceinline__ void st(const Site& s, int k, float v) const { SIO<ST>::st((GAS ST*)((GAS char*)p[k] + s), v); }
 };
+// spins in HBM read by site: the same 32-bit offsets from scalar bases
+template <int NC, typename ST>
+struct HbmSpins {
+  typedef ST value_type;
+  HbmView<NC, ST> v;
+  __device__ __forceinline__ HbmSpins(ST* p, int n) : v(gas(p), n) {}
+  __device__ __forceinline__ float get(int i, int c) const { return v.ld(v.at(i), c, 0); }
+};
 
 // What the updates of a sweep read besides spins and draws.  Neighbours come
 // from link patterns (rows in LDS, pat: the row of each position) or from the
@@ -1165,6 +1173,7 @@ struct PartFrame {
 // spins, F[32..) groups.  np = 1: the whole frame.  With `own`, the share
 // is instead own's pairs and circuits (their other sites being current in
 // the part's copy), and block spins and groups are not measured.
+static constexpr int FRAME_TRI = 2;  // triangles in flight per thread
 static constexpr int FSUMS = 88;     // frame sums per replica (F[0, 88))
 static constexpr int FSUMS_PQ = 9;   // of which pairs and circuits (F[0, 9))
 // Inlined wherever it is used: as a call it takes the batch, the graph and the
@@ -1216,19 +1225,39 @@ __device__ __forceinline__ void frame_sums(const SV& sp, const FrameCtx& C, cons
     float il = sqrtf(C.clsdat[4]);
     bool one_len = G.ncls <= 64;
     for (int q = 1; q < G.ncls && one_len; ++q) one_len = C.clsdat[q * 8 + 4] == C.clsdat[4];
-    for (int q = lo + lt; q < hi; q += TPR) {
-      const int p = own ? own->circs[q] : q;
-      const int ia = G.circ[3 * p], ib = G.circ[3 * p + 1], ic = G.circ[3 * p + 2];
-      float a[3], b[3], c[3];
-      spin_vec<NC>(sp, ia, cls, C.clsdat, a);
-      spin_vec<NC>(sp, ib, cls, C.clsdat, b);
-      spin_vec<NC>(sp, ic, cls, C.clsdat, c);
-      if (one_len)
-        v[0] += (double)signed_area(a, b, c, il, il, il);
-      else
-        v[0] += (double)signed_area(a, b, c, inv_len(C.clsdat, G.cls, ia), inv_len(C.clsdat, G.cls, ib),
-                                    inv_len(C.clsdat, G.cls, ic));
-    }
+    auto triangles = [&](auto one, auto uc) {
+      // U at a time: their indices, then their spins are in flight together
+      // (triangular 128^2 x 1024, 5 sweeps: one 1365 us, two 1304, three 1309)
+      constexpr int U = decltype(uc)::value;
+      for (int q = lo + lt; q < hi; q += U * TPR) {
+        int id[U][3];
+        float x[U][3][3];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int qu = min(q + u * TPR, hi - 1), p = own ? own->circs[qu] : qu;
+          const GAS int32_t* t = (const GAS int32_t*)((const GAS char*)gas(G.circ) + (uint32_t)p * 12u);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) id[u][k] = t[k];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) spin_vec<NC>(sp, id[u][k], nullptr, C.clsdat, x[u][k]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (u > 0 && q + u * TPR >= hi) break;
+          if constexpr (decltype(one)::value)
+            v[0] += (double)signed_area(x[u][0], x[u][1], x[u][2], il, il, il);
+          else
+            v[0] += (double)signed_area(x[u][0], x[u][1], x[u][2], inv_len(C.clsdat, G.cls, id[u][0]),
+                                        inv_len(C.clsdat, G.cls, id[u][1]), inv_len(C.clsdat, G.cls, id[u][2]));
+        }
+      }
+    };
+    if (one_len)
+      triangles(std::true_type(), std::integral_constant<int, FRAME_TRI>());
+    else
+      triangles(std::false_type(), std::integral_constant<int, 1>());
     group_add<1>(v, C.s_red, C.g, TPR, [&](int, double x) { F[8] = x; });
   }
   // --- block-spin observables
@@ -2946,7 +2975,7 @@ __global__ __launch_bounds__(256) void k_frame_part(mcg_batch B, const int32_t* 
   const mcg_graph G = B.graphs[rp.graph];
   __shared__ double s_red[4 * RK];
   __shared__ double s_frm[FSUMS];
-  const Spins<ST> sp{(ST*)B.spins + rp.spin_off, G.n};
+  const HbmSpins<NC, ST> sp((ST*)B.spins + rp.spin_off, G.n);
   const int row = rp.row0 + B.rung[rep];
   const float h = B.row_h[row];
   const int part = item % np;
