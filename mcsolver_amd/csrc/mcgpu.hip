@@ -170,12 +170,18 @@ struct Acc {
   float inv_unit;
   const uint32_t* thr0;
   int nthr;
-  __device__ __forceinline__ Acc(float b) : beta(b), thr(nullptr), inv_unit(0.0f), thr0(nullptr), nthr(0) {}
+  const uint32_t* lds;  // the table's copy in LDS, or nullptr; lds0: every group's, lstride words apart
+  const uint32_t* lds0;
+  int lstride;
+  __device__ __forceinline__ Acc(float b)
+      : beta(b), thr(nullptr), inv_unit(0.0f), thr0(nullptr), nthr(0), lds(nullptr), lds0(nullptr), lstride(0) {}
   __device__ __forceinline__ Acc(float b, const uint32_t* t, float iu, const uint32_t* t0, int n)
-      : beta(b), thr(t), inv_unit(iu), thr0(t0), nthr(n) {}
-  // the same table at another row (beta b)
-  __device__ __forceinline__ Acc at(float b, int row) const {
-    return Acc(b, thr0 ? thr0 + (size_t)row * nthr : nullptr, inv_unit, thr0, nthr);
+      : beta(b), thr(t), inv_unit(iu), thr0(t0), nthr(n), lds(nullptr), lds0(nullptr), lstride(0) {}
+  // the same table at another row (beta b), of group g
+  __device__ __forceinline__ Acc at(float b, int row, int g) const {
+    Acc x(b, thr0 ? thr0 + (size_t)row * nthr : nullptr, inv_unit, thr0, nthr);
+    if (lds0) x.lds = lds0 + g * lstride;
+    return x;
   }
 };
 // the acceptance of row `row` of the batch
@@ -295,6 +301,10 @@ __device__ __forceinline__ void metro_commit(const float* s, float* n, float is2
 __device__ __forceinline__ bool ising_decide(float s, float f, float h, const Acc& ac, uint32_t w_c, float& dE) {
   const float t = f - h;
   dE = (-2.0f * s) * t;
+  if (ac.lds) {  // as below; downhill flips read entry 0 and ignore it
+    const uint32_t x = ac.lds[max((int)(dE * ac.inv_unit), 0)];
+    return (dE <= 0.0f) | (w_c < x);
+  }
   if (ac.thr)
     // exact: couplings, fields and spin lengths are multiples of powers of
     // two small enough that every operation above is exact, dE = k u with
@@ -1513,6 +1523,7 @@ struct SweepArgs {
   int32_t fspin_n;
   int32_t max_export;
   int32_t nslots;
+  int32_t thr;               // LDS bytes per group for its row's Ising thresholds, after those (0: none)
   int32_t blk;               // LDS bytes per group for a frame's block spins, after the spins (0: none)
   int32_t rec_host;          // the full recompute is the host's (a launch ends at each
                              // recompute sweep, then k_measure recomputes every replica)
@@ -2074,7 +2085,7 @@ __device__ __forceinline__ void sweep_colours(const mcg_graph& G, const Spins<ST
             const float4 pv = pl.par[pl.pr];
             float pe = 0.0f, pm[3] = {0.0f, 0.0f, 0.0f};
             const LdsView<NC, ST> pv_s{pl.spin0 + pl.sstride * pl.pr, G.n};
-            metro_sites<NC, PAT, UNI, Z>(pv_s, b, cnt, qm + pl.pq, c, T, beta.at(pv.x, __float_as_int(pv.w)), pv.y, kk,
+            metro_sites<NC, PAT, UNI, Z>(pv_s, b, cnt, qm + pl.pq, c, T, beta.at(pv.x, __float_as_int(pv.w), pl.pr), pv.y, kk,
                                          key0, __float_as_uint(pv.z), pe, pm);
             // the first pool group after a tail stores, later ones add
             double* pp = pl.pp + threadIdx.x;
@@ -2130,7 +2141,7 @@ __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& 
                                            const Spins<ST>& sp, const float* coup,
                                            const float* clsdat, const int32_t* s_colptr, const uint8_t* s_pid,
                                            const int32_t* s_pat, double* st, FrameCtx& C, int lt, int TPR, int row,
-                                           float beta, float h, uint32_t key0, uint32_t key1, const PartInfo& pi,
+                                           const Acc& beta, float h, uint32_t key0, uint32_t key1, const PartInfo& pi,
                                            double& dE, double* dM, bool aniso, const PoolInfo<ST>& pl, double* mp) {
   const bool split = pi.np > 1;
   dE = 0.0;
@@ -2141,8 +2152,8 @@ __device__ __forceinline__ void lds_sweeps(const mcg_graph& G, const mcg_batch& 
     const uint64_t kk = (uint64_t)(a.philox_base + k);
     const bool meas = k >= a.nthermal && ((k - a.nthermal + 1) % a.spf) == 0;
     float fE = 0.0f, fM[3] = {0.0f, 0.0f, 0.0f};  // this sweep's accepted changes
-    sweep_colours<NC, ST, MODE>(G, sp, coup, clsdat, s_colptr, s_pid, s_pat, lt, TPR, acc_of(B, beta, row), h, kk, key0,
-                                key1, pi, fE, fM, aniso, pl, pfresh);
+    sweep_colours<NC, ST, MODE>(G, sp, coup, clsdat, s_colptr, s_pid, s_pat, lt, TPR, beta, h, kk, key0, key1, pi, fE,
+                                fM, aniso, pl, pfresh);
     pfresh = false;
     dE += (double)fE;
     dM[0] += (double)fM[0];
@@ -2715,8 +2726,22 @@ __global__ __launch_bounds__(1024) void k_lds(LdsArgs A) {
   } else {
   double dE, dM[3];
   double* mp = s_mp + g;
+  Acc acc = acc_of(B, beta, row);
+  if constexpr (NC == 1) {
+    // the rows' thresholds into LDS: a flip's decision is the last link of the
+    // chain of a colour's round, and waited for L2 there.
+    // Ising 32^2 x 16, 200 sweeps with frames: 964 -> 905 us.
+    if (a.thr) {
+      uint32_t* s_thr = (uint32_t*)((unsigned char*)s_spin + R * (lds_replica_bytes(NC, n, sizeof(ST)) + a.blk));
+      acc.lstride = a.thr / 4;
+      acc.lds0 = s_thr;
+      acc.lds = s_thr + g * acc.lstride;
+      for (int t = lt; t < B.nthr; t += TPR) s_thr[g * acc.lstride + t] = acc.thr[t];
+      __syncthreads();
+    }
+  }
   if (lt == 0) *mp = B.acc[(size_t)row * MCG_NACC + MCG_A_MPREV];  // read by the same thread
-  lds_sweeps<NC, ST, MODE, FULL>(G, B, a, sp, C.coup, C.clsdat, s_colptr, s_pid, s_pat, st, C, lt, TPR, row, beta, h,
+  lds_sweeps<NC, ST, MODE, FULL>(G, B, a, sp, C.coup, C.clsdat, s_colptr, s_pid, s_pat, st, C, lt, TPR, row, acc, h,
                                  key0, key1, pi, dE, dM, aniso, pl, mp);
   __syncthreads();
   if (pi.np == 1) {
@@ -3477,6 +3502,7 @@ struct RunCtx {
   int nslots = 0;  // split replicas (arrival counters)
   int max_export = 0;  // longest export list of a part
   int blk = 0;  // LDS bytes per replica for a frame's block spins (0: looked up at every use)
+  int thr = 0;  // and for its row's Ising thresholds (0: read from global memory)
   bool persist = false;  // persistent launches (barrier + tempering inside)
   int mode_begin[5] = {0, 0, 0, 0, 0};  // work items of link mode m: [mode_begin[m], mode_begin[m+1])
   size_t lds_max = 0;
@@ -3894,7 +3920,7 @@ size_t lds_bytes_for(const mcg_batch* B, const RunCtx& X, int i0, int i1) {
     const bool wide = G.lcid != nullptr || G.ncls > 256;
     const size_t b = lds_fixed_bytes(wide ? 0 : G.ncoup, wide ? 0 : G.ncls, G.ncol, G.npat, G.zmax, G.n, nwaves,
                                      w.nrep) +
-                     w.nrep * (lds_replica_bytes(NC, G.n, sizeof(ST)) + (w.nparts > 1 ? 0 : (size_t)X.blk));
+                     w.nrep * (lds_replica_bytes(NC, G.n, sizeof(ST)) + (w.nparts > 1 ? 0 : (size_t)(X.blk + X.thr)));
     mx = std::max(mx, b);
   }
   return mx;
@@ -3948,19 +3974,29 @@ int launch_lds(const mcg_batch* B, RunCtx& X, const SweepArgs& a, hipStream_t s,
   return 0;
 }
 
-// Room for a frame's block spins in LDS (X.blk): taken when the workgroups
-// still fit, and as many of them per CU as without it.
+// Room in LDS for a frame's block spins (X.blk) and for the rows' Ising
+// thresholds (X.thr): taken when the workgroups still fit, and as many of them
+// per CU as without it.
 template <int NC, typename ST>
 void plan_block_spins(const mcg_batch* B, RunCtx& X) {
-  X.blk = 0;
-  if (!(B->meas & MCG_MEAS_RNORM) || X.hitems.empty()) return;
+  X.blk = X.thr = 0;
+  if (X.hitems.empty()) return;
   const int ni = (int)X.hitems.size();
   const size_t pers = persist_lds_bytes(B->nrow);
   const size_t without = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
-  for (const WorkItem& w : X.hitems)
-    X.blk = std::max(X.blk, (int)align16((size_t)B->graphs_host[w.graph].nr * NC * 4));
-  const size_t with = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
-  if (with > X.lds_max || (ni > X.ncu && X.lds_max / with != X.lds_max / without)) X.blk = 0;
+  auto fits = [&] {
+    const size_t with = lds_bytes_for<NC, ST>(B, X, 0, ni) + pers;
+    return with <= X.lds_max && (ni <= X.ncu || X.lds_max / with == X.lds_max / without);
+  };
+  if (B->meas & MCG_MEAS_RNORM) {
+    for (const WorkItem& w : X.hitems)
+      X.blk = std::max(X.blk, (int)align16((size_t)B->graphs_host[w.graph].nr * NC * 4));
+    if (!fits()) X.blk = 0;
+  }
+  if (NC == 1 && B->ithr && B->nthr <= 1024) {
+    X.thr = (int)align16((size_t)B->nthr * 4);
+    if (!fits()) X.thr = 0;
+  }
 }
 
 // Can this run use a persistent launch?  All replicas on the LDS path, one
@@ -4430,6 +4466,7 @@ int exec_typed(const mcg_batch* B, const mcg_plan* P, hipStream_t s, RunCtx& X) 
     if (rec_host) ns = std::min<int64_t>(ns, B->recompute_every - (P->sweep0 + k) % B->recompute_every);
     SweepArgs a{k, P->sweep0, (int32_t)ns, (int32_t)nth, spf, P->frame0, X.sync, X.xpart, X.halo};
     a.blk = X.blk;
+    a.thr = B->ithr && (int64_t)B->nthr * 4 <= X.thr ? X.thr : 0;
     if (X.persist) {
       a.sync_base = (int32_t)sync_base;
       a.pt_every = pt_on ? P->pt_every : 0;
