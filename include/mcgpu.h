@@ -59,7 +59,7 @@ enum { MCG_S_E = 0, MCG_S_M = 1 /* 3 */, MCG_S_EREF = 4, MCG_S_DRIFT = 5, MCG_S_
 enum { MCG_NBINQ = 5 };
 
 /* bits of the device error flag (batch->err), raised by the kernels:
- * BARRIER    a grid barrier of a persistent launch timed out (the launch left)
+ * BARRIER    a wait between the workgroups of a persistent launch timed out (they left)
  * NONFINITE  a full FP64 recompute found a non-finite energy or magnetisation
  *            (NaN / Inf in the spins)
  * LENGTH     a full FP64 recompute found the mean relative spin-length
@@ -249,7 +249,7 @@ int mcg_runner_destroy(mcg_runner *runner);
  * it is for callers that cannot allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  Same plan, launches and
  * results as mcg_run; its device scratch (launch tables, arrival counters,
- * barrier words, published energies) lives in a file-scope array of
+ * published energies, exported sites) lives in a file-scope array of
  * MCG_NOALLOC_SCRATCH_BYTES per device, which every device that loads the
  * library holds until the process ends.  A run that needs more is refused
  * with an error before anything is launched (configs of a few thousand

@@ -10,7 +10,7 @@ itself and returns the fastest.  The plan dimensions (Batch.run options):
 
   parts           workgroups per LDS replica (the tile: 0 the planner's
                   rule, 1 whole replicas, 2 or 4 parts with halo groups)
-  no_persist      persistent launches (barrier and tempering inside) or not
+  no_persist      persistent launches (tempering and part exchange inside) or not
   reps_per_block  the planner's packing of replicas per workgroup, or one
   block           threads per workgroup of the LDS kernel (0: the planner's
                   1024, or 256 / 512)

@@ -2649,7 +2649,7 @@ __global__ __launch_bounds__(1024) void k_lds(LdsArgs A) {
           // this part's share of the spin-derived sums: from its own copy, or
           // over every part's published sites; part 0 gathers the others'
           if (own_frame) {
-            // the other parts' sums, stored before the barrier, added in
+            // the other parts' sums, stored before the exchange, added in
             // part order
             if (pi.part == 0 && tx < FSUMS_PQ) {
               const double* fp = a.fpart + ((size_t)par * a.nslots + w.slot) * (MAX_PARTS - 1) * FSUMS + tx;
@@ -2811,7 +2811,9 @@ __global__ __launch_bounds__(1024) void k_lds(LdsArgs A) {
 // others read the global link table.  Bound: HBM traffic and the round trips
 // of one update (pattern, spins, store).  Measured on cubic 64^3 x 128 T
 // (16.8M updates, 615 MB a pass): 241 -> 160 us when the links came to be read
-// together through 32-bit offsets (2.6 -> 3.8 TB/s; a copy reaches 5.3).
+// together through 32-bit offsets (2.6 -> 3.8 TB/s; a copy reaches 5.3), and
+// 61 us for each 64 replicas (5.0 TB/s) since they come in groups that the
+// last-level cache holds.
 // Changes of E and M: FP32 per thread, FP64 DPP wave sums, one device
 // atomic per value per block.
 // ---------------------------------------------------------------------------

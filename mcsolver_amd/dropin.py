@@ -86,8 +86,8 @@ def recompute_period(nbr, J, ising: bool, diag_only: bool = False) -> int:
 
 
 def check_health(b: Batch) -> None:
-    """Raise if the engine's device error flag is set: a persistent launch's
-    barrier timed out, or a full FP64 recompute found NaN / Inf in the spins
+    """Raise if the engine's device error flag is set: a wait between the
+    workgroups of a persistent launch timed out, or a full FP64 recompute found NaN / Inf in the spins
     or spin lengths off their S (include/mcgpu.h MCG_ERR_*)."""
     f = b.error_flag()
     if f:
