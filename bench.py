@@ -360,7 +360,8 @@ def profile_summary(d: str, workload: str, store: str) -> str:
     fig["traffic_bytes_per_launch"] = fig["fetch_bytes_per_launch"] + fig["write_bytes_per_launch"]
     v = _pick(_counters(os.path.join(d, "valu", "run_counter_collection.csv"))[kname], stream)
     cyc = v["GRBM_GUI_ACTIVE"] / NXCD
-    fig["valu_busy_frac"] = v["SQ_ACTIVE_INST_VALU"] / NCU / cyc
+    busy = v["SQ_ACTIVE_INST_VALU"] / NCU / cyc
+    fig["valu_busy_frac"] = min(busy, 1.0)  # a saturated kernel reads up to 1.01
     fig["valu_issue_frac"] = v["SQ_INSTS_VALU"] / NCU / cyc
     if "SQ_THREAD_CYCLES_VALU" in v:
         fig["valu_utilization"] = v["SQ_THREAD_CYCLES_VALU"] / (v["SQ_ACTIVE_INST_VALU"] * 64)
@@ -406,7 +407,7 @@ def profile_summary(d: str, workload: str, store: str) -> str:
     o.append("| figure | definition | value |")
     o.append("|---|---|---|")
     o.append("| VALU busy | SQ_ACTIVE_INST_VALU / %d CUs / cycles (rocprofv3's VALUBusy for gfx950, as a fraction) | "
-             "%.3f |" % (NCU, fig["valu_busy_frac"]))
+             "%.3f |" % (NCU, busy))
     o.append("| VALU issue | SQ_INSTS_VALU / %d CUs / cycles (one wave instruction per CU-cycle is the peak without "
              "packed FP32) | %.3f |" % (NCU, fig["valu_issue_frac"]))
     if "valu_utilization" in fig:
